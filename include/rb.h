@@ -254,10 +254,12 @@ rb_status rb_bvh_host_release(rb_host_bvh_t b);
  * terminators / uint32 index); MI355X is this library's traversal layout.
  * Call with NULL buffers to get the sizes in bytes. */
 enum { RB_LAYOUT_REF_COMPACT2 = 1, RB_LAYOUT_MI355X = 2,
-       RB_LAYOUT_MI355X_WIDE = 3 /* no counterpart: the MI355X triangles and index with the
-                                    wide (4-child, 64-byte) records the upload builds as nodes;
-                                    RB_ERR_UNSUPPORTED where the upload would keep the binary
-                                    walk only */ };
+       RB_LAYOUT_MI355X_WIDE = 3 /* no counterpart: the MI355X triangles and index with wide
+                                    (4-child, 64-byte) records as nodes, every inner child of a
+                                    binary record replaced by its own two and boxes in
+                                    power-of-two steps; RB_ERR_UNSUPPORTED where they cannot
+                                    hold a box.  (The records the upload walks choose their
+                                    children by surface area and have steps of any size) */ };
 rb_status rb_bvh_export(rb_host_bvh_t b, uint32_t layout, void* nodes, size_t* nodes_bytes,
                         void* tris, size_t* tris_bytes, void* index, size_t* index_bytes);
 
@@ -396,31 +398,33 @@ typedef struct rb_trace_config {
                                 speculative while-while (kepler_dynamic_fetch.h:222-243),
                                 whose leaf order depends on the other rays of the
                                 wave -- in rare boundary cases ids and t may differ */
-    uint32_t leaf_gate;      /* non-speculative order: a wave leaves its inner-node phase
-                                once at most this many lanes still search for a leaf
-                                (0..63; 0 = when all have one).  Any value gives the
-                                same results: only the interleaving of lanes changes */
-    uint32_t lds_nodes;      /* top-of-tree node records each block copies into LDS at
-                                start and reads from there (0..512, multiple of 64; 0 =
-                                none).  The MI355X layout stores the first 512 records
-                                breadth-first, so these are the top levels of the tree.
-                                Any value gives the same results */
+    uint32_t leaf_gate;      /* non-speculative order: the lanes of a wave that hold a
+                                leaf test their next triangle once at most this many
+                                lanes are at an inner node (0..63; 0 = when none is,
+                                63 = always).  Any value gives the same results: only
+                                the interleaving of lanes changes */
+    uint32_t lds_nodes;      /* speculative order: top-of-tree node records each block
+                                copies into LDS at start and reads from there (0..512,
+                                multiple of 64; 0 = none).  The MI355X layout stores
+                                the first 512 records breadth-first, so these are the
+                                top levels of the tree.  Any value gives the same
+                                results */
     uint32_t wide;           /* 1 (default): closest-hit traces without a visit-count
-                                buffer walk 4-child records (each binary record's
-                                children, inner ones replaced by their own two; 64
-                                bytes, boxes in 8-bit steps that hold the exact ones),
-                                about half the dependent fetches per ray; lds_nodes
-                                such records go to LDS.  The same (id, t) as the binary
-                                walk, whose order any-hit traces and visit counts keep;
-                                0: the binary records for every trace */
+                                buffer walk 4-child records (subtrees of the binary
+                                tree chosen by surface area; 64 bytes, boxes in 8-bit
+                                steps that hold the exact ones), about half the
+                                dependent fetches per ray.  The same (id, t) as the
+                                binary walk, whose order any-hit traces and visit
+                                counts keep; 0: the binary records for every trace */
 } rb_trace_config;
 rb_status rb_trace_get_config(rb_trace_config* c);
 rb_status rb_trace_set_config(const rb_trace_config* c);
 /* Autotuner (no reference counterpart; the reference hard-codes the launch
  * shape): times candidate configurations on the caller's device rays by
  * coordinate descent over block, lds_stack, chunk, fetch_threshold,
- * waves_per_cu and leaf_gate (speculative is kept as set), installs the
- * fastest and returns it with its time per launch. */
+ * waves_per_cu and leaf_gate (lds_nodes in the speculative order, which is
+ * kept as set), installs the fastest and returns it with its time per
+ * launch. */
 rb_status rb_trace_autotune(rb_bvh_t bvh, const rb_ray* rays, uint32_t n, uint32_t flags, rb_hit* hits,
                             uint32_t reps, rb_trace_config* best, float* best_ms, void* stream);
 /* Traversal error flags raised on the device since the last call (the

@@ -73,59 +73,57 @@ __device__ __forceinline__ rb_hit rb_trace_one(const rb_bvh_dev& b, const rb_ray
     while (nodeAddr != RB_DEV_SENTINEL) {
         /* wide records until a leaf is reached */
         while (wnodes && (uint32_t)nodeAddr < (uint32_t)RB_DEV_SENTINEL && leafAddr >= 0) {
-            /* record: origin p.xyz | biased exponents (byte a: e + 127 of axis
-               a); the children's 8-bit steps for lo.x, hi.x, lo.y, hi.y, lo.z,
-               hi.z (byte c = child c); four links (0x7fffffff: no child) */
+            /* record: origin p.xyz, steps 2^24 s.xyz; the children's 8-bit
+               steps for lo.x, hi.x, lo.y, hi.y, lo.z, hi.z (byte c = child c,
+               plane p + q s, on or outside the exact one); four links */
             const float4* np = wnodes + 4 * (size_t)nodeAddr;
-            const float4 r0 = np[0];
-            const uint4 r1 = *reinterpret_cast<const uint4*>(np + 1);
+            const float4 r0 = np[0], r1 = np[1];
             const uint4 r2 = *reinterpret_cast<const uint4*>(np + 2);
-            const uint4 r3 = *reinterpret_cast<const uint4*>(np + 3);
-            asm volatile("" ::"v"(r0.x), "v"(r1.x), "v"(r2.x), "v"(r3.x));
-            const uint32_t eb = __float_as_uint(r0.w);
-            const float sx = __uint_as_float((eb & 0xFFu) << 23);
-            const float sy = __uint_as_float(((eb >> 8) & 0xFFu) << 23);
-            const float sz = __uint_as_float(((eb >> 16) & 0xFFu) << 23);
-            const int lk[4] = {(int)r2.z, (int)r2.w, (int)r3.x, (int)r3.y};
-            float key[4];
-            int lnk[4];
+            const int4 lk = *reinterpret_cast<const int4*>(np + 3);
+            asm volatile("" ::"v"(r0.x), "v"(r1.x), "v"(r2.x), "v"(lk.x));
+            const float sx = r0.w * idx, sy = r1.x * idy, sz = r1.y * idz;
+            /* an overflowing step makes its axis NaN, left out by min / max */
+            const float bx = fmaf(sx, 0.0f, fmaf(r0.x, idx, -oodx));
+            const float by = fmaf(sy, 0.0f, fmaf(r0.y, idy, -oody));
+            const float bz = fmaf(sz, 0.0f, fmaf(r0.z, idz, -oodz));
+            const uint32_t lox = __float_as_uint(r1.z), hix = __float_as_uint(r1.w);
+            const uint32_t wnx = idx < 0.0f ? hix : lox, wfx = idx < 0.0f ? lox : hix;
+            const uint32_t wny = idy < 0.0f ? r2.y : r2.x, wfy = idy < 0.0f ? r2.x : r2.y;
+            const uint32_t wnz = idz < 0.0f ? r2.w : r2.z, wfz = idz < 0.0f ? r2.z : r2.w;
+            int lnk[4] = {lk.x, lk.y, lk.z, lk.w};
+            int key[4]; /* entry distance as an integer, RB_DEV_MISS past every float */
+#define RB_DEV_MISS 0x7fffffff
 #pragma unroll
             for (int c = 0; c < 4; c++) {
-                /* a plane is fmaf(step, 2^e, p), a box holding the exact one */
-#define RB_DEV_Q(w, s, p) fmaf((float)(((w) >> (8 * c)) & 0xFFu), s, p)
-                const float lx = RB_DEV_Q(r1.x, sx, r0.x), hx = RB_DEV_Q(r1.y, sx, r0.x);
-                const float ly = RB_DEV_Q(r1.z, sy, r0.y), hy = RB_DEV_Q(r1.w, sy, r0.y);
-                const float lz = RB_DEV_Q(r2.x, sz, r0.z), hz = RB_DEV_Q(r2.y, sz, r0.z);
+#define RB_DEV_Q(w, s, b) fmaf((float)((w) >> (8 * c) & 0xFFu) * 0x1p-24f, s, b)
+                const float near = fmaxf(fmaxf(RB_DEV_Q(wnx, sx, bx), RB_DEV_Q(wny, sy, by)),
+                                         fmaxf(RB_DEV_Q(wnz, sz, bz), tmin));
+                const float far = fminf(fminf(RB_DEV_Q(wfx, sx, bx), RB_DEV_Q(wfy, sy, by)),
+                                        fminf(RB_DEV_Q(wfz, sz, bz), hitT));
 #undef RB_DEV_Q
-                const float clox = fmaf(lx, idx, -oodx), chix = fmaf(hx, idx, -oodx);
-                const float cloy = fmaf(ly, idy, -oody), chiy = fmaf(hy, idy, -oody);
-                const float cloz = fmaf(lz, idz, -oodz), chiz = fmaf(hz, idz, -oodz);
-                const float cmin = fmaxf(fmaxf(fminf(clox, chix), fminf(cloy, chiy)), fmaxf(fminf(cloz, chiz), tmin));
-                const float cmax = fminf(fminf(fmaxf(clox, chix), fmaxf(cloy, chiy)), fminf(fmaxf(cloz, chiz), hitT));
-                const bool h = cmax >= cmin && lk[c] != 0x7fffffff;
-                key[c] = h ? fminf(cmin, 0x1.fffffep127f) : __builtin_inff();
-                lnk[c] = lk[c];
+                key[c] = fmaf(fabsf(far), 0x1p-22f, far) >= near ? __float_as_int(near) : RB_DEV_MISS;
             }
-            /* hit children nearest first, misses last */
+            /* the nearest hit child next, the others pushed */
 #define RB_DEV_CS(i, j)                                        \
     if (key[j] < key[i]) {                                     \
-        const float tk = key[i];                               \
+        const int tk = key[i];                                 \
         key[i] = key[j];                                       \
         key[j] = tk;                                           \
         const int tl = lnk[i];                                 \
         lnk[i] = lnk[j];                                       \
         lnk[j] = tl;                                           \
     }
-            RB_DEV_CS(0, 1) RB_DEV_CS(2, 3) RB_DEV_CS(0, 2) RB_DEV_CS(1, 3) RB_DEV_CS(1, 2)
+            RB_DEV_CS(0, 1) RB_DEV_CS(2, 3) RB_DEV_CS(0, 2)
 #undef RB_DEV_CS
-            if (key[0] == __builtin_inff()) {
+            if (key[0] == RB_DEV_MISS) {
                 RB_DEV_POP(nodeAddr);
             } else {
-                if (key[3] != __builtin_inff()) RB_DEV_PUSH(lnk[3]);
-                if (key[2] != __builtin_inff()) RB_DEV_PUSH(lnk[2]);
-                if (key[1] != __builtin_inff()) RB_DEV_PUSH(lnk[1]);
+                if (key[3] != RB_DEV_MISS) RB_DEV_PUSH(lnk[3]);
+                if (key[1] != RB_DEV_MISS) RB_DEV_PUSH(lnk[1]);
+                if (key[2] != RB_DEV_MISS) RB_DEV_PUSH(lnk[2]);
                 nodeAddr = lnk[0];
             }
+#undef RB_DEV_MISS
             if (nodeAddr < 0) {
                 leafAddr = nodeAddr;
                 RB_DEV_POP(nodeAddr);

@@ -47,16 +47,16 @@ static rb_status init_locked(int device) {
         uint64_t keep = ~0ull;
         (void)hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep);
     }
-    // the best measured shape on 2 Mi incoherent rays at 1M triangles: the
-    // 12-entry LDS stack and 384 cached top-of-tree records take 48 KB per
-    // 512-thread block, which keeps 3 blocks (24 waves) on a CU
-    g_dev.cfg.block = 512;
+    // the best measured shape on 2 Mi incoherent rays at 1M triangles: a
+    // 256-thread block's 12-entry stacks and staged records take 28 KB of LDS,
+    // which keeps 5 blocks (20 waves) on a CU
+    g_dev.cfg.block = 256;
     g_dev.cfg.lds_stack = 12;
     g_dev.cfg.chunk = 64;
-    g_dev.cfg.fetch_threshold = 60;
-    g_dev.cfg.waves_per_cu = 24;
+    g_dev.cfg.fetch_threshold = 52;
+    g_dev.cfg.waves_per_cu = 20;
     g_dev.cfg.speculative = 0;
-    g_dev.cfg.leaf_gate = 24;
+    g_dev.cfg.leaf_gate = 56;
     g_dev.cfg.lds_nodes = 384;
     g_dev.cfg.wide = 1;
     g_dev.device = device;
@@ -344,14 +344,12 @@ rb_status rb_bvh_upload(rb_host_bvh_t hb, rb_scene_t scene, rb_bvh_t* out) {
                         depth == UINT32_MAX ? "not a tree" : "too deep", kMaxStack);
         // wide records only where their walk fits the same stack and their
         // 8-bit steps can hold the boxes (else the binary walk alone)
-        if (wide_fits_stack(depth)) {
-            st = export_wide(L.nodes, wide);
-            if (st == RB_ERR_UNSUPPORTED) {
-                wide.clear();
-                set_error("");
-            } else if (st != RB_OK) {
-                return st;
-            }
+        st = export_walk(L.nodes, (uint32_t)L.index.size(), wide);
+        if (st == RB_ERR_UNSUPPORTED) {
+            wide.clear();
+            set_error("");
+        } else if (st != RB_OK) {
+            return st;
         }
     } catch (...) {
         return fail(RB_ERR_OOM, "layout export failed (host allocation)");
@@ -377,10 +375,19 @@ rb_status rb_bvh_upload(rb_host_bvh_t hb, rb_scene_t scene, rb_bvh_t* out) {
     if ((st = up((void**)&B->nodes, L.nodes.data(), L.nodes.size() * 4)) != RB_OK) { cleanup(); return st; }
     B->n_wnodes = (uint32_t)(wide.size() / kWideWords);
     if (!wide.empty() && (st = up((void**)&B->wnodes, wide.data(), wide.size() * 4)) != RB_OK) { cleanup(); return st; }
-    // one spare row after the triangle array keeps 16-byte loads in bounds
-    L.tris.resize(L.tris.size() + 4, 0.0f);
+    // after the references the zero triangle of the wide records' empty
+    // slots (no ray hits it)
+    L.tris.resize(L.tris.size() + 12, 0.0f);
     if ((st = up((void**)&B->tris, L.tris.data(), L.tris.size() * 4)) != RB_OK) { cleanup(); return st; }
     L.index.push_back(0);
+    {
+        std::vector<uint32_t> t4(((size_t)B->n_refs + 1) * 16, 0u);
+        for (uint32_t r = 0; r <= B->n_refs; r++) {
+            std::memcpy(&t4[16 * (size_t)r], &L.tris[12 * (size_t)r], 48);
+            t4[16 * (size_t)r + 12] = L.index[r];
+        }
+        if ((st = up((void**)&B->tris4, t4.data(), t4.size() * 4)) != RB_OK) { cleanup(); return st; }
+    }
     if ((st = up((void**)&B->index, L.index.data(), L.index.size() * 4)) != RB_OK) { cleanup(); return st; }
     if (scene) {
         const Scene& Sc = scene->s;
@@ -423,7 +430,8 @@ rb_status rb_bvh_release(rb_bvh_t b) {
     if (dev().device >= 0) {
         dfree(b->nodes, (size_t)b->n_nodes * 64);
         dfree(b->wnodes, (size_t)b->n_wnodes * kWideWords * 4);
-        dfree(b->tris, ((size_t)b->n_refs * 12 + 4) * 4);
+        dfree(b->tris, ((size_t)b->n_refs * 12 + 12) * 4);
+        dfree(b->tris4, ((size_t)b->n_refs + 1) * 64);
         dfree(b->index, ((size_t)b->n_refs + 1) * 4);
         dfree(b->tri_v, (size_t)b->n_tris * 48);
         dfree(b->tri_n, (size_t)b->n_tris * 48);

@@ -177,6 +177,29 @@ rb_status export_mi355x(const HostBvh& b, Mi355Layout& out);
 constexpr uint32_t kWideWords = 16;
 constexpr int32_t kWideEmpty = 0x7FFFFFFF;
 rb_status export_wide(const std::vector<uint32_t>& bin, std::vector<uint32_t>& wide);
+// The wide records the upload makes and the kernels walk, 16 words each:
+// words 0..2 the origin p (the smallest corner of the children), words 3..5
+// the step s of each axis times 2^24 (floats), words 6..11 the children's
+// 8-bit steps (byte c of each word = child c) for lo.x, hi.x, lo.y, hi.y,
+// lo.z, hi.z (plane = p + q s), words 12..15 their links (>= 0: wide record;
+// < 0: leaf, as in the binary records; a slot without a child: the leaf of
+// one zero triangle that the upload puts after the n_refs references, behind
+// a box that rays do not pass).  Record 0 is the root, the records are
+// numbered breadth-first.
+//
+// A ray tests a plane with one fused multiply-add of its step, q (s / d) +
+// (p / d - o / d), where the binary walk's plane / d - o / d rounds once.
+// The planes at the origin (q = 0) are exact and so are their distances.  An
+// axis whose step times 2^24 / d overflows (or whose extent is past 2^103: an
+// infinite step) is left out of the test.
+// For the others rounding may move the distance by 2^-23 of the time to
+// cross the record's children and by 2^-24 of the distance itself; their
+// planes lie outside the boxes by 2^-20 of the children's extent, and the
+// walk widens a span by 2^-22 of its far end.  So a ray passes a child's box
+// whenever it passes the binary walk's, every leaf the binary walk tests is
+// tested, and closest hits, which do not depend on the visit order (ties at
+// equal t go to the lowest triangle id), have the same (id, t).
+rb_status export_walk(const std::vector<uint32_t>& bin, uint32_t n_refs, std::vector<uint32_t>& walk);
 // Depth of the deepest inner record of an MI355X node array (root = 0);
 // UINT32_MAX when a link leaves the array or the links form a cycle.  A
 // traversal holds at most depth + 1 stack entries (the sentinel, then one

@@ -15,26 +15,28 @@
 //  * the work counter lives in a per-launch slot that the last block resets
 //    (the reference copies a zero into a global symbol before each launch,
 //    cudatracer.cu:164-165), so concurrent launches and graph replays work;
-//  * leaf order: by default a lane tests a leaf as soon as it reaches one,
-//    so every ray visits nodes and leaves in the same order whatever the
-//    other rays of its wave do -- the order of the single-ray restatement --
-//    and results are the same run to run.  SPEC = the reference's
-//    speculative form (a lane holding a leaf keeps walking inner nodes until
-//    the whole wave holds leaves, kepler_dynamic_fetch.h:222-243): fewer
-//    idle lanes, but the leaf order then depends on the wave, and where a
-//    slab test rounds a box entry past a hit inside it, which hit survives
-//    culling can change with it (rare; ids and t may then differ);
+//  * step loop: in one iteration every lane of a wave does one step of its
+//    own ray, a node record or one triangle (trace_steps); records come in
+//    through LDS, 64 bytes per cache access (stage_records);
+//  * leaf order: a lane tests a leaf as soon as it reaches one, so every ray
+//    visits nodes and leaves in the same order whatever the other rays of its
+//    wave do -- the order of the single-ray restatement -- and results are
+//    the same run to run.  SPEC = the reference's speculative form
+//    (trace_spec: a lane holding a leaf keeps walking inner nodes until the
+//    whole wave holds leaves, kepler_dynamic_fetch.h:222-243): the leaf order
+//    then depends on the wave, and where a slab test rounds a box entry past
+//    a hit inside it, which hit survives culling can change with it (rare;
+//    ids and t may then differ);
 //  * batched mode: one launch serves up to kMaxBatch ray batches against
-//    different resident BVHs; every lane carries the scene pointers and the
-//    any/closest flag of the batch its current ray belongs to, so a wave can
-//    mix rays of several scenes while it refills;
+//    different resident BVHs; every lane carries the batch its current ray
+//    belongs to and that scene's pointers, so a wave can mix rays of several
+//    scenes while it refills;
 //  * paired mode: two queued ray sets of one BVH (an any-hit or closest-hit
 //    set, then a closest-hit set) in one launch, so a render bounce pays
 //    one launch's ramp-up and tail instead of two;
-//  * top of the tree in LDS: each block copies the first lds_nodes node
-//    records (the layout stores them breadth-first) into LDS at start and
-//    reads them from there; every ray passes through them, often several
-//    times (the reference reads every node through the texture path).
+//  * top of the tree in LDS (speculative form): each block copies the first
+//    lds_nodes node records (the layout stores them breadth-first) into LDS
+//    at start and reads them from there.
 // Arithmetic (fp32, explicit fmaf, reciprocals equal to the IEEE division)
 // matches the oracle's restatement bit for bit.
 #include "rb_device.h"
@@ -43,7 +45,7 @@ namespace rb {
 
 struct TraceArgs {
     const float4* __restrict__ nodes;
-    const float4* __restrict__ tris;
+    const float4* __restrict__ tris;  // 3 rows per reference (speculative walk), or 4 with the id (step loop)
     const uint32_t* __restrict__ index;
     const float4* __restrict__ rays;
     const uint8_t* __restrict__ mask;
@@ -142,6 +144,18 @@ __device__ __forceinline__ float vmax3_(float a, float b, float c) {
     return r;
 }
 
+// Distances of one plane of two of a wide record's children (half h: 0 and
+// 1, or 2 and 3): their 8-bit steps, spread by one byte permute to the two
+// halves 0x00qq, which as half-precision numbers are q * 2^-24 (subnormal),
+// go straight into a mixed-precision fused multiply-add each, q s + b (the
+// record holds s * 2^24).
+__device__ __forceinline__ void walk_planes(uint32_t w, int h, float s, float b, float t[2]) {
+    typedef _Float16 H2 __attribute__((ext_vector_type(2)));
+    const H2 p = __builtin_bit_cast(H2, __builtin_amdgcn_perm(0u, w, h ? 0x0C030C02u : 0x0C010C00u));
+    t[0] = fmaf((float)p.x, s, b);
+    t[1] = fmaf((float)p.y, s, b);
+}
+
 // Every single-precision bit pattern through rcp_rn's fast path and through
 // rcp_rn itself, against the division: out[0] += inputs whose refined
 // reciprocal is taken, out[1] += inputs where either differs from 1.0f / x
@@ -176,23 +190,30 @@ __global__ __launch_bounds__(256) void k_rcp_check(unsigned long long* out) {
     }
 }
 
-// PAIR: rays [0, n0) are the first set (a.rays / a.hits; any hit when
-// a.any0), rays [n0, nrays) the closest-hit set (a.rays2 / a.hits2).
-// WIDE: a.nodes holds wide (4-child) records (export_wide); for closest
-// hit, whose (id, t) does not depend on the visit order, and for occlusion
-// sets (any hit read only as hit / miss).
-template <bool ANY_T, bool COUNT, int S, int BLOCK, bool MULTI, bool SPEC, bool PAIR = false, bool WIDE = false>
-__device__ __forceinline__ void trace_body(const TraceArgs& a, const BatchDesc* tab, uint32_t nb, uint32_t nrays,
-                                           uint32_t n0 = 0) {
-    __shared__ int lstack[S * BLOCK];
-    int spill[kMaxStack - S];
-    const int tid = threadIdx.x;
-    const uint32_t lane = __lane_id();
-    const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+// The last block out resets the launch's counters.
+template <bool MULTI>
+__device__ __forceinline__ void end_launch(const TraceArgs& a) {
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        __threadfence();
+        if (atomicAdd(a.counter + 1, 1u) == gridDim.x - 1) {
+            atomicExch(a.counter + 1, 0u);
+            if (MULTI) {
+                atomicExch(a.counter + 0, 0u);
+            } else {
+                // unrolled: as a loop it took the batched kernel from 71 to
+                // 81 VGPRs (7 -> 5 waves per SIMD)
+#pragma unroll
+                for (uint32_t b = 0; b < kRayBands; b++) atomicExch(a.counter + kBandStride * (b + 1), 0u);
+            }
+        }
+    }
+}
 
-    // The upload refuses trees deep enough to fill the stack, so the else
-    // branch is unreachable for a library BVH; it flags the launch instead of
-    // writing past the stack.
+// The traversal stack of a lane: entries 0..S-1 in LDS (lstack), deeper ones
+// in private memory (spill).  The upload refuses trees deep enough to fill
+// it, so the else branch of a push is unreachable for a library BVH; it
+// flags the launch instead of writing past the stack.
 #define RB_PUSH(v)                                            \
     do {                                                      \
         if (sp + 1 < kMaxStack) {                             \
@@ -205,37 +226,409 @@ __device__ __forceinline__ void trace_body(const TraceArgs& a, const BatchDesc* 
             atomicOr(a.errors, (uint32_t)RB_TRACE_ERR_STACK); \
         }                                                     \
     } while (0)
-    // Pops happen only at sp >= 0 (the sentinel at entry 0 ends the ray).  The
-    // LDS read is unconditional (the empty asm takes its value, so it cannot
-    // be folded away) and the spill read a separate branch: a select between
-    // the two arrays would become one generic (flat) load, which waits on
-    // both the vector-memory and the LDS counters.
-#define RB_POP(dst)                                                        \
-    do {                                                                   \
-        int v_ = lstack[(sp < S ? sp : S - 1) * BLOCK + tid];              \
-        asm volatile("" : "+v"(v_));                                       \
-        if (sp >= S) v_ = spill[sp - S];                                   \
-        (dst) = v_;                                                        \
-        --sp;                                                              \
+// Pops happen only at sp >= 0 (the sentinel at entry 0 ends the ray).  The
+// LDS read is unconditional (the empty asm takes its value, so it cannot be
+// folded away) and the spill read a separate branch: a select between the
+// two arrays would become one generic (flat) load, which waits on both the
+// vector-memory and the LDS counters.
+#define RB_POP(dst)                                          \
+    do {                                                     \
+        int v_ = lstack[(sp < S ? sp : S - 1) * BLOCK + tid]; \
+        asm volatile("" : "+v"(v_));                         \
+        if (sp >= S) v_ = spill[sp - S];                     \
+        (dst) = v_;                                          \
+        --sp;                                                \
     } while (0)
+
+// Claims of a wave on the launch's rays (wave-uniform).  Rays are split into
+// kRayBands contiguous ranges of chunk-multiple length: a wave claims from
+// the band of its XCD until that runs out, then from the next band in turn,
+// so every ray is claimed exactly once.  A batched launch claims in order
+// from counter word 0: its batches come from several scenes, and with bands
+// the chip works on up to eight of them at once, more than the Infinity
+// Cache holds (config-4 batches 2.97-3.01 against 3.48-3.49 Grays/s).
+template <bool MULTI>
+struct RayPool {
+    uint32_t next = 0, end = 0;  // claimed rays not handed out yet
+    uint32_t band = 0, band_len = 0;
+    bool drained = false;  // nothing left to claim
+    __device__ __forceinline__ void init(const TraceArgs& a, uint32_t nrays) {
+        if (MULTI) return;
+        band_len = ((nrays + kRayBands - 1) / kRayBands + a.chunk - 1) / a.chunk * a.chunk;
+        asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(band));
+        band &= kRayBands - 1;
+    }
+    // Hands rays to the lanes of mask m by rank; *mine is this lane's ray.
+    // Returns whether this lane got one (lanes outside m: false).
+    __device__ __forceinline__ bool take(const TraceArgs& a, uint32_t nrays, uint64_t m, uint32_t* mine) {
+        const uint32_t lane = __lane_id();
+        const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+        const uint32_t want = __popcll(m);
+        const uint32_t avail = end - next;
+        uint32_t base = next;  // lanes past the claimed ones: base + rank
+        uint32_t got = want;
+        *mine = base + rank;
+        if (avail < want) {
+            const int leader = __builtin_ctzll(m);
+            base = nrays;  // every band claimed: nothing for the lanes past `avail`
+            uint32_t lim = nrays;
+            if ((int)lane == leader) {
+                if (MULTI) {
+                    base = atomicAdd(a.counter, a.chunk);
+                    if (base > nrays) base = nrays;
+                } else {
+                    for (uint32_t t = 0; t < kRayBands; t++) {
+                        const uint32_t o = atomicAdd(a.counter + kBandStride * (band + 1), a.chunk);
+                        if (o < band_len && band * band_len + o < nrays) {  // the last band ends at nrays
+                            base = band * band_len + o;
+                            break;
+                        }
+                        band = (band + 1) & (kRayBands - 1);
+                    }
+                }
+            }
+            base = __builtin_amdgcn_readlane(base, leader);
+            band = MULTI ? 0u : __builtin_amdgcn_readlane(band, leader);
+            drained = base >= nrays;
+            if (nrays - base > a.chunk) lim = base + a.chunk;
+            const uint32_t more = want - avail < lim - base ? want - avail : lim - base;
+            if (rank >= avail) *mine = base + (rank - avail);
+            got = avail + more;
+            next = base + more;
+            end = lim;
+        } else {
+            next += want;
+        }
+        return ((m >> lane) & 1u) && rank < got;
+    }
+};
+
+// One 64-byte record per lane (rec, 64-byte aligned) into the wave's 4 KB of
+// LDS: load k brings the records of lane k of every quad, its quad's lanes
+// 16 bytes each, row (j ^ k) of it at 16-byte slot j of the quad's 64 bytes,
+// so the lanes of a quad read one row of theirs from different banks.  The L1
+// cache serves a record with one 64-byte access this way; 16 bytes per lane of
+// 64 records are 64 accesses per load, and their rate bound large launches:
+// 340 M -> 130 M accesses on 2 Mi diffuse rays at 1M triangles, 745 -> 684 us,
+// and a path-traced frame of 2M triangles 24.1 -> 19.3 ms.
+__device__ __forceinline__ void stage_records(const V4f* rec, uint32_t lane, V4f* stage) {
+    const uint64_t p = (uint64_t)rec;
+    const int lo = (int)(uint32_t)p, hi = (int)(uint32_t)(p >> 32);
+    const uint32_t row = (lane & 3) * 16;
+#define RB_STAGE(k)                                                                                            \
+    do {                                                                                                       \
+        const uint32_t l_ = (uint32_t)__builtin_amdgcn_mov_dpp(lo, 0x55 * (k), 0xF, 0xF, true) | (row ^ (16 * (k))); \
+        const uint32_t h_ = (uint32_t)__builtin_amdgcn_mov_dpp(hi, 0x55 * (k), 0xF, 0xF, true);                 \
+        const uint64_t q_ = (uint64_t)h_ << 32 | l_;                                                           \
+        __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void*)q_,                          \
+                                         (__attribute__((address_space(3))) void*)(stage + 64 * (k)), 16, 0, 0); \
+    } while (0)
+    RB_STAGE(0);
+    RB_STAGE(1);
+    RB_STAGE(2);
+    RB_STAGE(3);
+#undef RB_STAGE
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+// One traversal body for every launch form but the speculative one.
+// PAIR: rays [0, n0) are the first set (a.rays / a.hits; any hit when
+// a.any0), rays [n0, nrays) the closest-hit set (a.rays2 / a.hits2).
+// WIDE: a.nodes holds wide (4-child) records; for closest hit, whose (id, t)
+// does not depend on the visit order, and for occlusion sets (any hit read
+// only as hit / miss).
+//
+// A step loop: in one iteration every lane of the wave does one step of its
+// own ray, a node record or one triangle of a leaf, and the records of both
+// kinds are loaded together before either kind of step runs.  The launch is
+// bound by VALU issue (2 Mi diffuse rays, 1M triangles: 85% of the issue
+// slots; 348 M instructions per launch), with the drain of the last rays
+// behind it, so what counts is instructions per step and the lanes each
+// instruction serves.  Measured on that launch against a node loop and a leaf
+// loop in turn over power-of-two records (lanes that reached a leaf waited
+// for the rest, lanes without one for the longest leaf): 504 M instructions
+// and 36% of their lanes at work before, 0.935 -> 0.684 ms; 1920x1080 camera
+// rays of 200k triangles 0.486 -> 0.410 ms; a 1024x1024x8-spp path-traced
+// frame of 2M triangles 21.9 -> 19.3 ms.  Tried and left out: the top of the
+// tree in LDS (a branch per step, more than it saved), and waves of a
+// workgroup joining their last rays in one of them (720 against 684 us: the
+// drain waits for the longest ray's steps, not for issue slots).  A ray still
+// tests its nodes and leaves in its own order, whatever the other rays of its
+// wave do, so results are the same run to run and launch shape to launch
+// shape.
+template <bool ANY_T, bool COUNT, int S, int BLOCK, bool MULTI, bool PAIR, bool WIDE>
+__device__ __forceinline__ void trace_steps(const TraceArgs& a, const BatchDesc* tab, uint32_t nb, uint32_t nrays,
+                                            uint32_t n0 = 0) {
+    __shared__ int lstack[S * BLOCK];
+    __shared__ V4f staged[4 * BLOCK];
+    int spill[kMaxStack - S];
+    const int tid = threadIdx.x;
+    const uint32_t lane = __lane_id();
+    // this wave's 64 staged records (wave-uniform), and where this lane's lies
+    V4f* const stage = staged + 256 * __builtin_amdgcn_readfirstlane(tid >> 6);
+    const V4f* const mine_staged = stage + 64 * (lane & 3) + 4 * (lane >> 2);
+
+    lstack[tid] = kSentinel;
+    RayPool<MULTI> pool;
+    pool.init(a, nrays);
+    // cur: the ray's next step -- an inner record (>= 0), a leaf's remaining
+    // triangles ~(first << 5 | count), or kSentinel when the ray is done
+    int cur = kSentinel, sp = 0, hitId = -1;
+    bool live = false;  // the lane holds a ray whose result is not stored yet
+    uint32_t mine = 0;  // the ray's index in the launch
+    uint32_t batch = 0;  // MULTI: its batch
+    float ox = 0.f, oy = 0.f, oz = 0.f, tmin = 0.f, dx = 0.f, dy = 0.f, dz = 0.f, hitT = 0.f;
+    float idx_ = 0.f, idy_ = 0.f, idz_ = 0.f, oodx = 0.f, oody = 0.f, oodz = 0.f;
+    uint32_t c_inner = 0, c_tri = 0, c_leaf = 0;
+    // scene of the lane's current ray (uniform in single-batch mode); a lane
+    // that has had no ray yet still loads a record with its quad, the first
+    // scene's root
+    GF4 nodes = MULTI ? (GF4)tab[0].nodes : (GF4)a.nodes;
+    GF4 tris = MULTI ? (GF4)tab[0].tris : (GF4)a.tris;
+    // where the lane's ray came from: looked up again at its rare uses
+    // instead of carried in registers through every step
+    auto second = [&]() -> bool { return PAIR && mine >= n0; };
+    auto any = [&]() -> bool { return MULTI ? tab[batch].any != 0 : PAIR ? !second() && a.any0 != 0 : ANY_T; };
+    auto rayidx = [&]() -> uint32_t { return MULTI ? mine - tab[batch].start : second() ? mine - n0 : mine; };
+    auto rays = [&]() -> GF4 { return MULTI ? (GF4)tab[batch].rays : second() ? (GF4)a.rays2 : (GF4)a.rays; };
+    auto hits = [&]() -> GI2 { return MULTI ? (GI2)tab[batch].hits : second() ? (GI2)a.hits2 : (GI2)a.hits; };
+
+    while (true) {
+        // ---- refill (wave-uniform control): results of the finished rays
+        // out, new rays in, once too few lanes are busy ----
+        const uint64_t tm = __ballot(cur == kSentinel);
+        const uint32_t busy = 64 - __popcll(tm);
+        if (busy == 0 || (!pool.drained && busy < a.threshold)) {
+            if (cur == kSentinel && live) {
+                const size_t i = rayidx();
+                V2i r;
+                if (hitId < 0) {  // a miss reports the caller's tmax, bit for bit
+                    r.x = -1;
+                    r.y = __float_as_int(((const __attribute__((address_space(1))) float*)(rays() + 2 * i + 1))[3]);
+                } else {
+                    r.x = hitId;
+                    r.y = __float_as_int(hitT);
+                }
+                hits()[i] = r;
+                if (COUNT) {
+                    a.counts[3 * i + 0] = c_inner;
+                    a.counts[3 * i + 1] = c_tri;
+                    a.counts[3 * i + 2] = c_leaf;
+                }
+                live = false;
+            }
+            if (pool.drained) break;
+            uint32_t ray;
+            if (pool.take(a, nrays, tm, &ray)) {
+                mine = ray;
+                const uint8_t* mk = a.mask;
+                if (MULTI) {
+                    // the last batch starting at or before `mine` (empty
+                    // batches share their successor's start)
+                    uint32_t lo = 0, hi = nb;
+                    while (hi - lo > 1) {
+                        const uint32_t mid = (lo + hi) >> 1;
+                        if (tab[mid].start <= mine) lo = mid;
+                        else hi = mid;
+                    }
+                    batch = lo;
+                    nodes = (GF4)tab[lo].nodes;
+                    tris = (GF4)tab[lo].tris;
+                    mk = tab[lo].mask;
+                }
+                const uint32_t i = rayidx();
+                const V4f o = rays()[2 * (size_t)i];
+                const V4f d = rays()[2 * (size_t)i + 1];
+                ox = o.x; oy = o.y; oz = o.z;
+                dx = d.x; dy = d.y; dz = d.z;
+                // quiet copies for the slab min / max (comparisons treat every
+                // NaN alike)
+                tmin = __builtin_canonicalizef(o.w);
+                hitT = __builtin_canonicalizef(d.w);
+                const float ooeps = 0x1p-80f;
+                idx_ = rcp_rn(fabsf(dx) > ooeps ? dx : copysignf(ooeps, dx));
+                idy_ = rcp_rn(fabsf(dy) > ooeps ? dy : copysignf(ooeps, dy));
+                idz_ = rcp_rn(fabsf(dz) > ooeps ? dz : copysignf(ooeps, dz));
+                oodx = ox * idx_;
+                oody = oy * idy_;
+                oodz = oz * idz_;
+                sp = 0;
+                hitId = -1;
+                live = true;
+                cur = (mk && mk[i] == 0) ? kSentinel : 0;
+                if (COUNT) { c_inner = 0; c_tri = 0; c_leaf = 0; }
+            }
+            continue;
+        }
+
+        // ---- one step of every busy lane's ray ----
+        const bool at_node = (uint32_t)cur < (uint32_t)kSentinel;
+        // triangles wait until few enough lanes are at a node
+        const bool tri_now = __popcll(__ballot(at_node)) <= a.leaf_gate;
+        const bool at_tri = tri_now && cur < 0;
+        const V4f* const rec = (const V4f*)(at_tri ? tris + 4 * (size_t)(~(uint32_t)cur >> 5)
+                                                   : nodes + 4 * (size_t)(at_node ? cur : 0));
+        stage_records(rec, lane, stage);
+        const V4f r0 = mine_staged[0 ^ (lane & 3)], r1 = mine_staged[1 ^ (lane & 3)], r2 = mine_staged[2 ^ (lane & 3)],
+                  r3 = mine_staged[3 ^ (lane & 3)];
+        asm volatile("" ::"v"(r0.x), "v"(r1.x), "v"(r2.x), "v"(r3.x) : "memory");
+        bool pop = false;
+        if (at_node) {
+            if (COUNT) c_inner++;
+            const V4i lk4 = __builtin_bit_cast(V4i, r3);
+            if (WIDE) {
+                // the four children's slab tests, then the nearest hit child
+                // next and the others pushed
+                const V4i q1 = __builtin_bit_cast(V4i, r1), q2 = __builtin_bit_cast(V4i, r2);
+                const float sx = r0.w * idx_, sy = r1.x * idy_, sz = r1.y * idz_;
+                // (a step that overflows, a scene past 4e9 units and a ray
+                // along an axis plane, makes its axis NaN, which the min and
+                // max below leave out: the box is not culled by that axis)
+                const float bx = fmaf(sx, 0.0f, fmaf(r0.x, idx_, -oodx));
+                const float by = fmaf(sy, 0.0f, fmaf(r0.y, idy_, -oody));
+                const float bz = fmaf(sz, 0.0f, fmaf(r0.z, idz_, -oodz));
+                const uint32_t wnx = idx_ < 0.0f ? q1.w : q1.z, wfx = idx_ < 0.0f ? q1.z : q1.w;
+                const uint32_t wny = idy_ < 0.0f ? q2.y : q2.x, wfy = idy_ < 0.0f ? q2.x : q2.y;
+                const uint32_t wnz = idz_ < 0.0f ? q2.w : q2.z, wfz = idz_ < 0.0f ? q2.z : q2.w;
+                int lnk[4] = {lk4.x, lk4.y, lk4.z, lk4.w};
+                int key[4];  // entry distance as an integer (in order from 0 up), kMiss past every float
+                constexpr int kMiss = 0x7FFFFFFF;
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    float nx[2], ny[2], nz[2], fx[2], fy[2], fz[2];
+                    walk_planes(wnx, h, sx, bx, nx);
+                    walk_planes(wny, h, sy, by, ny);
+                    walk_planes(wnz, h, sz, bz, nz);
+                    walk_planes(wfx, h, sx, bx, fx);
+                    walk_planes(wfy, h, sy, by, fy);
+                    walk_planes(wfz, h, sz, bz, fz);
+#pragma unroll
+                    for (int c = 0; c < 2; c++) {
+                        const float near = vmax3_(nx[c], ny[c], vmax_(nz[c], tmin));
+                        const float far = vmin3_(fx[c], fy[c], vmin_(fz[c], hitT));
+                        key[2 * h + c] = fmaf(fabsf(far), 0x1p-22f, far) >= near ? __float_as_int(near) : kMiss;
+                    }
+                    // two children at a time: all four at once take 89
+                    // registers, past the 80 that six waves per SIMD leave
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                // the nearest to slot 0, the next candidate to slot 2: the
+                // full sort (two more exchanges) reads 1.5-2% fewer records,
+                // less than its instructions cost
+#define RB_CS(i, j)                 \
+    if (key[j] < key[i]) {          \
+        const int tk = key[i];      \
+        key[i] = key[j];            \
+        key[j] = tk;                \
+        const int tl = lnk[i];      \
+        lnk[i] = lnk[j];            \
+        lnk[j] = tl;                \
+    }
+                RB_CS(0, 1) RB_CS(2, 3) RB_CS(0, 2)
+#undef RB_CS
+                if (key[0] == kMiss) {
+                    pop = true;
+                } else {
+                    cur = lnk[0];
+                    if (sp + 3 < S) {
+                        // straight-line stores: one of a missed child is
+                        // above the new top and overwritten by the next
+                        lstack[(sp + 1) * BLOCK + tid] = lnk[3];
+                        sp += key[3] != kMiss;
+                        lstack[(sp + 1) * BLOCK + tid] = lnk[1];
+                        sp += key[1] != kMiss;
+                        lstack[(sp + 1) * BLOCK + tid] = lnk[2];
+                        sp += key[2] != kMiss;
+                    } else {
+                        if (key[3] != kMiss) RB_PUSH(lnk[3]);
+                        if (key[1] != kMiss) RB_PUSH(lnk[1]);
+                        if (key[2] != kMiss) RB_PUSH(lnk[2]);
+                    }
+                }
+            } else {
+                const float c0lox = fmaf(r0.x, idx_, -oodx), c0hix = fmaf(r0.y, idx_, -oodx);
+                const float c0loy = fmaf(r0.z, idy_, -oody), c0hiy = fmaf(r0.w, idy_, -oody);
+                const float c0loz = fmaf(r2.x, idz_, -oodz), c0hiz = fmaf(r2.y, idz_, -oodz);
+                const float c1loz = fmaf(r2.z, idz_, -oodz), c1hiz = fmaf(r2.w, idz_, -oodz);
+                const float c1lox = fmaf(r1.x, idx_, -oodx), c1hix = fmaf(r1.y, idx_, -oodx);
+                const float c1loy = fmaf(r1.z, idy_, -oody), c1hiy = fmaf(r1.w, idy_, -oody);
+                const float c0min = vmax3_(vmin_(c0lox, c0hix), vmin_(c0loy, c0hiy), vmax_(vmin_(c0loz, c0hiz), tmin));
+                const float c0max = vmin3_(vmax_(c0lox, c0hix), vmax_(c0loy, c0hiy), vmin_(vmax_(c0loz, c0hiz), hitT));
+                const float c1min = vmax3_(vmin_(c1lox, c1hix), vmin_(c1loy, c1hiy), vmax_(vmin_(c1loz, c1hiz), tmin));
+                const float c1max = vmin3_(vmax_(c1lox, c1hix), vmax_(c1loy, c1hiy), vmin_(vmax_(c1loz, c1hiz), hitT));
+                const bool swp = c1min < c0min;
+                const bool t0 = c0max >= c0min;
+                const bool t1 = c1max >= c1min;
+                if (!t0 && !t1) {
+                    pop = true;
+                } else {
+                    const bool second = t1 && (!t0 || swp);
+                    cur = second ? lk4.y : lk4.x;
+                    if (t0 && t1) RB_PUSH(second ? lk4.x : lk4.y);
+                }
+            }
+            if (COUNT && !pop && cur < 0) c_leaf++;
+        }
+        if (at_tri) {
+            const uint32_t l = ~(uint32_t)cur;
+            const int id = __float_as_int(r3.x);
+            // (binary records may link an empty leaf: count 0; its record is the
+            // next leaf's first, or the zero one)
+            bool done = (l & 31u) <= 1u;
+            cur = (int)~(l + 31u);  // first + 1, count - 1
+            if (WIDE || (l & 31u) != 0u) {
+                if (COUNT) c_tri++;
+                const float Oz = fmaf(-oz, r0.z, fmaf(-oy, r0.y, fmaf(-ox, r0.x, r0.w)));
+                const float invDz = rcp_rn(fmaf(dz, r0.z, fmaf(dy, r0.y, dx * r0.x)));
+                const float t = Oz * invDz;
+                const float Ox = fmaf(oz, r1.z, fmaf(oy, r1.y, fmaf(ox, r1.x, r1.w)));
+                const float Dx = fmaf(dz, r1.z, fmaf(dy, r1.y, dx * r1.x));
+                const float u = fmaf(t, Dx, Ox);
+                const float Oy = fmaf(oz, r2.z, fmaf(oy, r2.y, fmaf(ox, r2.x, r2.w)));
+                const float Dy = fmaf(dz, r2.z, fmaf(dy, r2.y, dx * r2.x));
+                const float v = fmaf(t, Dy, Oy);
+                // ties at equal t go to the lowest id
+                const bool nearer = t < hitT || (t == hitT && id < hitId);
+                if (t > tmin && nearer && u >= 0.0f && v >= 0.0f && u + v <= 1.0f) {
+                    hitT = t;
+                    hitId = id;
+                    if (any()) {
+                        cur = kSentinel;
+                        done = false;
+                    }
+                }
+            }
+            pop |= done;
+        }
+        if (pop) {
+            RB_POP(cur);
+            if (COUNT && cur < 0) c_leaf++;
+        }
+    }
+    end_launch<MULTI>(a);
+}
+
+// The reference's speculative order over the binary records (rb_trace_config
+// .speculative): a lane that holds a leaf keeps walking inner nodes until the
+// whole wave holds leaves.
+template <bool ANY_T, bool COUNT, int S, int BLOCK, bool MULTI>
+__device__ __forceinline__ void trace_spec(const TraceArgs& a, const BatchDesc* tab, uint32_t nb, uint32_t nrays) {
+    __shared__ int lstack[S * BLOCK];
+    int spill[kMaxStack - S];
+    const int tid = threadIdx.x;
+    const uint32_t lane = __lane_id();
+    const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
 
     lstack[tid] = kSentinel;
     // top of the tree (the layout's first records, breadth-first) in LDS
     extern __shared__ V4f lnodes[];
     const uint32_t top = MULTI ? 0u : a.top_nodes;
-    if (top) {  // 4 float4 rows per record, binary or wide
+    if (top) {
         const GF4 src = (GF4)a.nodes;
         for (uint32_t i = tid; i < 4 * top; i += BLOCK) lnodes[i] = src[i];
         __syncthreads();
     }
     uint32_t pool_next = 0, pool_end = 0;
-    // ray bands: kRayBands contiguous ranges of chunk-multiple length; a
-    // wave claims from the band of its XCD until that runs out, then from
-    // the next band in turn (so every ray is claimed exactly once).  A
-    // batched launch claims in order from counter word 0: its batches come
-    // from several scenes, and with bands the chip works on up to eight of
-    // them at once, more than the Infinity Cache holds (config-4 batches
-    // 2.97-3.01 against 3.48-3.49 Grays/s)
     const uint32_t band_len = MULTI ? 0u : ((nrays + kRayBands - 1) / kRayBands + a.chunk - 1) / a.chunk * a.chunk;
     uint32_t band = 0;
     if (!MULTI) {
@@ -294,13 +687,6 @@ __device__ __forceinline__ void trace_body(const TraceArgs& a, const BatchDesc* 
                 if (mine >= nrays) break;
                 GF4 rays = (GF4)a.rays;
                 rayidx = mine;
-                if (PAIR) {
-                    const bool second = mine >= n0;
-                    rays = second ? (GF4)a.rays2 : (GF4)a.rays;
-                    hits = second ? (GI2)a.hits2 : (GI2)a.hits;
-                    any = !second && a.any0 != 0;
-                    rayidx = second ? mine - n0 : mine;
-                }
                 const uint8_t* mk = a.mask;
                 if (MULTI) {
                     // the last batch starting at or before `mine` (empty
@@ -347,94 +733,7 @@ __device__ __forceinline__ void trace_body(const TraceArgs& a, const BatchDesc* 
 
         // ---- traversal ----
         while (nodeAddr != kSentinel) {
-            while (WIDE && (uint32_t)nodeAddr < (uint32_t)kSentinel && leafAddr >= 0) {
-                // a wide record: the four children's slab tests on their
-                // decoded boxes, then the hit children nearest first (the
-                // rest pushed, farthest deepest)
-                V4f r0;
-                V4i r1, r2, r3;
-                if ((uint32_t)nodeAddr < top) {
-                    const V4f* ln = lnodes + 4 * nodeAddr;
-                    r0 = ln[0];
-                    r1 = __builtin_bit_cast(V4i, ln[1]);
-                    r2 = __builtin_bit_cast(V4i, ln[2]);
-                    r3 = __builtin_bit_cast(V4i, ln[3]);
-                } else {
-                    const GF4 np = nodes + 4 * (size_t)nodeAddr;
-                    r0 = np[0];
-                    r1 = *(GI4)(np + 1);
-                    r2 = *(GI4)(np + 2);
-                    r3 = *(GI4)(np + 3);
-                    asm volatile("" ::"v"(r0.x), "v"(r1.x), "v"(r2.x), "v"(r3.x));
-                }
-                if (COUNT) c_inner++;
-                // step sizes 2^e from the biased exponents (bytes of word 3)
-                const uint32_t eb = __float_as_uint(r0.w);
-                const float sx = __uint_as_float((eb & 0xFFu) << 23);
-                const float sy = __uint_as_float(((eb >> 8) & 0xFFu) << 23);
-                const float sz = __uint_as_float(((eb >> 16) & 0xFFu) << 23);
-                const int lk[4] = {r2.z, r2.w, r3.x, r3.y};
-                float key[4];
-                int lnk[4];
-#pragma unroll
-                for (int c = 0; c < 4; c++) {
-#define RB_Q(w, s, p) fmaf((float)(((uint32_t)(w) >> (8 * c)) & 0xFFu), s, p)
-                    const float lx = RB_Q(r1.x, sx, r0.x), hx = RB_Q(r1.y, sx, r0.x);
-                    const float ly = RB_Q(r1.z, sy, r0.y), hy = RB_Q(r1.w, sy, r0.y);
-                    const float lz = RB_Q(r2.x, sz, r0.z), hz = RB_Q(r2.y, sz, r0.z);
-#undef RB_Q
-                    const float clox = fmaf(lx, idx_, -oodx), chix = fmaf(hx, idx_, -oodx);
-                    const float cloy = fmaf(ly, idy_, -oody), chiy = fmaf(hy, idy_, -oody);
-                    const float cloz = fmaf(lz, idz_, -oodz), chiz = fmaf(hz, idz_, -oodz);
-                    const float cmin = vmax3_(vmin_(clox, chix), vmin_(cloy, chiy), vmax_(vmin_(cloz, chiz), tmin));
-                    const float cmax = vmin3_(vmax_(clox, chix), vmax_(cloy, chiy), vmin_(vmax_(cloz, chiz), hitT));
-                    const bool h = cmax >= cmin && lk[c] != kWideEmpty;
-                    // a hit box's key stays finite (misses sort last as inf)
-                    key[c] = h ? fminf(cmin, 0x1.fffffep127f) : __builtin_inff();
-                    lnk[c] = lk[c];
-                }
-                // sort the four (entry distance, link) pairs, misses last
-#define RB_CS(i, j)                                   \
-    if (key[j] < key[i]) {                            \
-        const float tk = key[i];                      \
-        key[i] = key[j];                              \
-        key[j] = tk;                                  \
-        const int tl = lnk[i];                        \
-        lnk[i] = lnk[j];                              \
-        lnk[j] = tl;                                  \
-    }
-                RB_CS(0, 1) RB_CS(2, 3) RB_CS(0, 2) RB_CS(1, 3) RB_CS(1, 2)
-#undef RB_CS
-                // the hit children are a prefix of the sorted four
-                const int npush = (int)(key[1] != __builtin_inff()) + (int)(key[2] != __builtin_inff()) +
-                                  (int)(key[3] != __builtin_inff());
-                if (key[0] == __builtin_inff()) {
-                    RB_POP(nodeAddr);
-                } else {
-                    nodeAddr = lnk[0];
-                    if (sp + 3 < S) {
-                        // entries sp+1..sp+npush take lnk[npush..1]
-                        // (farthest deepest), written as three straight-line
-                        // stores: those past sp+npush lie above the new top
-                        const int e1 = npush == 3 ? lnk[3] : npush == 2 ? lnk[2] : lnk[1];
-                        const int e2 = npush == 3 ? lnk[2] : lnk[1];
-                        lstack[(sp + 1) * BLOCK + tid] = e1;
-                        lstack[(sp + 2) * BLOCK + tid] = e2;
-                        lstack[(sp + 3) * BLOCK + tid] = lnk[1];
-                        sp += npush;
-                    } else {
-                        if (npush == 3) RB_PUSH(lnk[3]);
-                        if (npush >= 2) RB_PUSH(lnk[2]);
-                        if (npush >= 1) RB_PUSH(lnk[1]);
-                    }
-                }
-                if (nodeAddr < 0 && leafAddr >= 0) {
-                    leafAddr = nodeAddr;
-                    RB_POP(nodeAddr);
-                }
-                if (__popcll(__ballot(1)) <= a.leaf_gate) break;
-            }
-            while (!WIDE && (uint32_t)nodeAddr < (uint32_t)kSentinel && (SPEC || leafAddr >= 0)) {
+            while ((uint32_t)nodeAddr < (uint32_t)kSentinel) {
                 V4f n0, n1, nz;
                 V4i lk;
                 if ((uint32_t)nodeAddr < top) {
@@ -489,11 +788,7 @@ __device__ __forceinline__ void trace_body(const TraceArgs& a, const BatchDesc* 
                     leafAddr = nodeAddr;
                     RB_POP(nodeAddr);
                 }
-                if (SPEC) {
-                    if (!__any(leafAddr >= 0)) break;
-                } else if (__popcll(__ballot(1)) <= a.leaf_gate) {
-                    break;  // the rest keep their place and go on after the leaf phase
-                }
+                if (!__any(leafAddr >= 0)) break;
             }
 
             while (leafAddr < 0) {
@@ -553,30 +848,19 @@ __device__ __forceinline__ void trace_body(const TraceArgs& a, const BatchDesc* 
             }
         }
     }
+    end_launch<MULTI>(a);
+}
+
 #undef RB_PUSH
 #undef RB_POP
-
-    __syncthreads();
-    if (tid == 0) {
-        __threadfence();
-        if (atomicAdd(a.counter + 1, 1u) == gridDim.x - 1) {
-            atomicExch(a.counter + 1, 0u);
-            if (MULTI) {
-                atomicExch(a.counter + 0, 0u);
-            } else {
-                // unrolled: as a loop it took the batched kernel from 71 to
-                // 81 VGPRs (7 -> 5 waves per SIMD)
-#pragma unroll
-                for (uint32_t b = 0; b < kRayBands; b++) atomicExch(a.counter + kBandStride * (b + 1), 0u);
-            }
-        }
-    }
-}
 
 template <bool ANY, bool COUNT, int S, int BLOCK, bool SPEC>
 __global__ __launch_bounds__(BLOCK) void k_trace(TraceArgs a) {
     const uint32_t nrays = a.n_dev ? __builtin_nontemporal_load(a.n_dev) : a.n;
-    trace_body<ANY, COUNT, S, BLOCK, false, SPEC>(a, nullptr, 0, nrays);
+    if (SPEC)
+        trace_spec<ANY, COUNT, S, BLOCK, false>(a, nullptr, 0, nrays);
+    else
+        trace_steps<ANY, COUNT, S, BLOCK, false, false, false>(a, nullptr, 0, nrays);
 }
 
 // Closest hit, or occlusion (ANY), over the wide records (COUNT: inner =
@@ -584,14 +868,14 @@ __global__ __launch_bounds__(BLOCK) void k_trace(TraceArgs a) {
 template <bool ANY, bool COUNT, int S, int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_trace_wide(TraceArgs a) {
     const uint32_t nrays = a.n_dev ? __builtin_nontemporal_load(a.n_dev) : a.n;
-    trace_body<ANY, COUNT, S, BLOCK, false, false, false, true>(a, nullptr, 0, nrays);
+    trace_steps<ANY, COUNT, S, BLOCK, false, false, true>(a, nullptr, 0, nrays);
 }
 
 template <int S, int BLOCK, bool WIDE>
 __global__ __launch_bounds__(BLOCK) void k_trace_pair(TraceArgs a) {
     const uint32_t n0 = __builtin_nontemporal_load(a.n_dev);
     const uint32_t n1 = __builtin_nontemporal_load(a.n_dev2);
-    trace_body<true, false, S, BLOCK, false, false, true, WIDE>(a, nullptr, 0, n0 + n1, n0);
+    trace_steps<true, false, S, BLOCK, false, true, WIDE>(a, nullptr, 0, n0 + n1, n0);
 }
 
 template <int S, int BLOCK, bool SPEC, bool WIDE>
@@ -614,7 +898,10 @@ __global__ __launch_bounds__(BLOCK) void k_trace_batch(TraceArgs a, BatchTable t
         s_total = sum;
     }
     __syncthreads();
-    trace_body<false, false, S, BLOCK, true, SPEC, false, WIDE>(a, tab, t.nb, s_total);
+    if (SPEC)
+        trace_spec<false, false, S, BLOCK, true>(a, tab, t.nb, s_total);
+    else
+        trace_steps<false, false, S, BLOCK, true, false, WIDE>(a, tab, t.nb, s_total);
 }
 
 // ---------------------------------------------------------------- launch --
@@ -672,6 +959,12 @@ static bool wide_walk(const rb_trace_config& cfg, rb_bvh_t bvh, uint32_t flags) 
     return cfg.wide && !cfg.speculative && bvh->wnodes && (!(flags & RB_ANY) || (flags & kOcclusion));
 }
 
+// Static LDS of a trace block: the stack and, in the step loop, a staged
+// 64-byte record per lane.
+static size_t trace_lds(const rb_trace_config& cfg) {
+    return (size_t)cfg.block * (4 * cfg.lds_stack + (cfg.speculative ? 0 : 64));
+}
+
 static uint32_t persistent_blocks(const rb_trace_config& cfg, uint64_t n) {
     const uint32_t waves = dev().num_cus * cfg.waves_per_cu;
     uint32_t blocks = waves * 64 / cfg.block;
@@ -705,7 +998,7 @@ rb_status launch_trace(rb_bvh_t bvh, const rb_ray* rays, uint32_t n, uint32_t fl
     TraceArgs a;
     std::memset(&a, 0, sizeof(a));
     a.nodes = bvh->nodes;
-    a.tris = bvh->tris;
+    a.tris = cfg.speculative ? bvh->tris : bvh->tris4;
     a.index = bvh->index;
     a.rays = reinterpret_cast<const float4*>(rays);
     a.mask = (flags & RB_MASKED) ? mask : nullptr;
@@ -717,13 +1010,11 @@ rb_status launch_trace(rb_bvh_t bvh, const rb_ray* rays, uint32_t n, uint32_t fl
     a.chunk = cfg.chunk;
     a.threshold = cfg.fetch_threshold;
     a.leaf_gate = cfg.leaf_gate;
-    a.top_nodes = cfg.lds_nodes < bvh->n_nodes ? cfg.lds_nodes : bvh->n_nodes;
-    if (wide) {  // wide records are 64 bytes too
-        a.nodes = bvh->wnodes;
-        a.top_nodes = cfg.lds_nodes < bvh->n_wnodes ? cfg.lds_nodes : bvh->n_wnodes;
-    }
+    if (wide) a.nodes = bvh->wnodes;
+    // top-of-tree records in LDS: the speculative walk only
+    a.top_nodes = !cfg.speculative ? 0 : cfg.lds_nodes < bvh->n_nodes ? cfg.lds_nodes : bvh->n_nodes;
     const size_t top_bytes = (size_t)a.top_nodes * 64;
-    const size_t lds = (size_t)cfg.lds_stack * cfg.block * 4 + top_bytes;
+    const size_t lds = trace_lds(cfg) + top_bytes;
     if (lds > dev().lds_per_block)
         return fail(RB_ERR_INVALID, "trace config needs %zu bytes of LDS per block (stack %u x %u lanes + %u node records); "
                     "the device allows %zu", lds, cfg.lds_stack, cfg.block, a.top_nodes, dev().lds_per_block);
@@ -763,7 +1054,7 @@ rb_status launch_trace_pair(rb_bvh_t bvh, const rb_ray* rays0, uint32_t cap0, co
     TraceArgs a;
     std::memset(&a, 0, sizeof(a));
     a.nodes = wide ? bvh->wnodes : bvh->nodes;
-    a.tris = bvh->tris;
+    a.tris = bvh->tris4;
     a.index = bvh->index;
     a.rays = reinterpret_cast<const float4*>(rays0);
     a.hits = reinterpret_cast<int2*>(hits0);
@@ -777,9 +1068,7 @@ rb_status launch_trace_pair(rb_bvh_t bvh, const rb_ray* rays0, uint32_t cap0, co
     a.chunk = cfg.chunk;
     a.threshold = cfg.fetch_threshold;
     a.leaf_gate = cfg.leaf_gate;
-    const uint32_t nrec = wide ? bvh->n_wnodes : bvh->n_nodes;
-    a.top_nodes = cfg.lds_nodes < nrec ? cfg.lds_nodes : nrec;
-    const size_t lds = (size_t)cfg.lds_stack * cfg.block * 4 + (size_t)a.top_nodes * 64;
+    const size_t lds = trace_lds(cfg);
     if (lds > dev().lds_per_block)
         return fail(RB_ERR_INVALID, "trace config needs %zu bytes of LDS per block; the device allows %zu", lds,
                     dev().lds_per_block);
@@ -787,7 +1076,7 @@ rb_status launch_trace_pair(rb_bvh_t bvh, const rb_ray* rays0, uint32_t cap0, co
     if (L.st != RB_OK) return L.st;
     if (!L.counter) return fail(RB_ERR_INVALID, "render graph: out of work-counter slots");
     a.counter = L.counter;
-    hipLaunchKernelGGL(k, dim3(persistent_blocks(cfg, a.n)), dim3(cfg.block), (size_t)a.top_nodes * 64, stream, a);
+    hipLaunchKernelGGL(k, dim3(persistent_blocks(cfg, a.n)), dim3(cfg.block), 0, stream, a);
     const hipError_t e = hipGetLastError();
     release_counter_slot(L, stream);
     if (e != hipSuccess) return hip_fail(e, "paired trace launch");
@@ -829,7 +1118,7 @@ static rb_status launch_trace_sets_pass(const BatchSet* b, uint32_t nb, hipStrea
             if (total + b[i].n > 0x7FFFFFFFull) break;  // the next launch takes it
             BatchDesc& d = t.d[t.nb++];
             d.nodes = wide ? b[i].bvh->wnodes : b[i].bvh->nodes;
-            d.tris = b[i].bvh->tris;
+            d.tris = cfg.speculative ? b[i].bvh->tris : b[i].bvh->tris4;
             d.index = b[i].bvh->index;
             d.rays = b[i].rays;
             d.hits = b[i].hits;
@@ -972,8 +1261,8 @@ rb_status rb_trace_autotune(rb_bvh_t bvh, const rb_ray* rays, uint32_t n, uint32
         const uint32_t stacks[] = {8, 12, 16, 20, 24};
         const uint32_t chunks[] = {64, 128, 256, 1024};
         const uint32_t thresholds[] = {0, 16, 32, 40, 48, 56, 60};
-        const uint32_t waves[] = {8, 12, 16, 24, 32};
-        const uint32_t gates[] = {0, 4, 8, 16, 24, 32};
+        const uint32_t waves[] = {8, 12, 16, 20, 24, 32};
+        const uint32_t gates[] = {16, 24, 32, 40, 48, 56, 63};
         const uint32_t tops[] = {0, 64, 128, 192, 256, 384};
         for (int pass = 0; pass < 2; pass++) {
             for (int dim = 0; dim < 7; dim++) {
@@ -984,11 +1273,12 @@ rb_status rb_trace_autotune(rb_bvh_t bvh, const rb_ray* rays, uint32_t n, uint32
                     case 1: vals = stacks; nv = 5; break;
                     case 2: vals = chunks; nv = 4; break;
                     case 3: vals = thresholds; nv = 7; break;
-                    case 4: vals = waves; nv = 5; break;
-                    case 5: vals = gates; nv = 6; break;
+                    case 4: vals = waves; nv = 6; break;
+                    case 5: vals = gates; nv = 7; break;
                     default: vals = tops; nv = 6; break;
                 }
-                if (dim == 5 && cur.speculative) continue;  // the gate only acts on the non-speculative order
+                if (dim == 5 && cur.speculative) continue;   // the gate acts on the step loop,
+                if (dim == 6 && !cur.speculative) continue;  // the records in LDS on the speculative walk
                 for (int k = 0; k < nv; k++) {
                     rb_trace_config c = cur;
                     uint32_t* f = dim == 0 ? &c.block : dim == 1 ? &c.lds_stack : dim == 2 ? &c.chunk
@@ -997,7 +1287,7 @@ rb_status rb_trace_autotune(rb_bvh_t bvh, const rb_ray* rays, uint32_t n, uint32
                     if (*f == vals[k]) continue;
                     *f = vals[k];
                     if (!pick<false, false>(c) ||
-                        (size_t)c.lds_stack * c.block * 4 + (size_t)c.lds_nodes * 64 > dev().lds_per_block)
+                        trace_lds(c) + (c.speculative ? (size_t)c.lds_nodes * 64 : 0) > dev().lds_per_block)
                         continue;  // no kernel for this shape, or more LDS than a block gets
                     float ms = 0.f;
                     if ((st = measure(c, &ms)) != RB_OK) goto done;
