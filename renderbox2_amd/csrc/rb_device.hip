@@ -48,10 +48,10 @@ static rb_status init_locked(int device) {
         (void)hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep);
     }
     // the best measured shape on 2 Mi incoherent rays at 1M triangles: a
-    // 256-thread block's 12-entry stacks and staged records take 28 KB of LDS,
+    // 256-thread block's 16-entry stacks and staged records take 31 KB of LDS,
     // which keeps 5 blocks (20 waves) on a CU
     g_dev.cfg.block = 256;
-    g_dev.cfg.lds_stack = 12;
+    g_dev.cfg.lds_stack = 16;
     g_dev.cfg.chunk = 64;
     g_dev.cfg.fetch_threshold = 52;
     g_dev.cfg.waves_per_cu = 20;

@@ -144,14 +144,14 @@ __device__ __forceinline__ float vmax3_(float a, float b, float c) {
     return r;
 }
 
-// Distances of one plane of two of a wide record's children (half h: 0 and
-// 1, or 2 and 3): their 8-bit steps, spread by one byte permute to the two
-// halves 0x00qq, which as half-precision numbers are q * 2^-24 (subnormal),
-// go straight into a mixed-precision fused multiply-add each, q s + b (the
-// record holds s * 2^24).
-__device__ __forceinline__ void walk_planes(uint32_t w, int h, float s, float b, float t[2]) {
+// Distances of one plane of two of a wide record's children: their 8-bit
+// steps, picked from the lo and hi words by the selector and spread by one
+// byte permute to the two halves 0x00qq, which as half-precision numbers are
+// q * 2^-24 (subnormal), go straight into a mixed-precision fused
+// multiply-add each, q s + b (the record holds s * 2^24).
+__device__ __forceinline__ void walk_planes(uint32_t lo, uint32_t hi, uint32_t sel, float s, float b, float t[2]) {
     typedef _Float16 H2 __attribute__((ext_vector_type(2)));
-    const H2 p = __builtin_bit_cast(H2, __builtin_amdgcn_perm(0u, w, h ? 0x0C030C02u : 0x0C010C00u));
+    const H2 p = __builtin_bit_cast(H2, __builtin_amdgcn_perm(hi, lo, sel));
     t[0] = fmaf((float)p.x, s, b);
     t[1] = fmaf((float)p.y, s, b);
 }
@@ -359,16 +359,22 @@ __device__ __forceinline__ void stage_records(const V4f* rec, uint32_t lane, V4f
 template <bool ANY_T, bool COUNT, int S, int BLOCK, bool MULTI, bool PAIR, bool WIDE>
 __device__ __forceinline__ void trace_steps(const TraceArgs& a, const BatchDesc* tab, uint32_t nb, uint32_t nrays,
                                             uint32_t n0 = 0) {
-    __shared__ int lstack[S * BLOCK];
+    // the stack: S - 1 entries of each lane in LDS, lane-interleaved, deeper
+    // ones in private memory; empty, it gives the sentinel that ends the ray.
+    // (With S = 12, a lane in most waves is past the straight-line stores of
+    // a push and the wave goes through the branches of the deep ones; 15 rows
+    // are the most that keep 20 waves on a CU, which 16 did not: 671 us on 2
+    // Mi diffuse rays against 684 with 12 and 720 with 16)
+    constexpr int R = S - 1;
+    __shared__ int lstack[R * BLOCK];
     __shared__ V4f staged[4 * BLOCK];
-    int spill[kMaxStack - S];
+    int spill[kMaxStack - 1 - R];
     const int tid = threadIdx.x;
     const uint32_t lane = __lane_id();
     // this wave's 64 staged records (wave-uniform), and where this lane's lies
     V4f* const stage = staged + 256 * __builtin_amdgcn_readfirstlane(tid >> 6);
     const V4f* const mine_staged = stage + 64 * (lane & 3) + 4 * (lane >> 2);
 
-    lstack[tid] = kSentinel;
     RayPool<MULTI> pool;
     pool.init(a, nrays);
     // cur: the ray's next step -- an inner record (>= 0), a leaf's remaining
@@ -379,6 +385,11 @@ __device__ __forceinline__ void trace_steps(const TraceArgs& a, const BatchDesc*
     uint32_t batch = 0;  // MULTI: its batch
     float ox = 0.f, oy = 0.f, oz = 0.f, tmin = 0.f, dx = 0.f, dy = 0.f, dz = 0.f, hitT = 0.f;
     float idx_ = 0.f, idy_ = 0.f, idz_ = 0.f, oodx = 0.f, oody = 0.f, oodz = 0.f;
+    // byte selectors of a wide record's near and far planes by the sign of the
+    // direction (walk_planes): per axis near of children 0 and 1, of 2 and 3,
+    // far of both.  Set per ray: twelve registers for fifteen instructions
+    // less per record
+    uint32_t sel[3][4] = {};
     uint32_t c_inner = 0, c_tri = 0, c_leaf = 0;
     // scene of the lane's current ray (uniform in single-batch mode); a lane
     // that has had no ray yet still loads a record with its quad, the first
@@ -392,6 +403,29 @@ __device__ __forceinline__ void trace_steps(const TraceArgs& a, const BatchDesc*
     auto rayidx = [&]() -> uint32_t { return MULTI ? mine - tab[batch].start : second() ? mine - n0 : mine; };
     auto rays = [&]() -> GF4 { return MULTI ? (GF4)tab[batch].rays : second() ? (GF4)a.rays2 : (GF4)a.rays; };
     auto hits = [&]() -> GI2 { return MULTI ? (GI2)tab[batch].hits : second() ? (GI2)a.hits2 : (GI2)a.hits; };
+
+    // The upload refuses trees deep enough to fill the stack, so the last
+    // branch is unreachable for a library BVH; it flags the launch instead of
+    // writing past the stack.
+    auto push = [&](int v) {
+        if (sp < R)
+            lstack[sp++ * BLOCK + tid] = v;
+        else if (sp < kMaxStack - 1)
+            spill[sp++ - R] = v;
+        else
+            atomicOr(a.errors, (uint32_t)RB_TRACE_ERR_STACK);
+    };
+    // The LDS read is unconditional (the empty asm takes its value, so it
+    // cannot be folded away) and the spill read a separate branch: a select
+    // between the two arrays would become one generic (flat) load, which
+    // waits on both the vector-memory and the LDS counters.
+    auto pop_entry = [&]() -> int {
+        --sp;
+        int v = lstack[((uint32_t)sp < (uint32_t)R ? sp : R - 1) * BLOCK + tid];
+        asm volatile("" : "+v"(v));
+        if (sp >= R) v = spill[sp - R];
+        return sp < 0 ? kSentinel : v;
+    };
 
     while (true) {
         // ---- refill (wave-uniform control): results of the finished rays
@@ -452,6 +486,17 @@ __device__ __forceinline__ void trace_steps(const TraceArgs& a, const BatchDesc*
                 oodx = ox * idx_;
                 oody = oy * idy_;
                 oodz = oz * idz_;
+                if (WIDE) {
+                    const float dir[3] = {idx_, idy_, idz_};
+#pragma unroll
+                    for (int c = 0; c < 3; c++) {
+                        const bool neg = dir[c] < 0.0f;
+                        sel[c][0] = neg ? 0x0C050C04u : 0x0C010C00u;
+                        sel[c][1] = neg ? 0x0C070C06u : 0x0C030C02u;
+                        sel[c][2] = neg ? 0x0C010C00u : 0x0C050C04u;
+                        sel[c][3] = neg ? 0x0C030C02u : 0x0C070C06u;
+                    }
+                }
                 sp = 0;
                 hitId = -1;
                 live = true;
@@ -487,21 +532,18 @@ __device__ __forceinline__ void trace_steps(const TraceArgs& a, const BatchDesc*
                 const float bx = fmaf(sx, 0.0f, fmaf(r0.x, idx_, -oodx));
                 const float by = fmaf(sy, 0.0f, fmaf(r0.y, idy_, -oody));
                 const float bz = fmaf(sz, 0.0f, fmaf(r0.z, idz_, -oodz));
-                const uint32_t wnx = idx_ < 0.0f ? q1.w : q1.z, wfx = idx_ < 0.0f ? q1.z : q1.w;
-                const uint32_t wny = idy_ < 0.0f ? q2.y : q2.x, wfy = idy_ < 0.0f ? q2.x : q2.y;
-                const uint32_t wnz = idz_ < 0.0f ? q2.w : q2.z, wfz = idz_ < 0.0f ? q2.z : q2.w;
                 int lnk[4] = {lk4.x, lk4.y, lk4.z, lk4.w};
                 int key[4];  // entry distance as an integer (in order from 0 up), kMiss past every float
                 constexpr int kMiss = 0x7FFFFFFF;
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
                     float nx[2], ny[2], nz[2], fx[2], fy[2], fz[2];
-                    walk_planes(wnx, h, sx, bx, nx);
-                    walk_planes(wny, h, sy, by, ny);
-                    walk_planes(wnz, h, sz, bz, nz);
-                    walk_planes(wfx, h, sx, bx, fx);
-                    walk_planes(wfy, h, sy, by, fy);
-                    walk_planes(wfz, h, sz, bz, fz);
+                    walk_planes(q1.z, q1.w, sel[0][h], sx, bx, nx);
+                    walk_planes(q2.x, q2.y, sel[1][h], sy, by, ny);
+                    walk_planes(q2.z, q2.w, sel[2][h], sz, bz, nz);
+                    walk_planes(q1.z, q1.w, sel[0][2 + h], sx, bx, fx);
+                    walk_planes(q2.x, q2.y, sel[1][2 + h], sy, by, fy);
+                    walk_planes(q2.z, q2.w, sel[2][2 + h], sz, bz, fz);
 #pragma unroll
                     for (int c = 0; c < 2; c++) {
                         const float near = vmax3_(nx[c], ny[c], vmax_(nz[c], tmin));
@@ -530,19 +572,19 @@ __device__ __forceinline__ void trace_steps(const TraceArgs& a, const BatchDesc*
                     pop = true;
                 } else {
                     cur = lnk[0];
-                    if (sp + 3 < S) {
+                    if (sp + 3 <= R) {
                         // straight-line stores: one of a missed child is
                         // above the new top and overwritten by the next
-                        lstack[(sp + 1) * BLOCK + tid] = lnk[3];
+                        lstack[sp * BLOCK + tid] = lnk[3];
                         sp += key[3] != kMiss;
-                        lstack[(sp + 1) * BLOCK + tid] = lnk[1];
+                        lstack[sp * BLOCK + tid] = lnk[1];
                         sp += key[1] != kMiss;
-                        lstack[(sp + 1) * BLOCK + tid] = lnk[2];
+                        lstack[sp * BLOCK + tid] = lnk[2];
                         sp += key[2] != kMiss;
                     } else {
-                        if (key[3] != kMiss) RB_PUSH(lnk[3]);
-                        if (key[1] != kMiss) RB_PUSH(lnk[1]);
-                        if (key[2] != kMiss) RB_PUSH(lnk[2]);
+                        if (key[3] != kMiss) push(lnk[3]);
+                        if (key[1] != kMiss) push(lnk[1]);
+                        if (key[2] != kMiss) push(lnk[2]);
                     }
                 }
             } else {
@@ -564,7 +606,7 @@ __device__ __forceinline__ void trace_steps(const TraceArgs& a, const BatchDesc*
                 } else {
                     const bool second = t1 && (!t0 || swp);
                     cur = second ? lk4.y : lk4.x;
-                    if (t0 && t1) RB_PUSH(second ? lk4.x : lk4.y);
+                    if (t0 && t1) push(second ? lk4.x : lk4.y);
                 }
             }
             if (COUNT && !pop && cur < 0) c_leaf++;
@@ -601,7 +643,7 @@ __device__ __forceinline__ void trace_steps(const TraceArgs& a, const BatchDesc*
             pop |= done;
         }
         if (pop) {
-            RB_POP(cur);
+            cur = pop_entry();
             if (COUNT && cur < 0) c_leaf++;
         }
     }
