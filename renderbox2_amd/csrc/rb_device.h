@@ -208,6 +208,7 @@ struct rb_bvh_s {
     float4* nodes = nullptr;    // 4 float4 per inner node (MI355X layout)
     float4* wnodes = nullptr;   // 4 float4 per wide (4-child) record (export_wide)
     uint32_t n_wnodes = 0;
+    uint32_t stack = 0, wide_stack = 0;  // most stack entries a ray of the binary / wide walk can need
     float4* tris = nullptr;     // 3 float4 Woop rows per triangle reference
     float4* tris4 = nullptr;    // the same in 64 bytes each: 3 Woop rows, then id|0|0|0; one more, all zero
     uint32_t* index = nullptr;  // original triangle id per reference

@@ -334,6 +334,7 @@ rb_status rb_bvh_upload(rb_host_bvh_t hb, rb_scene_t scene, rb_bvh_t* out) {
     RB_ENSURE();
     Mi355Layout L;
     std::vector<uint32_t> wide;
+    uint32_t stack = 0, wide_stack = 0;
     try {
         rb_status st = export_mi355x(*hb->b, L);
         if (st != RB_OK) return st;
@@ -344,7 +345,8 @@ rb_status rb_bvh_upload(rb_host_bvh_t hb, rb_scene_t scene, rb_bvh_t* out) {
                         depth == UINT32_MAX ? "not a tree" : "too deep", kMaxStack);
         // wide records only where their walk fits the same stack and their
         // 8-bit steps can hold the boxes (else the binary walk alone)
-        st = export_walk(L.nodes, (uint32_t)L.index.size(), wide);
+        stack = depth + 1;  // one postponed child per record on the way
+        st = export_walk(L.nodes, (uint32_t)L.index.size(), wide, &wide_stack);
         if (st == RB_ERR_UNSUPPORTED) {
             wide.clear();
             set_error("");
@@ -372,6 +374,8 @@ rb_status rb_bvh_upload(rb_host_bvh_t hb, rb_scene_t scene, rb_bvh_t* out) {
     rb_status st;
     B->n_nodes = (uint32_t)(L.nodes.size() / 16);
     B->n_refs = (uint32_t)L.index.size();
+    B->stack = stack;
+    B->wide_stack = wide_stack;
     if ((st = up((void**)&B->nodes, L.nodes.data(), L.nodes.size() * 4)) != RB_OK) { cleanup(); return st; }
     B->n_wnodes = (uint32_t)(wide.size() / kWideWords);
     if (!wide.empty() && (st = up((void**)&B->wnodes, wide.data(), wide.size() * 4)) != RB_OK) { cleanup(); return st; }

@@ -199,7 +199,9 @@ rb_status export_wide(const std::vector<uint32_t>& bin, std::vector<uint32_t>& w
 // whenever it passes the binary walk's, every leaf the binary walk tests is
 // tested, and closest hits, which do not depend on the visit order (ties at
 // equal t go to the lowest triangle id), have the same (id, t).
-rb_status export_walk(const std::vector<uint32_t>& bin, uint32_t n_refs, std::vector<uint32_t>& walk);
+// *entries: the most stack entries a ray can need.
+rb_status export_walk(const std::vector<uint32_t>& bin, uint32_t n_refs, std::vector<uint32_t>& walk,
+                      uint32_t* entries);
 // Depth of the deepest inner record of an MI355X node array (root = 0);
 // UINT32_MAX when a link leaves the array or the links form a cycle.  A
 // traversal holds at most depth + 1 stack entries (the sentinel, then one

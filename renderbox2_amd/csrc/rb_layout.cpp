@@ -551,7 +551,8 @@ bool walk_axis(const WalkChild* ch, uint32_t k, int a, float* p_out, float* s_ou
 
 }  // namespace
 
-rb_status export_walk(const std::vector<uint32_t>& bin, uint32_t n_refs, std::vector<uint32_t>& walk) {
+rb_status export_walk(const std::vector<uint32_t>& bin, uint32_t n_refs, std::vector<uint32_t>& walk,
+                      uint32_t* entries) {
     const uint32_t n = (uint32_t)(bin.size() / 16);
     walk.clear();
     if (n == 0) return RB_OK;
@@ -574,13 +575,16 @@ rb_status export_walk(const std::vector<uint32_t>& bin, uint32_t n_refs, std::ve
         else P.split.assign(n, {2, 1, 0, 2});
         walk.clear();
         std::vector<uint32_t> order{0};  // binary record of each wide record
-        std::vector<uint32_t> held{1};   // stack entries in use, at most, when a ray reaches it (1: the sentinel)
-        uint32_t deepest = 1;
+        // stack entries in use, at most, when a ray reaches it: three more per
+        // level whatever the children (a ray with a NaN origin passes the
+        // boxes of empty slots too)
+        std::vector<uint32_t> held{0};
+        uint32_t deepest = 0;
         for (size_t h = 0; h < order.size(); h++) {
             WalkChild ch[4];
             uint32_t k = 0;
             walk_children(bin, P, order[h], 4, ch, &k);
-            const uint32_t below = held[h] + (k ? k - 1 : 0);
+            const uint32_t below = held[h] + 3;
             deepest = std::max(deepest, below);
             const size_t base = walk.size();
             walk.resize(base + kWideWords, 0);
@@ -614,7 +618,8 @@ rb_status export_walk(const std::vector<uint32_t>& bin, uint32_t n_refs, std::ve
             }
             if (order.size() > 0x7FFFFFF0u) return fail(RB_ERR_UNSUPPORTED, "too many BVH nodes");
         }
-        if (deepest + 3 < kTraceStackEntries) return RB_OK;
+        *entries = deepest;
+        if (deepest < kTraceStackEntries) return RB_OK;
     }
     walk.clear();
     return fail(RB_ERR_UNSUPPORTED, "the tree is too deep for the wide walk's stack");

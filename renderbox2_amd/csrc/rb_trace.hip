@@ -17,7 +17,8 @@
 //    cudatracer.cu:164-165), so concurrent launches and graph replays work;
 //  * step loop: in one iteration every lane of a wave does one step of its
 //    own ray, a node record or one triangle (trace_steps); records come in
-//    through LDS, 64 bytes per cache access (stage_records);
+//    through LDS, 64 bytes per cache access (stage_records); launches of few
+//    rays give each ray four lanes (trace_quads);
 //  * leaf order: a lane tests a leaf as soon as it reaches one, so every ray
 //    visits nodes and leaves in the same order whatever the other rays of its
 //    wave do -- the order of the single-ray restatement -- and results are
@@ -39,6 +40,8 @@
 //    at start and reads them from there.
 // Arithmetic (fp32, explicit fmaf, reciprocals equal to the IEEE division)
 // matches the oracle's restatement bit for bit.
+#include <algorithm>
+
 #include "rb_device.h"
 
 namespace rb {
@@ -65,6 +68,7 @@ struct TraceArgs {
     uint32_t threshold;
     uint32_t leaf_gate;  // non-speculative: leave the inner-node phase once <= this many lanes still search
     uint32_t top_nodes;  // node records 0..top_nodes-1 are read from a copy in LDS
+    uint32_t stack_rows;  // trace_quads: rows of four entries that a ray's stack can need
 };
 
 constexpr uint32_t kMaxBatch = 64;
@@ -154,6 +158,21 @@ __device__ __forceinline__ void walk_planes(uint32_t lo, uint32_t hi, uint32_t s
     const H2 p = __builtin_bit_cast(H2, __builtin_amdgcn_perm(hi, lo, sel));
     t[0] = fmaf((float)p.x, s, b);
     t[1] = fmaf((float)p.y, s, b);
+}
+
+// The same for one child: the selector picks its step into the low half.
+__device__ __forceinline__ float walk_plane(uint32_t lo, uint32_t hi, uint32_t sel, float s, float b) {
+    typedef _Float16 H2 __attribute__((ext_vector_type(2)));
+    const H2 p = __builtin_bit_cast(H2, __builtin_amdgcn_perm(hi, lo, sel));
+    return fmaf((float)p.x, s, b);
+}
+
+// A value of another lane of the quad (lanes 4q..4q+3): of its lane 0 or 1,
+// of the other lane of the pair, of the same lane of the other pair.
+constexpr int kQuad0 = 0x00, kQuad1 = 0x55, kQuadXor1 = 0xB1, kQuadXor2 = 0x4E;
+template <int PERM>
+__device__ __forceinline__ int quad(int x) {
+    return __builtin_amdgcn_mov_dpp(x, PERM, 0xF, 0xF, true);
 }
 
 // Every single-precision bit pattern through rcp_rn's fast path and through
@@ -896,6 +915,208 @@ __device__ __forceinline__ void trace_spec(const TraceArgs& a, const BatchDesc* 
 #undef RB_PUSH
 #undef RB_POP
 
+// The step loop for launches of few rays: four lanes per ray, sixteen rays per
+// one-wave block, no refill and so no work counters.
+//
+// With a lane per ray such a launch takes as long as its longest ray, whose
+// steps wait for each other: 0.78 us a step, the chain of its instructions
+// (8-10 cycles for each that needs the one before, 80 for each branch that
+// part of the lanes take) and a record from L2 (240).  With a quad per ray
+// each lane tests one child of a record or one triangle of a leaf, a leaf of
+// four triangles is one step, and no lane branches: a wave skips the node or
+// the triangle half of a step when no lane is in it, and lanes with nothing to
+// push store to a spare row.  0.37 us a step.  Two children per record leave
+// half of the quad idle, but keep the latency.  Steps and arithmetic of a ray
+// and the order of its stack are trace_steps', so its result does not depend
+// on which of the two took it.
+//
+// Measured, trace_steps -> trace_quads (us), rays from surfaces among 1M
+// triangles: 64 rays 109 -> 54, 16 Ki 173 -> 95, 64 Ki 196 -> 129, 128 Ki 226
+// -> 188, 256 Ki 281 -> 282, 512 Ki 349 -> 485; first camera rays of 200k
+// triangles: 32 Ki 30 -> 10, 128 Ki 50 -> 25, 256 Ki 106 -> 66, 1 Mi 258 ->
+// 338; 4099 rays of 20k triangles 107 -> 48.  Any hit over the binary records:
+// 128 Ki 322 -> 251, 192 Ki 346 -> 336, 256 Ki 375 -> 394.  (The launch is
+// bound by VALU issue from about 100k rays on: a quad's node step is 105
+// instructions for 16 rays where the other loop's is 110 for up to 64.)  Rows
+// of the stack for what the tree can need, not for the most any tree may: 4 KB
+// a wave for 1M triangles, so that eight waves fit a SIMD (256 Ki rays 292 ->
+// 282).
+template <bool ANY_T, bool MULTI, bool PAIR, bool WIDE>
+__device__ __forceinline__ void trace_quads(const TraceArgs& a, const BatchDesc* tab, uint32_t nb, uint32_t nrays,
+                                            uint32_t n0 = 0) {
+    // a quad's stack: entry e in row e / 4, column e % 4 of its four words; the
+    // row behind the last takes the stores of lanes that have nothing to push
+    extern __shared__ int lstack[];
+    const int rows = (int)a.stack_rows;
+    const int lane = threadIdx.x, j = lane & 3;
+    if (blockIdx.x * 16 >= nrays) return;
+    uint32_t mine = blockIdx.x * 16 + ((uint32_t)lane >> 2);
+    const bool live = mine < nrays;
+    mine = live ? mine : 0u;
+    uint32_t batch = 0;
+    if (MULTI) {  // the last batch starting at or before `mine` (empty batches share their successor's start)
+        uint32_t lo = 0, hi = nb;
+        while (hi - lo > 1) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (tab[mid].start <= mine) lo = mid;
+            else hi = mid;
+        }
+        batch = lo;
+    }
+    const bool second = PAIR && mine >= n0;
+    const bool an = MULTI ? tab[batch].any != 0 : PAIR ? !second && a.any0 != 0 : ANY_T;
+    const GF4 nodes = MULTI ? (GF4)tab[batch].nodes : (GF4)a.nodes;
+    const GF4 tris = MULTI ? (GF4)tab[batch].tris : (GF4)a.tris;
+    const GF4 rays = MULTI ? (GF4)tab[batch].rays : second ? (GF4)a.rays2 : (GF4)a.rays;
+    const uint8_t* const mk = MULTI ? tab[batch].mask : a.mask;
+    const size_t ray = MULTI ? mine - tab[batch].start : second ? mine - n0 : mine;
+    const V4f o = rays[2 * ray], d = rays[2 * ray + 1];
+    const float ox = o.x, oy = o.y, oz = o.z, dx = d.x, dy = d.y, dz = d.z;
+    const float tmin = __builtin_canonicalizef(o.w);
+    float hitT = __builtin_canonicalizef(d.w);
+    const float ooeps = 0x1p-80f;
+    const float idx_ = rcp_rn(fabsf(dx) > ooeps ? dx : copysignf(ooeps, dx));
+    const float idy_ = rcp_rn(fabsf(dy) > ooeps ? dy : copysignf(ooeps, dy));
+    const float idz_ = rcp_rn(fabsf(dz) > ooeps ? dz : copysignf(ooeps, dz));
+    const float oodx = ox * idx_, oody = oy * idy_, oodz = oz * idz_;
+    const uint32_t selx = 0x0C0C0C00u | ((idx_ < 0.0f ? 4 : 0) + j);
+    const uint32_t sely = 0x0C0C0C00u | ((idy_ < 0.0f ? 4 : 0) + j);
+    const uint32_t selz = 0x0C0C0C00u | ((idz_ < 0.0f ? 4 : 0) + j);
+    int cur = live && !(mk && mk[ray] == 0) ? 0 : kSentinel, sp = 0, hitId = -1;
+    bool full = false;
+
+    while (__ballot(cur != kSentinel) != 0) {
+        const bool at_tri = cur < 0;
+        const bool at_node = (uint32_t)cur < (uint32_t)kSentinel;
+        const uint32_t l = ~(uint32_t)cur, cnt = l & 31u;
+        const bool there = at_tri & ((uint32_t)j < cnt);
+        // the node's record, or the lane's triangle
+        const uint32_t rec = at_tri ? (l >> 5) + (there ? (uint32_t)j : 0u) : at_node ? (uint32_t)cur : 0u;
+        const GF4 p = (at_tri ? tris : nodes) + 4 * (size_t)rec;
+        const V4f r0 = p[0], r1 = p[1], r2 = p[2], r3 = p[3];
+        // the entry that a pop at the end of this step takes
+        const int below = sp > 0 ? sp - 1 : 0;
+        const int upper = lstack[(below >> 2) * 64 + (lane & ~3) + (below & 3)];
+        asm volatile("" ::"v"(r0.x), "v"(r1.x), "v"(r2.x), "v"(r3.x));
+
+        bool pop = false;
+        int next = cur;
+        if (__ballot(at_tri) != 0) {  // (a branch of the wave: no lane is masked out)
+            const float Oz = fmaf(-oz, r0.z, fmaf(-oy, r0.y, fmaf(-ox, r0.x, r0.w)));
+            const float t = Oz * rcp_rn(fmaf(dz, r0.z, fmaf(dy, r0.y, dx * r0.x)));
+            const float Ox = fmaf(oz, r1.z, fmaf(oy, r1.y, fmaf(ox, r1.x, r1.w)));
+            const float Dx = fmaf(dz, r1.z, fmaf(dy, r1.y, dx * r1.x));
+            const float u = fmaf(t, Dx, Ox);
+            const float Oy = fmaf(oz, r2.z, fmaf(oy, r2.y, fmaf(ox, r2.x, r2.w)));
+            const float Dy = fmaf(dz, r2.z, fmaf(dy, r2.y, dx * r2.x));
+            const float v = fmaf(t, Dy, Oy);
+            const int id = __float_as_int(r3.x);
+            const bool hit = there & (t > tmin) & ((t < hitT) | ((t == hitT) & (id < hitId))) & (u >= 0.0f) &
+                             (v >= 0.0f) & (u + v <= 1.0f);
+            bool found = false;
+            if (__ballot(hit) != 0) {
+                // one after the other the triangles would leave the nearest
+                // hit (the lowest id on ties), or the first for any hit
+                float tn = hit ? t : __builtin_inff();
+                tn = vmin_(tn, __int_as_float(quad<kQuadXor1>(__float_as_int(tn))));
+                tn = vmin_(tn, __int_as_float(quad<kQuadXor2>(__float_as_int(tn))));
+                const int own = (hit & (an | (t == tn))) ? (an ? j : id) : 0x7FFFFFFF;
+                const int o1 = quad<kQuadXor1>(own), p1 = o1 < own ? o1 : own;
+                const int o2 = quad<kQuadXor2>(p1), best = o2 < p1 ? o2 : p1;
+                found = best != 0x7FFFFFFF;
+                const bool take = found & (own == best);
+                int tb = take ? __float_as_int(t) : 0, ib = take ? id : 0;
+                tb |= quad<kQuadXor1>(tb);
+                ib |= quad<kQuadXor1>(ib);
+                tb |= quad<kQuadXor2>(tb);
+                ib |= quad<kQuadXor2>(ib);
+                hitT = found ? __int_as_float(tb) : hitT;
+                hitId = found ? ib : hitId;
+            }
+            const bool over = found & an;
+            pop = at_tri & (cnt <= 4) & !over;
+            next = over ? kSentinel : at_tri ? (int)~(l + 124u) : cur;  // first + 4, count - 4
+        }
+        if (__ballot(at_node) != 0) {
+            int link, first_link, top, at;
+            bool push, none;
+            if (WIDE) {
+                const uint32_t lox = __float_as_uint(r1.z), hix = __float_as_uint(r1.w), loy = __float_as_uint(r2.x),
+                               hiy = __float_as_uint(r2.y), loz = __float_as_uint(r2.z), hiz = __float_as_uint(r2.w);
+                const float sx = r0.w * idx_, sy = r1.x * idy_, sz = r1.y * idz_;
+                const float bx = fmaf(sx, 0.0f, fmaf(r0.x, idx_, -oodx));
+                const float by = fmaf(sy, 0.0f, fmaf(r0.y, idy_, -oody));
+                const float bz = fmaf(sz, 0.0f, fmaf(r0.z, idz_, -oodz));
+                const float nx = walk_plane(lox, hix, selx, sx, bx), fx = walk_plane(lox, hix, selx ^ 4, sx, bx);
+                const float ny = walk_plane(loy, hiy, sely, sy, by), fy = walk_plane(loy, hiy, sely ^ 4, sy, by);
+                const float nz = walk_plane(loz, hiz, selz, sz, bz), fz = walk_plane(loz, hiz, selz ^ 4, sz, bz);
+                const int l01 = __float_as_int((j & 1) ? r3.y : r3.x), l23 = __float_as_int((j & 1) ? r3.w : r3.z);
+                link = j < 2 ? l01 : l23;
+                const float near = vmax3_(nx, ny, vmax_(nz, tmin));
+                const float far = vmin3_(fx, fy, vmin_(fz, hitT));
+                constexpr int kMiss = 0x7FFFFFFF;
+                const int key = fmaf(fabsf(far), 0x1p-22f, far) >= near ? __float_as_int(near) : kMiss;
+                // the three exchanges of trace_steps: (0, 1), (2, 3), then the
+                // winners of both (the lower child on ties)
+                const int kp = quad<kQuadXor1>(key);
+                const bool won = (j & 1) ? key < kp : key <= kp;
+                const int wk = key < kp ? key : kp, lk = key < kp ? kp : key;  // winner and loser of the pair
+                const int ow = quad<kQuadXor2>(wk), ol = quad<kQuadXor2>(lk);
+                const bool first = won & (j < 2 ? wk <= ow : wk < ow);
+                const int lose_a = (j < 2 ? lk : ol) != kMiss, lose_b = (j < 2 ? ol : lk) != kMiss;
+                // pushed: loser of (2, 3), loser of (0, 1), second winner
+                push = (key != kMiss) & !first;
+                at = sp + (won ? lose_a + lose_b : j < 2 ? lose_b : 0);
+                top = sp + lose_a + lose_b + ((wk < ow ? ow : wk) != kMiss);
+                first_link = first ? link : 0;
+                first_link |= quad<kQuadXor1>(first_link);
+                first_link |= quad<kQuadXor2>(first_link);
+                none = (wk == kMiss) & (ow == kMiss);
+            } else {
+                const bool c = (j & 1) != 0;
+                const float lx = c ? r1.x : r0.x, hx = c ? r1.y : r0.y, ly = c ? r1.z : r0.z, hy = c ? r1.w : r0.w;
+                const float lz = c ? r2.z : r2.x, hz = c ? r2.w : r2.y;
+                const int l0 = __float_as_int(r3.x), l1 = __float_as_int(r3.y);
+                const float clox = fmaf(lx, idx_, -oodx), chix = fmaf(hx, idx_, -oodx);
+                const float cloy = fmaf(ly, idy_, -oody), chiy = fmaf(hy, idy_, -oody);
+                const float cloz = fmaf(lz, idz_, -oodz), chiz = fmaf(hz, idz_, -oodz);
+                const float cmin = vmax3_(vmin_(clox, chix), vmin_(cloy, chiy), vmax_(vmin_(cloz, chiz), tmin));
+                const float cmax = vmin3_(vmax_(clox, chix), vmax_(cloy, chiy), vmin_(vmax_(cloz, chiz), hitT));
+                const int h = cmax >= cmin ? 1 : 0, m = __float_as_int(cmin);
+                const bool t0 = quad<kQuad0>(h) != 0, t1 = quad<kQuad1>(h) != 0;
+                const bool far_first =
+                    t1 & (!t0 | (__int_as_float(quad<kQuad1>(m)) < __int_as_float(quad<kQuad0>(m))));
+                push = t0 & t1 & (j == 0);
+                link = far_first ? l0 : l1;  // the farther one
+                at = sp;
+                top = sp + (t0 & t1);
+                none = !t0 & !t1;
+                first_link = far_first ? l1 : l0;
+            }
+            push = push & at_node;
+            // (the upload refuses trees deep enough to fill the stack: a
+            // launch that still did so is flagged, nothing written past it)
+            full = full | (push & (at >= 4 * rows));
+            lstack[(push & (at < 4 * rows)) ? (at >> 2) * 64 + (lane & ~3) + (at & 3) : rows * 64 + lane] = link;
+            pop = at_node ? none : pop;
+            next = at_node ? first_link : next;
+            sp = at_node ? (top < 4 * rows ? top : 4 * rows) : sp;
+        }
+        cur = pop ? (sp == 0 ? kSentinel : upper) : next;
+        sp -= pop & (sp > 0);
+    }
+    if (full) atomicOr(a.errors, (uint32_t)RB_TRACE_ERR_STACK);
+    if (live && j == 0) {
+        V2i r;
+        r.x = hitId;
+        // a miss reports the caller's tmax, bit for bit
+        r.y = hitId < 0 ? __float_as_int(((const __attribute__((address_space(1))) float*)(rays + 2 * ray + 1))[3])
+                        : __float_as_int(hitT);
+        const GI2 hits = MULTI ? (GI2)tab[batch].hits : second ? (GI2)a.hits2 : (GI2)a.hits;
+        hits[ray] = r;
+    }
+}
+
 template <bool ANY, bool COUNT, int S, int BLOCK, bool SPEC>
 __global__ __launch_bounds__(BLOCK) void k_trace(TraceArgs a) {
     const uint32_t nrays = a.n_dev ? __builtin_nontemporal_load(a.n_dev) : a.n;
@@ -920,11 +1141,9 @@ __global__ __launch_bounds__(BLOCK) void k_trace_pair(TraceArgs a) {
     trace_steps<true, false, S, BLOCK, false, true, WIDE>(a, nullptr, 0, n0 + n1, n0);
 }
 
-template <int S, int BLOCK, bool SPEC, bool WIDE>
-__global__ __launch_bounds__(BLOCK) void k_trace_batch(TraceArgs a, BatchTable t) {
-    __shared__ BatchDesc tab[kMaxBatch];
-    __shared__ uint32_t s_total;
-    for (uint32_t i = threadIdx.x; i < t.nb; i += BLOCK) tab[i] = t.d[i];
+// The launch's batch table in LDS, with each batch's first global ray.
+__device__ __forceinline__ void batch_table(const BatchTable& t, BatchDesc* tab, uint32_t* total) {
+    for (uint32_t i = threadIdx.x; i < t.nb; i += blockDim.x) tab[i] = t.d[i];
     __syncthreads();
     if (threadIdx.x == 0) {  // batch starts from the counts (device counts were final before the launch)
         uint32_t sum = 0;
@@ -937,13 +1156,41 @@ __global__ __launch_bounds__(BLOCK) void k_trace_batch(TraceArgs a, BatchTable t
             tab[i].start = sum;
             sum += n;
         }
-        s_total = sum;
+        *total = sum;
     }
     __syncthreads();
+}
+
+template <int S, int BLOCK, bool SPEC, bool WIDE>
+__global__ __launch_bounds__(BLOCK) void k_trace_batch(TraceArgs a, BatchTable t) {
+    __shared__ BatchDesc tab[kMaxBatch];
+    __shared__ uint32_t s_total;
+    batch_table(t, tab, &s_total);
     if (SPEC)
         trace_spec<false, false, S, BLOCK, true>(a, tab, t.nb, s_total);
     else
         trace_steps<false, false, S, BLOCK, true, false, WIDE>(a, tab, t.nb, s_total);
+}
+
+template <bool ANY, bool WIDE>
+__global__ __launch_bounds__(64) void k_trace_few(TraceArgs a) {
+    const uint32_t nrays = a.n_dev ? __builtin_nontemporal_load(a.n_dev) : a.n;
+    trace_quads<ANY, false, false, WIDE>(a, nullptr, 0, nrays);
+}
+
+template <bool WIDE>
+__global__ __launch_bounds__(64) void k_trace_few_pair(TraceArgs a) {
+    const uint32_t n0 = __builtin_nontemporal_load(a.n_dev);
+    const uint32_t n1 = __builtin_nontemporal_load(a.n_dev2);
+    trace_quads<true, false, true, WIDE>(a, nullptr, 0, n0 + n1, n0);
+}
+
+template <bool WIDE>
+__global__ __launch_bounds__(64) void k_trace_few_batch(TraceArgs a, BatchTable t) {
+    __shared__ BatchDesc tab[kMaxBatch];
+    __shared__ uint32_t s_total;
+    batch_table(t, tab, &s_total);
+    trace_quads<false, true, false, WIDE>(a, tab, t.nb, s_total);
 }
 
 // ---------------------------------------------------------------- launch --
@@ -1000,6 +1247,17 @@ static BatchKernel pick_batch(const rb_trace_config& c, bool wide) {
 static bool wide_walk(const rb_trace_config& cfg, rb_bvh_t bvh, uint32_t flags) {
     return cfg.wide && !cfg.speculative && bvh->wnodes && (!(flags & RB_ANY) || (flags & kOcclusion));
 }
+
+// Whether a launch of at most n rays takes trace_quads: up to where both loops
+// are level on rays that scatter (the figures are at trace_quads), 1024 rays
+// per CU over the wide records and 768 over the binary ones, whose two
+// children use half of the quad.
+static bool few_rays(const rb_trace_config& cfg, bool wide, uint64_t n) {
+    return !cfg.speculative && n <= (uint64_t)dev().num_cus * (wide ? 1024 : 768);
+}
+static uint32_t few_blocks(uint64_t n) { return (uint32_t)((n + 15) / 16); }
+static uint32_t stack_rows(rb_bvh_t bvh, bool wide) { return ((wide ? bvh->wide_stack : bvh->stack) + 3) / 4; }
+static size_t few_lds(const TraceArgs& a) { return (a.stack_rows + 1) * 64 * sizeof(int); }
 
 // Static LDS of a trace block: the stack and, in the step loop, a staged
 // 64-byte record per lane.
@@ -1060,6 +1318,14 @@ rb_status launch_trace(rb_bvh_t bvh, const rb_ray* rays, uint32_t n, uint32_t fl
     if (lds > dev().lds_per_block)
         return fail(RB_ERR_INVALID, "trace config needs %zu bytes of LDS per block (stack %u x %u lanes + %u node records); "
                     "the device allows %zu", lds, cfg.lds_stack, cfg.block, a.top_nodes, dev().lds_per_block);
+    if (!counts && few_rays(cfg, wide, n)) {
+        a.stack_rows = stack_rows(bvh, wide);
+        TraceKernel q = wide ? (any ? k_trace_few<true, true> : k_trace_few<false, true>)
+                             : (any ? k_trace_few<true, false> : k_trace_few<false, false>);
+        hipLaunchKernelGGL(q, dim3(few_blocks(n)), dim3(64), few_lds(a), stream, a);
+        const hipError_t e = hipGetLastError();
+        return e != hipSuccess ? hip_fail(e, "trace launch") : RB_OK;
+    }
     SlotLease L;
     if (counter) {
         L.counter = counter;
@@ -1114,6 +1380,13 @@ rb_status launch_trace_pair(rb_bvh_t bvh, const rb_ray* rays0, uint32_t cap0, co
     if (lds > dev().lds_per_block)
         return fail(RB_ERR_INVALID, "trace config needs %zu bytes of LDS per block; the device allows %zu", lds,
                     dev().lds_per_block);
+    if (few_rays(cfg, wide, a.n)) {
+        a.stack_rows = stack_rows(bvh, wide);
+        TraceKernel q = wide ? k_trace_few_pair<true> : k_trace_few_pair<false>;
+        hipLaunchKernelGGL(q, dim3(few_blocks(a.n)), dim3(64), few_lds(a), stream, a);
+        const hipError_t e = hipGetLastError();
+        return e != hipSuccess ? hip_fail(e, "paired trace launch") : RB_OK;
+    }
     const SlotLease L = take_counter_slot(stream);
     if (L.st != RB_OK) return L.st;
     if (!L.counter) return fail(RB_ERR_INVALID, "render graph: out of work-counter slots");
@@ -1154,6 +1427,7 @@ static rb_status launch_trace_sets_pass(const BatchSet* b, uint32_t nb, hipStrea
         BatchTable t;
         std::memset(&t, 0, sizeof(t));
         uint64_t total = 0;  // bound of the launch's rays (sizes the grid)
+        uint32_t rows = 0;
         uint32_t i = i0;
         for (; i < nb && t.nb < kMaxBatch; i++) {
             if (b[i].n == 0 || !in_pass(b[i])) continue;
@@ -1168,6 +1442,7 @@ static rb_status launch_trace_sets_pass(const BatchSet* b, uint32_t nb, hipStrea
             d.n_dev = b[i].n_dev;
             d.n = b[i].n;
             d.any = b[i].any ? 1u : 0u;
+            rows = std::max(rows, stack_rows(b[i].bvh, wide));
             total += b[i].n;
         }
         i0 = i;
@@ -1179,6 +1454,14 @@ static rb_status launch_trace_sets_pass(const BatchSet* b, uint32_t nb, hipStrea
         a.chunk = cfg.chunk;
         a.threshold = cfg.fetch_threshold;
         a.leaf_gate = cfg.leaf_gate;
+        if (few_rays(cfg, wide, total)) {
+            a.stack_rows = rows;
+            BatchKernel q = wide ? k_trace_few_batch<true> : k_trace_few_batch<false>;
+            hipLaunchKernelGGL(q, dim3(few_blocks(total)), dim3(64), few_lds(a), stream, a, t);
+            const hipError_t e = hipGetLastError();
+            if (e != hipSuccess) return hip_fail(e, "batched trace launch");
+            continue;
+        }
         const SlotLease L = take_counter_slot(stream);
         if (L.st != RB_OK) return L.st;
         if (!L.counter) return fail(RB_ERR_INVALID, "render graph: out of work-counter slots");

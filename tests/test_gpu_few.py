@@ -1,0 +1,76 @@
+"""GPU parity of the two loops a launch may take: a quad of lanes per ray for
+launches of few rays, a lane per ray for the rest.  The same rays traced alone
+and as the head of a launch past the line (1024 rays per CU) give the same
+(id, t), bit for bit, which are the oracle's -- over the wide and the binary
+records, closest and any hit, masked, at the edges of a block (16 rays), with
+leaves of more triangles than a quad has lanes, ties, NaN and zero rays."""
+import numpy as np
+import pytest
+
+from conftest import random_rays, random_triangles
+
+pytestmark = pytest.mark.gpu
+
+PAST = 1024 * 256 + 1
+
+
+@pytest.fixture(scope="module")
+def scene(gpu):
+    from renderbox2_amd import _lib as L
+    v, idx = random_triangles(1500, seed=500)
+    # 23 copies of one triangle (a leaf of many, all ties) and 6 nested ones
+    extra = [idx[:1]] * 23 + [idx[7:8]] * 6
+    idx = np.concatenate([idx] + extra).astype(idx.dtype)
+    b = gpu.BVH((v, idx))
+    c = b.export(L.RB_LAYOUT_REF_COMPACT2)
+    centre = v[idx[0]].mean(axis=0)
+    return gpu.CudaTracer(b), (c[0].reshape(-1, 4), c[1].reshape(-1, 4), c[2]), centre
+
+
+def _rays(n, centre):
+    rays = random_rays(n, seed=501)
+    rays[: n // 2, 4:7] = centre - rays[: n // 2, 0:3]  # through the copies
+    if n > 8:
+        rays[1, 4:7] = 0.0
+        rays[2, 0:3] = np.nan
+        rays[3, 5] = 0.0
+        rays[4, 7] = np.inf
+        rays[5, 3] = np.nan
+        rays[6, 4:7] = np.inf
+    return rays
+
+
+def _trace(gpu, tr, rays, n, any_hit, mask):
+    d_rays, d_hits = gpu.DeviceBuffer.from_array(rays), gpu.DeviceBuffer(n * 8)
+    d_mask = gpu.DeviceBuffer.from_array(mask) if mask is not None else None
+    tr.trace_device(d_rays.ptr, n, d_hits.ptr, any_hit=any_hit, d_mask=d_mask.ptr if d_mask else None)
+    return d_hits.download(gpu.HIT_DTYPE, n)
+
+
+@pytest.mark.parametrize("wide", [1, 0])
+@pytest.mark.parametrize("any_hit", [False, True])
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("n", [1, 15, 17, 4099])
+def test_both_loops_give_the_same_hits(gpu, orc, scene, wide, any_hit, masked, n):
+    tr, c2, centre = scene
+    rays = _rays(n, centre)
+    mask = (np.arange(PAST) % 3 != 0).astype(np.uint8) if masked else None
+    cfg = gpu.get_trace_config()
+    gpu.set_trace_config(**{**cfg, "wide": wide})
+    try:
+        few = _trace(gpu, tr, rays, n, any_hit, mask)
+        tail = np.zeros((PAST - n, 8), np.float32)
+        tail[:, 0:3] = 1e6  # rays that miss the root
+        tail[:, 4] = tail[:, 7] = 1.0
+        many = _trace(gpu, tr, np.concatenate([rays, tail]), PAST, any_hit, mask)[:n]
+    finally:
+        gpu.set_trace_config(**cfg)
+    assert np.array_equal(few["id"], many["id"])
+    assert np.array_equal(few["t"].view(np.uint32), many["t"].view(np.uint32))
+    ok = np.isfinite(rays[:, :7]).all(axis=1)
+    if masked:
+        ok &= mask[:n] != 0
+    oid, ot = orc.trace_compact2(*c2, np.ascontiguousarray(rays[ok]), any_hit=any_hit)
+    assert np.array_equal(few["id"][ok], oid) and np.array_equal(few["t"][ok].view(np.uint32), ot.view(np.uint32))
+    if n > 1000 and not masked:
+        assert (oid >= 0).sum() > n // 4
