@@ -119,6 +119,9 @@ rb_bvh_dev device_view(rb_bvh_t bvh);
 // find a hit exactly when the binary walk does but not necessarily the same
 // first one.  The public entry points refuse the bit.
 constexpr uint32_t kOcclusion = 1u << 16;
+// And: neighbouring rays of the set start together and run alike (camera
+// rays), which moves the line up to which launches give each ray a quad.
+constexpr uint32_t kCoherent = 1u << 17;
 
 // Persistent traversal launch (rb_trace.hip).  n_dev, when set, holds the ray
 // count in device memory (queues sized by earlier kernels); n is then an
@@ -160,7 +163,7 @@ struct TraceSet {
     int2* hits;
     uint32_t n;             // rays, or the bound of *n_dev
     const uint32_t* n_dev;  // device count (NULL: n)
-    uint32_t flags;         // RB_CLOSEST or RB_ANY (with kOcclusion), with RB_MASKED
+    uint32_t flags;         // RB_CLOSEST (with kCoherent) or RB_ANY (with kOcclusion), with RB_MASKED
     const uint8_t* mask;
     rb_trace_config cfg;    // launch shape when the set is traced on its own
 };

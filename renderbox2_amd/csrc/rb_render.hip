@@ -835,7 +835,7 @@ struct AoJob : RenderJob {
         *done = false;
         if (state == 0) {
             if ((st = rb_raygen_camera(&cam, x0, y0, w, h, p.spp, p.seed, 1, (rb_ray*)rays, s)) != RB_OK) return st;
-            sets[0] = TraceSet{rays, hits, n, nullptr, RB_CLOSEST, nullptr, dev().cfg};
+            sets[0] = TraceSet{rays, hits, n, nullptr, RB_CLOSEST | kCoherent, nullptr, dev().cfg};
             *nsets = 1;
         } else if (state == 1) {
             TileArgs T{cam.width, x0, y0, w, p.spp};
@@ -880,7 +880,7 @@ struct RaycastJob : RenderJob {
         *done = false;
         if (state == 0) {
             if ((st = rb_raygen_camera(&cam, x0, y0, w, h, p.spp, p.seed, 1, (rb_ray*)rays, s)) != RB_OK) return st;
-            sets[0] = TraceSet{rays, hits, n, nullptr, RB_CLOSEST, nullptr, dev().cfg};
+            sets[0] = TraceSet{rays, hits, n, nullptr, RB_CLOSEST | kCoherent, nullptr, dev().cfg};
             *nsets = 1;
         } else {
             if (p.ray_counter) hipLaunchKernelGGL(k_add64, dim3(1), dim3(64), 0, s, p.ray_counter, (unsigned long long)n);
@@ -958,7 +958,7 @@ struct CameraJob : RenderJob {
         if (phase == 0) {
             if ((st = rb_raygen_camera(&cam, x0, y0, w, h, p.spp, p.seed, 1, (rb_ray*)prim, s)) != RB_OK) return st;
             if (!bd) {
-                sets[0] = TraceSet{prim, phits, n, nullptr, RB_CLOSEST, nullptr, dev().cfg};
+                sets[0] = TraceSet{prim, phits, n, nullptr, RB_CLOSEST | kCoherent, nullptr, dev().cfg};
                 *nsets = 1;
                 phase = 2;
                 return RB_OK;

@@ -68,7 +68,7 @@ struct TraceArgs {
     uint32_t threshold;
     uint32_t leaf_gate;  // non-speculative: leave the inner-node phase once <= this many lanes still search
     uint32_t top_nodes;  // node records 0..top_nodes-1 are read from a copy in LDS
-    uint32_t stack_rows;  // trace_quads: rows of four entries that a ray's stack can need
+    uint32_t stack_rows;  // a ray's stack needs at most four times as many entries
 };
 
 constexpr uint32_t kMaxBatch = 64;
@@ -350,6 +350,164 @@ __device__ __forceinline__ void stage_records(const V4f* rec, uint32_t lane, V4f
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
+// A ray in registers.
+struct RayRegs {
+    float ox, oy, oz, dx, dy, dz, tmin;
+    float idx, idy, idz;     // reciprocal direction
+    float oodx, oody, oodz;  // origin * reciprocal direction
+};
+__device__ __forceinline__ RayRegs ray_regs(V4f o, V4f d) {
+    RayRegs r;
+    r.ox = o.x, r.oy = o.y, r.oz = o.z;
+    r.dx = d.x, r.dy = d.y, r.dz = d.z;
+    // a quiet copy for the slab max (comparisons treat every NaN alike)
+    r.tmin = __builtin_canonicalizef(o.w);
+    const float ooeps = 0x1p-80f;
+    r.idx = rcp_rn(fabsf(r.dx) > ooeps ? r.dx : copysignf(ooeps, r.dx));
+    r.idy = rcp_rn(fabsf(r.dy) > ooeps ? r.dy : copysignf(ooeps, r.dy));
+    r.idz = rcp_rn(fabsf(r.dz) > ooeps ? r.dz : copysignf(ooeps, r.dz));
+    r.oodx = r.ox * r.idx;
+    r.oody = r.oy * r.idy;
+    r.oodz = r.oz * r.idz;
+    return r;
+}
+
+// One step of every quad of the wave: four lanes per ray, each testing one
+// child of a record (two of them over the binary records) or one triangle of
+// a leaf.  No lane branches: the wave skips the node or the triangle half when
+// no lane is in it, and a lane with nothing to push stores to `spare`.  Steps
+// and arithmetic of a ray and the order of its stack are trace_steps', so its
+// result does not depend on which lanes took it.
+// at_entry(e): where the quad keeps stack entry e (room entries).
+template <bool WIDE, typename Entry>
+__device__ __forceinline__ void quad_step(GF4 nodes, GF4 tris, const RayRegs& ray, bool an, int j, Entry at_entry,
+                                          int room, int* spare, int& cur, int& sp, float& hitT, int& hitId,
+                                          bool& full) {
+    const float ox = ray.ox, oy = ray.oy, oz = ray.oz, dx = ray.dx, dy = ray.dy, dz = ray.dz, tmin = ray.tmin;
+    const float idx_ = ray.idx, idy_ = ray.idy, idz_ = ray.idz;
+    const float oodx = ray.oodx, oody = ray.oody, oodz = ray.oodz;
+    const bool at_tri = cur < 0;
+    const bool at_node = (uint32_t)cur < (uint32_t)kSentinel;
+    const uint32_t l = ~(uint32_t)cur, cnt = l & 31u;
+    const bool there = at_tri & ((uint32_t)j < cnt);
+    // the node's record, or the lane's triangle
+    const uint32_t rec = at_tri ? (l >> 5) + (there ? (uint32_t)j : 0u) : at_node ? (uint32_t)cur : 0u;
+    const GF4 p = (at_tri ? tris : nodes) + 4 * (size_t)rec;
+    const V4f r0 = p[0], r1 = p[1], r2 = p[2], r3 = p[3];
+    // the entry that a pop at the end of this step takes
+    const int upper = *at_entry(sp > 0 ? sp - 1 : 0);
+    asm volatile("" ::"v"(r0.x), "v"(r1.x), "v"(r2.x), "v"(r3.x));
+
+    bool pop = false;
+    int next = cur;
+    if (__ballot(at_tri) != 0) {  // (a branch of the wave: no lane is masked out)
+        const float Oz = fmaf(-oz, r0.z, fmaf(-oy, r0.y, fmaf(-ox, r0.x, r0.w)));
+        const float t = Oz * rcp_rn(fmaf(dz, r0.z, fmaf(dy, r0.y, dx * r0.x)));
+        const float Ox = fmaf(oz, r1.z, fmaf(oy, r1.y, fmaf(ox, r1.x, r1.w)));
+        const float Dx = fmaf(dz, r1.z, fmaf(dy, r1.y, dx * r1.x));
+        const float u = fmaf(t, Dx, Ox);
+        const float Oy = fmaf(oz, r2.z, fmaf(oy, r2.y, fmaf(ox, r2.x, r2.w)));
+        const float Dy = fmaf(dz, r2.z, fmaf(dy, r2.y, dx * r2.x));
+        const float v = fmaf(t, Dy, Oy);
+        const int id = __float_as_int(r3.x);
+        const bool hit = there & (t > tmin) & ((t < hitT) | ((t == hitT) & (id < hitId))) & (u >= 0.0f) &
+                         (v >= 0.0f) & (u + v <= 1.0f);
+        bool found = false;
+        if (__ballot(hit) != 0) {
+            // one after the other the triangles would leave the nearest
+            // hit (the lowest id on ties), or the first for any hit
+            float tn = hit ? t : __builtin_inff();
+            tn = vmin_(tn, __int_as_float(quad<kQuadXor1>(__float_as_int(tn))));
+            tn = vmin_(tn, __int_as_float(quad<kQuadXor2>(__float_as_int(tn))));
+            const int own = (hit & (an | (t == tn))) ? (an ? j : id) : 0x7FFFFFFF;
+            const int o1 = quad<kQuadXor1>(own), p1 = o1 < own ? o1 : own;
+            const int o2 = quad<kQuadXor2>(p1), best = o2 < p1 ? o2 : p1;
+            found = best != 0x7FFFFFFF;
+            const bool take = found & (own == best);
+            int tb = take ? __float_as_int(t) : 0, ib = take ? id : 0;
+            tb |= quad<kQuadXor1>(tb);
+            ib |= quad<kQuadXor1>(ib);
+            tb |= quad<kQuadXor2>(tb);
+            ib |= quad<kQuadXor2>(ib);
+            hitT = found ? __int_as_float(tb) : hitT;
+            hitId = found ? ib : hitId;
+        }
+        const bool over = found & an;
+        pop = at_tri & (cnt <= 4) & !over;
+        next = over ? kSentinel : at_tri ? (int)~(l + 124u) : cur;  // first + 4, count - 4
+    }
+    if (__ballot(at_node) != 0) {
+        int link, first_link, top, at;
+        bool push, none;
+        if (WIDE) {
+            const uint32_t lox = __float_as_uint(r1.z), hix = __float_as_uint(r1.w), loy = __float_as_uint(r2.x),
+                           hiy = __float_as_uint(r2.y), loz = __float_as_uint(r2.z), hiz = __float_as_uint(r2.w);
+            const float sx = r0.w * idx_, sy = r1.x * idy_, sz = r1.y * idz_;
+            const float bx = fmaf(sx, 0.0f, fmaf(r0.x, idx_, -oodx));
+            const float by = fmaf(sy, 0.0f, fmaf(r0.y, idy_, -oody));
+            const float bz = fmaf(sz, 0.0f, fmaf(r0.z, idz_, -oodz));
+            const uint32_t selx = 0x0C0C0C00u | ((idx_ < 0.0f ? 4 : 0) + j);
+            const uint32_t sely = 0x0C0C0C00u | ((idy_ < 0.0f ? 4 : 0) + j);
+            const uint32_t selz = 0x0C0C0C00u | ((idz_ < 0.0f ? 4 : 0) + j);
+            const float nx = walk_plane(lox, hix, selx, sx, bx), fx = walk_plane(lox, hix, selx ^ 4, sx, bx);
+            const float ny = walk_plane(loy, hiy, sely, sy, by), fy = walk_plane(loy, hiy, sely ^ 4, sy, by);
+            const float nz = walk_plane(loz, hiz, selz, sz, bz), fz = walk_plane(loz, hiz, selz ^ 4, sz, bz);
+            const int l01 = __float_as_int((j & 1) ? r3.y : r3.x), l23 = __float_as_int((j & 1) ? r3.w : r3.z);
+            link = j < 2 ? l01 : l23;
+            const float near = vmax3_(nx, ny, vmax_(nz, tmin));
+            const float far = vmin3_(fx, fy, vmin_(fz, hitT));
+            constexpr int kMiss = 0x7FFFFFFF;
+            const int key = fmaf(fabsf(far), 0x1p-22f, far) >= near ? __float_as_int(near) : kMiss;
+            // the three exchanges of trace_steps: (0, 1), (2, 3), then the
+            // winners of both (the lower child on ties)
+            const int kp = quad<kQuadXor1>(key);
+            const bool won = (j & 1) ? key < kp : key <= kp;
+            const int wk = key < kp ? key : kp, lk = key < kp ? kp : key;  // winner and loser of the pair
+            const int ow = quad<kQuadXor2>(wk), ol = quad<kQuadXor2>(lk);
+            const bool first = won & (j < 2 ? wk <= ow : wk < ow);
+            const int lose_a = (j < 2 ? lk : ol) != kMiss, lose_b = (j < 2 ? ol : lk) != kMiss;
+            // pushed: loser of (2, 3), loser of (0, 1), second winner
+            push = (key != kMiss) & !first;
+            at = sp + (won ? lose_a + lose_b : j < 2 ? lose_b : 0);
+            top = sp + lose_a + lose_b + ((wk < ow ? ow : wk) != kMiss);
+            first_link = first ? link : 0;
+            first_link |= quad<kQuadXor1>(first_link);
+            first_link |= quad<kQuadXor2>(first_link);
+            none = (wk == kMiss) & (ow == kMiss);
+        } else {
+            const bool c = (j & 1) != 0;
+            const float lx = c ? r1.x : r0.x, hx = c ? r1.y : r0.y, ly = c ? r1.z : r0.z, hy = c ? r1.w : r0.w;
+            const float lz = c ? r2.z : r2.x, hz = c ? r2.w : r2.y;
+            const int l0 = __float_as_int(r3.x), l1 = __float_as_int(r3.y);
+            const float clox = fmaf(lx, idx_, -oodx), chix = fmaf(hx, idx_, -oodx);
+            const float cloy = fmaf(ly, idy_, -oody), chiy = fmaf(hy, idy_, -oody);
+            const float cloz = fmaf(lz, idz_, -oodz), chiz = fmaf(hz, idz_, -oodz);
+            const float cmin = vmax3_(vmin_(clox, chix), vmin_(cloy, chiy), vmax_(vmin_(cloz, chiz), tmin));
+            const float cmax = vmin3_(vmax_(clox, chix), vmax_(cloy, chiy), vmin_(vmax_(cloz, chiz), hitT));
+            const int h = cmax >= cmin ? 1 : 0, m = __float_as_int(cmin);
+            const bool t0 = quad<kQuad0>(h) != 0, t1 = quad<kQuad1>(h) != 0;
+            const bool far_first =
+                t1 & (!t0 | (__int_as_float(quad<kQuad1>(m)) < __int_as_float(quad<kQuad0>(m))));
+            push = t0 & t1 & (j == 0);
+            link = far_first ? l0 : l1;  // the farther one
+            at = sp;
+            top = sp + (t0 & t1);
+            none = !t0 & !t1;
+            first_link = far_first ? l1 : l0;
+        }
+        push = push & at_node;
+        // (the upload refuses trees deep enough to fill the stack: a
+        // launch that still did so is flagged, nothing written past it)
+        full = full | (push & (at >= room));
+        *((push & (at < room)) ? at_entry(at) : spare) = link;
+        pop = at_node ? none : pop;
+        next = at_node ? first_link : next;
+        sp = at_node ? (top < room ? top : room) : sp;
+    }
+    cur = pop ? (sp == 0 ? kSentinel : upper) : next;
+    sp -= pop & (sp > 0);
+}
+
 // One traversal body for every launch form but the speculative one.
 // PAIR: rays [0, n0) are the first set (a.rays / a.hits; any hit when
 // a.any0), rays [n0, nrays) the closest-hit set (a.rays2 / a.hits2).
@@ -371,12 +529,16 @@ __device__ __forceinline__ void stage_records(const V4f* rec, uint32_t lane, V4f
 // frame of 2M triangles 21.9 -> 19.3 ms.  Tried and left out: the top of the
 // tree in LDS (a branch per step, more than it saved), and waves of a
 // workgroup joining their last rays in one of them (720 against 684 us: the
-// drain waits for the longest ray's steps, not for issue slots).  A ray still
-// tests its nodes and leaves in its own order, whatever the other rays of its
-// wave do, so results are the same run to run and launch shape to launch
-// shape.
+// drain waits for the longest ray's steps, not for issue slots).  So once no
+// rays are left to claim and sixteen or fewer of the wave's are under way, each
+// of those gets a quad of lanes (quad_step), whose steps are half as long: 2 Mi
+// diffuse rays 671 -> 610 us, as any hit 559 -> 501, 512 Ki of them 349 -> 280,
+// the camera rays 402 -> 389, the path-traced frame 18.8 -> 18.5 ms.  A ray
+// still tests its nodes and leaves in its own order, whatever the other rays
+// of its wave do, so results are the same run to run and launch shape to
+// launch shape.
 template <bool ANY_T, bool COUNT, int S, int BLOCK, bool MULTI, bool PAIR, bool WIDE>
-__device__ __forceinline__ void trace_steps(const TraceArgs& a, const BatchDesc* tab, uint32_t nb, uint32_t nrays,
+__device__ __forceinline__ void trace_steps(const TraceArgs& a, const BatchDesc* tab, uint32_t nb, uint32_t n_rays,
                                             uint32_t n0 = 0) {
     // the stack: S - 1 entries of each lane in LDS, lane-interleaved, deeper
     // ones in private memory; empty, it gives the sentinel that ends the ray.
@@ -388,12 +550,14 @@ __device__ __forceinline__ void trace_steps(const TraceArgs& a, const BatchDesc*
     __shared__ int lstack[R * BLOCK];
     __shared__ V4f staged[4 * BLOCK];
     int spill[kMaxStack - 1 - R];
+    constexpr int kDeep = 48;  // a quad's entries past those, once a wave has given its last rays a quad each
     const int tid = threadIdx.x;
     const uint32_t lane = __lane_id();
     // this wave's 64 staged records (wave-uniform), and where this lane's lies
     V4f* const stage = staged + 256 * __builtin_amdgcn_readfirstlane(tid >> 6);
     const V4f* const mine_staged = stage + 64 * (lane & 3) + 4 * (lane >> 2);
 
+    const uint32_t nrays = __builtin_amdgcn_readfirstlane(n_rays);
     RayPool<MULTI> pool;
     pool.init(a, nrays);
     // cur: the ray's next step -- an inner record (>= 0), a leaf's remaining
@@ -446,31 +610,59 @@ __device__ __forceinline__ void trace_steps(const TraceArgs& a, const BatchDesc*
         return sp < 0 ? kSentinel : v;
     };
 
+    // the finished ray's result
+    auto store = [&]() {
+        const size_t i = rayidx();
+        V2i r;
+        if (hitId < 0) {  // a miss reports the caller's tmax, bit for bit
+            r.x = -1;
+            r.y = __float_as_int(((const __attribute__((address_space(1))) float*)(rays() + 2 * i + 1))[3]);
+        } else {
+            r.x = hitId;
+            r.y = __float_as_int(hitT);
+        }
+        hits()[i] = r;
+        if (COUNT) {
+            a.counts[3 * i + 0] = c_inner;
+            a.counts[3 * i + 1] = c_tri;
+            a.counts[3 * i + 2] = c_leaf;
+        }
+        live = false;
+    };
+
+    uint32_t left = 0;  // rays that the loop leaves to the wave's quads
+    const uint32_t tail = COUNT || 4 * a.stack_rows > (uint32_t)(R + kDeep) ? 0 : 16;
     while (true) {
         // ---- refill (wave-uniform control): results of the finished rays
         // out, new rays in, once too few lanes are busy ----
         const uint64_t tm = __ballot(cur == kSentinel);
         const uint32_t busy = 64 - __popcll(tm);
-        if (busy == 0 || (!pool.drained && busy < a.threshold)) {
-            if (cur == kSentinel && live) {
-                const size_t i = rayidx();
-                V2i r;
-                if (hitId < 0) {  // a miss reports the caller's tmax, bit for bit
-                    r.x = -1;
-                    r.y = __float_as_int(((const __attribute__((address_space(1))) float*)(rays() + 2 * i + 1))[3]);
-                } else {
-                    r.x = hitId;
-                    r.y = __float_as_int(hitT);
+        if (busy == 0 || (pool.drained ? busy <= tail : busy < a.threshold)) {
+            if (cur == kSentinel && live) store();
+            uint32_t done = pool.drained;
+            if (!COUNT && done && busy) {
+                // what is left of the wave's rays to LDS, for the quads below.
+                // (The value below is opaque so that this stays in the loop:
+                // used on the way out, every register of the ray would be
+                // copied twice per step)
+                asm volatile("" ::: "memory");
+                const uint32_t rank =
+                    __builtin_amdgcn_mbcnt_hi((uint32_t)(~tm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)~tm, 0u));
+                if (cur != kSentinel) {
+                    V4f* const to = stage + 16 * rank;
+                    to[0] = V4f{ox, oy, oz, tmin};
+                    to[1] = V4f{dx, dy, dz, hitT};
+                    to[2] = __builtin_bit_cast(V4f, V4i{hitId, cur, sp, (int)mine});
+                    to[3] = __builtin_bit_cast(V4f, V4i{(int)batch, (int)lane, 0, 0});
+                    for (int e = R; e < sp; e++) ((int*)to)[16 + e - R] = spill[e - R];
                 }
-                hits()[i] = r;
-                if (COUNT) {
-                    a.counts[3 * i + 0] = c_inner;
-                    a.counts[3 * i + 1] = c_tri;
-                    a.counts[3 * i + 2] = c_leaf;
-                }
-                live = false;
+                asm volatile("" ::: "memory");
             }
-            if (pool.drained) break;
+            asm volatile("" : "+s"(done));
+            if (done) {
+                left = busy;
+                break;
+            }
             uint32_t ray;
             if (pool.take(a, nrays, tm, &ray)) {
                 mine = ray;
@@ -665,6 +857,35 @@ __device__ __forceinline__ void trace_steps(const TraceArgs& a, const BatchDesc*
             cur = pop_entry();
             if (COUNT && cur < 0) c_leaf++;
         }
+    }
+    if (!COUNT && left) {
+        // ---- the wave's last rays: a quad each ----
+        const int q = (int)(lane >> 2), j = (int)(lane & 3);
+        const bool has = (uint32_t)q < left;
+        const V4f* const was = stage + 16 * (has ? q : 0);
+        const V4f o = was[0], d = was[1];
+        const V4i w = __builtin_bit_cast(V4i, was[2]), x = __builtin_bit_cast(V4i, was[3]);
+        const RayRegs r = ray_regs(o, d);
+        hitT = d.w;
+        hitId = w.x;
+        cur = has ? w.y : kSentinel;
+        sp = w.z;
+        mine = (uint32_t)w.w;
+        batch = (uint32_t)x.x;
+        if (MULTI) {
+            nodes = (GF4)tab[batch].nodes;
+            tris = (GF4)tab[batch].tris;
+        }
+        const bool an = any();
+        int* const column = lstack + (tid & ~63) + x.y;
+        int* const deep = (int*)(stage + 16 * q) + 16;
+        int* const spare = (int*)(stage + 16 * q) + j;
+        auto at_entry = [&](int e) -> int* { return e < R ? column + e * BLOCK : deep + (e - R); };
+        bool full = false;
+        while (__ballot(cur != kSentinel) != 0)
+            quad_step<WIDE>(nodes, tris, r, an, j, at_entry, R + kDeep, spare, cur, sp, hitT, hitId, full);
+        if (full) atomicOr(a.errors, (uint32_t)RB_TRACE_ERR_STACK);
+        if (has && j == 0) store();
     }
     end_launch<MULTI>(a);
 }
@@ -915,39 +1136,33 @@ __device__ __forceinline__ void trace_spec(const TraceArgs& a, const BatchDesc* 
 #undef RB_PUSH
 #undef RB_POP
 
-// The step loop for launches of few rays: four lanes per ray, sixteen rays per
-// one-wave block, no refill and so no work counters.
+// The step loop for launches of few rays: four lanes per ray from the start,
+// sixteen rays per one-wave block, no refill and so no work counters.
 //
 // With a lane per ray such a launch takes as long as its longest ray, whose
 // steps wait for each other: 0.78 us a step, the chain of its instructions
 // (8-10 cycles for each that needs the one before, 80 for each branch that
-// part of the lanes take) and a record from L2 (240).  With a quad per ray
-// each lane tests one child of a record or one triangle of a leaf, a leaf of
-// four triangles is one step, and no lane branches: a wave skips the node or
-// the triangle half of a step when no lane is in it, and lanes with nothing to
-// push store to a spare row.  0.37 us a step.  Two children per record leave
-// half of the quad idle, but keep the latency.  Steps and arithmetic of a ray
-// and the order of its stack are trace_steps', so its result does not depend
-// on which of the two took it.
+// part of the lanes take) and a record from L2 (240).  With a quad per ray a
+// leaf of four triangles is one step and no lane branches: 0.37 us a step.
+// Two children per record leave half of the quad idle, but keep the latency.
 //
-// Measured, trace_steps -> trace_quads (us), rays from surfaces among 1M
-// triangles: 64 rays 109 -> 54, 16 Ki 173 -> 95, 64 Ki 196 -> 129, 128 Ki 226
-// -> 188, 256 Ki 281 -> 282, 512 Ki 349 -> 485; first camera rays of 200k
-// triangles: 32 Ki 30 -> 10, 128 Ki 50 -> 25, 256 Ki 106 -> 66, 1 Mi 258 ->
-// 338; 4099 rays of 20k triangles 107 -> 48.  Any hit over the binary records:
-// 128 Ki 322 -> 251, 192 Ki 346 -> 336, 256 Ki 375 -> 394.  (The launch is
-// bound by VALU issue from about 100k rays on: a quad's node step is 105
-// instructions for 16 rays where the other loop's is 110 for up to 64.)  Rows
-// of the stack for what the tree can need, not for the most any tree may: 4 KB
-// a wave for 1M triangles, so that eight waves fit a SIMD (256 Ki rays 292 ->
-// 282).
+// Measured, a lane per ray throughout -> a quad for each wave's last rays
+// (trace_steps) -> quads throughout (us), rays from surfaces among 1M
+// triangles: 64 rays 109 -> 83 -> 54, 16 Ki 173 -> 132 -> 95, 64 Ki 196 -> 153
+// -> 129, 128 Ki 226 -> 178 -> 186, 256 Ki 281 -> 226 -> 282; first camera rays
+// of 200k triangles: 32 Ki 30 -> 22 -> 9, 128 Ki 50 -> 51 -> 24, 256 Ki 106 ->
+// 97 -> 66; 4099 rays of 20k triangles 107 -> 83 -> 48.  Any hit over the
+// binary records: 128 Ki 322 -> 262 -> 252, 192 Ki 346 -> 286 -> 336.  (Quads
+// are bound by VALU issue from about 100k rays on: a node step is 105
+// instructions for 16 rays, in the other loop 115 for up to 64.)  Rows of the
+// stack for what the tree can need, not for the most any tree may: 4 KB a wave
+// for 1M triangles, so that eight waves fit a SIMD (256 Ki rays 292 -> 282).
 template <bool ANY_T, bool MULTI, bool PAIR, bool WIDE>
 __device__ __forceinline__ void trace_quads(const TraceArgs& a, const BatchDesc* tab, uint32_t nb, uint32_t nrays,
                                             uint32_t n0 = 0) {
     // a quad's stack: entry e in row e / 4, column e % 4 of its four words; the
     // row behind the last takes the stores of lanes that have nothing to push
     extern __shared__ int lstack[];
-    const int rows = (int)a.stack_rows;
     const int lane = threadIdx.x, j = lane & 3;
     if (blockIdx.x * 16 >= nrays) return;
     uint32_t mine = blockIdx.x * 16 + ((uint32_t)lane >> 2);
@@ -971,149 +1186,25 @@ __device__ __forceinline__ void trace_quads(const TraceArgs& a, const BatchDesc*
     const uint8_t* const mk = MULTI ? tab[batch].mask : a.mask;
     const size_t ray = MULTI ? mine - tab[batch].start : second ? mine - n0 : mine;
     const V4f o = rays[2 * ray], d = rays[2 * ray + 1];
-    const float ox = o.x, oy = o.y, oz = o.z, dx = d.x, dy = d.y, dz = d.z;
-    const float tmin = __builtin_canonicalizef(o.w);
+    const RayRegs r = ray_regs(o, d);
     float hitT = __builtin_canonicalizef(d.w);
-    const float ooeps = 0x1p-80f;
-    const float idx_ = rcp_rn(fabsf(dx) > ooeps ? dx : copysignf(ooeps, dx));
-    const float idy_ = rcp_rn(fabsf(dy) > ooeps ? dy : copysignf(ooeps, dy));
-    const float idz_ = rcp_rn(fabsf(dz) > ooeps ? dz : copysignf(ooeps, dz));
-    const float oodx = ox * idx_, oody = oy * idy_, oodz = oz * idz_;
-    const uint32_t selx = 0x0C0C0C00u | ((idx_ < 0.0f ? 4 : 0) + j);
-    const uint32_t sely = 0x0C0C0C00u | ((idy_ < 0.0f ? 4 : 0) + j);
-    const uint32_t selz = 0x0C0C0C00u | ((idz_ < 0.0f ? 4 : 0) + j);
     int cur = live && !(mk && mk[ray] == 0) ? 0 : kSentinel, sp = 0, hitId = -1;
     bool full = false;
 
-    while (__ballot(cur != kSentinel) != 0) {
-        const bool at_tri = cur < 0;
-        const bool at_node = (uint32_t)cur < (uint32_t)kSentinel;
-        const uint32_t l = ~(uint32_t)cur, cnt = l & 31u;
-        const bool there = at_tri & ((uint32_t)j < cnt);
-        // the node's record, or the lane's triangle
-        const uint32_t rec = at_tri ? (l >> 5) + (there ? (uint32_t)j : 0u) : at_node ? (uint32_t)cur : 0u;
-        const GF4 p = (at_tri ? tris : nodes) + 4 * (size_t)rec;
-        const V4f r0 = p[0], r1 = p[1], r2 = p[2], r3 = p[3];
-        // the entry that a pop at the end of this step takes
-        const int below = sp > 0 ? sp - 1 : 0;
-        const int upper = lstack[(below >> 2) * 64 + (lane & ~3) + (below & 3)];
-        asm volatile("" ::"v"(r0.x), "v"(r1.x), "v"(r2.x), "v"(r3.x));
-
-        bool pop = false;
-        int next = cur;
-        if (__ballot(at_tri) != 0) {  // (a branch of the wave: no lane is masked out)
-            const float Oz = fmaf(-oz, r0.z, fmaf(-oy, r0.y, fmaf(-ox, r0.x, r0.w)));
-            const float t = Oz * rcp_rn(fmaf(dz, r0.z, fmaf(dy, r0.y, dx * r0.x)));
-            const float Ox = fmaf(oz, r1.z, fmaf(oy, r1.y, fmaf(ox, r1.x, r1.w)));
-            const float Dx = fmaf(dz, r1.z, fmaf(dy, r1.y, dx * r1.x));
-            const float u = fmaf(t, Dx, Ox);
-            const float Oy = fmaf(oz, r2.z, fmaf(oy, r2.y, fmaf(ox, r2.x, r2.w)));
-            const float Dy = fmaf(dz, r2.z, fmaf(dy, r2.y, dx * r2.x));
-            const float v = fmaf(t, Dy, Oy);
-            const int id = __float_as_int(r3.x);
-            const bool hit = there & (t > tmin) & ((t < hitT) | ((t == hitT) & (id < hitId))) & (u >= 0.0f) &
-                             (v >= 0.0f) & (u + v <= 1.0f);
-            bool found = false;
-            if (__ballot(hit) != 0) {
-                // one after the other the triangles would leave the nearest
-                // hit (the lowest id on ties), or the first for any hit
-                float tn = hit ? t : __builtin_inff();
-                tn = vmin_(tn, __int_as_float(quad<kQuadXor1>(__float_as_int(tn))));
-                tn = vmin_(tn, __int_as_float(quad<kQuadXor2>(__float_as_int(tn))));
-                const int own = (hit & (an | (t == tn))) ? (an ? j : id) : 0x7FFFFFFF;
-                const int o1 = quad<kQuadXor1>(own), p1 = o1 < own ? o1 : own;
-                const int o2 = quad<kQuadXor2>(p1), best = o2 < p1 ? o2 : p1;
-                found = best != 0x7FFFFFFF;
-                const bool take = found & (own == best);
-                int tb = take ? __float_as_int(t) : 0, ib = take ? id : 0;
-                tb |= quad<kQuadXor1>(tb);
-                ib |= quad<kQuadXor1>(ib);
-                tb |= quad<kQuadXor2>(tb);
-                ib |= quad<kQuadXor2>(ib);
-                hitT = found ? __int_as_float(tb) : hitT;
-                hitId = found ? ib : hitId;
-            }
-            const bool over = found & an;
-            pop = at_tri & (cnt <= 4) & !over;
-            next = over ? kSentinel : at_tri ? (int)~(l + 124u) : cur;  // first + 4, count - 4
-        }
-        if (__ballot(at_node) != 0) {
-            int link, first_link, top, at;
-            bool push, none;
-            if (WIDE) {
-                const uint32_t lox = __float_as_uint(r1.z), hix = __float_as_uint(r1.w), loy = __float_as_uint(r2.x),
-                               hiy = __float_as_uint(r2.y), loz = __float_as_uint(r2.z), hiz = __float_as_uint(r2.w);
-                const float sx = r0.w * idx_, sy = r1.x * idy_, sz = r1.y * idz_;
-                const float bx = fmaf(sx, 0.0f, fmaf(r0.x, idx_, -oodx));
-                const float by = fmaf(sy, 0.0f, fmaf(r0.y, idy_, -oody));
-                const float bz = fmaf(sz, 0.0f, fmaf(r0.z, idz_, -oodz));
-                const float nx = walk_plane(lox, hix, selx, sx, bx), fx = walk_plane(lox, hix, selx ^ 4, sx, bx);
-                const float ny = walk_plane(loy, hiy, sely, sy, by), fy = walk_plane(loy, hiy, sely ^ 4, sy, by);
-                const float nz = walk_plane(loz, hiz, selz, sz, bz), fz = walk_plane(loz, hiz, selz ^ 4, sz, bz);
-                const int l01 = __float_as_int((j & 1) ? r3.y : r3.x), l23 = __float_as_int((j & 1) ? r3.w : r3.z);
-                link = j < 2 ? l01 : l23;
-                const float near = vmax3_(nx, ny, vmax_(nz, tmin));
-                const float far = vmin3_(fx, fy, vmin_(fz, hitT));
-                constexpr int kMiss = 0x7FFFFFFF;
-                const int key = fmaf(fabsf(far), 0x1p-22f, far) >= near ? __float_as_int(near) : kMiss;
-                // the three exchanges of trace_steps: (0, 1), (2, 3), then the
-                // winners of both (the lower child on ties)
-                const int kp = quad<kQuadXor1>(key);
-                const bool won = (j & 1) ? key < kp : key <= kp;
-                const int wk = key < kp ? key : kp, lk = key < kp ? kp : key;  // winner and loser of the pair
-                const int ow = quad<kQuadXor2>(wk), ol = quad<kQuadXor2>(lk);
-                const bool first = won & (j < 2 ? wk <= ow : wk < ow);
-                const int lose_a = (j < 2 ? lk : ol) != kMiss, lose_b = (j < 2 ? ol : lk) != kMiss;
-                // pushed: loser of (2, 3), loser of (0, 1), second winner
-                push = (key != kMiss) & !first;
-                at = sp + (won ? lose_a + lose_b : j < 2 ? lose_b : 0);
-                top = sp + lose_a + lose_b + ((wk < ow ? ow : wk) != kMiss);
-                first_link = first ? link : 0;
-                first_link |= quad<kQuadXor1>(first_link);
-                first_link |= quad<kQuadXor2>(first_link);
-                none = (wk == kMiss) & (ow == kMiss);
-            } else {
-                const bool c = (j & 1) != 0;
-                const float lx = c ? r1.x : r0.x, hx = c ? r1.y : r0.y, ly = c ? r1.z : r0.z, hy = c ? r1.w : r0.w;
-                const float lz = c ? r2.z : r2.x, hz = c ? r2.w : r2.y;
-                const int l0 = __float_as_int(r3.x), l1 = __float_as_int(r3.y);
-                const float clox = fmaf(lx, idx_, -oodx), chix = fmaf(hx, idx_, -oodx);
-                const float cloy = fmaf(ly, idy_, -oody), chiy = fmaf(hy, idy_, -oody);
-                const float cloz = fmaf(lz, idz_, -oodz), chiz = fmaf(hz, idz_, -oodz);
-                const float cmin = vmax3_(vmin_(clox, chix), vmin_(cloy, chiy), vmax_(vmin_(cloz, chiz), tmin));
-                const float cmax = vmin3_(vmax_(clox, chix), vmax_(cloy, chiy), vmin_(vmax_(cloz, chiz), hitT));
-                const int h = cmax >= cmin ? 1 : 0, m = __float_as_int(cmin);
-                const bool t0 = quad<kQuad0>(h) != 0, t1 = quad<kQuad1>(h) != 0;
-                const bool far_first =
-                    t1 & (!t0 | (__int_as_float(quad<kQuad1>(m)) < __int_as_float(quad<kQuad0>(m))));
-                push = t0 & t1 & (j == 0);
-                link = far_first ? l0 : l1;  // the farther one
-                at = sp;
-                top = sp + (t0 & t1);
-                none = !t0 & !t1;
-                first_link = far_first ? l1 : l0;
-            }
-            push = push & at_node;
-            // (the upload refuses trees deep enough to fill the stack: a
-            // launch that still did so is flagged, nothing written past it)
-            full = full | (push & (at >= 4 * rows));
-            lstack[(push & (at < 4 * rows)) ? (at >> 2) * 64 + (lane & ~3) + (at & 3) : rows * 64 + lane] = link;
-            pop = at_node ? none : pop;
-            next = at_node ? first_link : next;
-            sp = at_node ? (top < 4 * rows ? top : 4 * rows) : sp;
-        }
-        cur = pop ? (sp == 0 ? kSentinel : upper) : next;
-        sp -= pop & (sp > 0);
-    }
+    int* const own = lstack + (lane & ~3);
+    auto at_entry = [&](int e) -> int* { return own + (e >> 2) * 64 + (e & 3); };
+    while (__ballot(cur != kSentinel) != 0)
+        quad_step<WIDE>(nodes, tris, r, an, j, at_entry, 4 * (int)a.stack_rows, lstack + a.stack_rows * 64 + lane, cur, sp,
+                        hitT, hitId, full);
     if (full) atomicOr(a.errors, (uint32_t)RB_TRACE_ERR_STACK);
     if (live && j == 0) {
-        V2i r;
-        r.x = hitId;
+        V2i h;
+        h.x = hitId;
         // a miss reports the caller's tmax, bit for bit
-        r.y = hitId < 0 ? __float_as_int(((const __attribute__((address_space(1))) float*)(rays + 2 * ray + 1))[3])
+        h.y = hitId < 0 ? __float_as_int(((const __attribute__((address_space(1))) float*)(rays + 2 * ray + 1))[3])
                         : __float_as_int(hitT);
         const GI2 hits = MULTI ? (GI2)tab[batch].hits : second ? (GI2)a.hits2 : (GI2)a.hits;
-        hits[ray] = r;
+        hits[ray] = h;
     }
 }
 
@@ -1249,11 +1340,12 @@ static bool wide_walk(const rb_trace_config& cfg, rb_bvh_t bvh, uint32_t flags) 
 }
 
 // Whether a launch of at most n rays takes trace_quads: up to where both loops
-// are level on rays that scatter (the figures are at trace_quads), 1024 rays
-// per CU over the wide records and 768 over the binary ones, whose two
-// children use half of the quad.
-static bool few_rays(const rb_trace_config& cfg, bool wide, uint64_t n) {
-    return !cfg.speculative && n <= (uint64_t)dev().num_cus * (wide ? 1024 : 768);
+// are level on rays that scatter (the figures are at trace_quads), over the
+// wide and the binary records alike; three times as many camera rays, whose
+// quads share their lines and branches (384 Ki: 148 us in trace_steps, 115 in
+// trace_quads; 512 Ki: 171 and 161).
+static bool few_rays(const rb_trace_config& cfg, uint64_t n, bool coherent = false) {
+    return !cfg.speculative && n <= (uint64_t)dev().num_cus * (coherent ? 1536 : 512);
 }
 static uint32_t few_blocks(uint64_t n) { return (uint32_t)((n + 15) / 16); }
 static uint32_t stack_rows(rb_bvh_t bvh, bool wide) { return ((wide ? bvh->wide_stack : bvh->stack) + 3) / 4; }
@@ -1311,6 +1403,7 @@ rb_status launch_trace(rb_bvh_t bvh, const rb_ray* rays, uint32_t n, uint32_t fl
     a.threshold = cfg.fetch_threshold;
     a.leaf_gate = cfg.leaf_gate;
     if (wide) a.nodes = bvh->wnodes;
+    a.stack_rows = stack_rows(bvh, wide);
     // top-of-tree records in LDS: the speculative walk only
     a.top_nodes = !cfg.speculative ? 0 : cfg.lds_nodes < bvh->n_nodes ? cfg.lds_nodes : bvh->n_nodes;
     const size_t top_bytes = (size_t)a.top_nodes * 64;
@@ -1318,8 +1411,7 @@ rb_status launch_trace(rb_bvh_t bvh, const rb_ray* rays, uint32_t n, uint32_t fl
     if (lds > dev().lds_per_block)
         return fail(RB_ERR_INVALID, "trace config needs %zu bytes of LDS per block (stack %u x %u lanes + %u node records); "
                     "the device allows %zu", lds, cfg.lds_stack, cfg.block, a.top_nodes, dev().lds_per_block);
-    if (!counts && few_rays(cfg, wide, n)) {
-        a.stack_rows = stack_rows(bvh, wide);
+    if (!counts && few_rays(cfg, n, (flags & kCoherent) != 0)) {
         TraceKernel q = wide ? (any ? k_trace_few<true, true> : k_trace_few<false, true>)
                              : (any ? k_trace_few<true, false> : k_trace_few<false, false>);
         hipLaunchKernelGGL(q, dim3(few_blocks(n)), dim3(64), few_lds(a), stream, a);
@@ -1362,6 +1454,7 @@ rb_status launch_trace_pair(rb_bvh_t bvh, const rb_ray* rays0, uint32_t cap0, co
     TraceArgs a;
     std::memset(&a, 0, sizeof(a));
     a.nodes = wide ? bvh->wnodes : bvh->nodes;
+    a.stack_rows = stack_rows(bvh, wide);
     a.tris = bvh->tris4;
     a.index = bvh->index;
     a.rays = reinterpret_cast<const float4*>(rays0);
@@ -1380,8 +1473,7 @@ rb_status launch_trace_pair(rb_bvh_t bvh, const rb_ray* rays0, uint32_t cap0, co
     if (lds > dev().lds_per_block)
         return fail(RB_ERR_INVALID, "trace config needs %zu bytes of LDS per block; the device allows %zu", lds,
                     dev().lds_per_block);
-    if (few_rays(cfg, wide, a.n)) {
-        a.stack_rows = stack_rows(bvh, wide);
+    if (few_rays(cfg, a.n)) {
         TraceKernel q = wide ? k_trace_few_pair<true> : k_trace_few_pair<false>;
         hipLaunchKernelGGL(q, dim3(few_blocks(a.n)), dim3(64), few_lds(a), stream, a);
         const hipError_t e = hipGetLastError();
@@ -1451,11 +1543,11 @@ static rb_status launch_trace_sets_pass(const BatchSet* b, uint32_t nb, hipStrea
         std::memset(&a, 0, sizeof(a));
         a.errors = dev().errors;
         a.n = (uint32_t)total;
+        a.stack_rows = rows;
         a.chunk = cfg.chunk;
         a.threshold = cfg.fetch_threshold;
         a.leaf_gate = cfg.leaf_gate;
-        if (few_rays(cfg, wide, total)) {
-            a.stack_rows = rows;
+        if (few_rays(cfg, total)) {
             BatchKernel q = wide ? k_trace_few_batch<true> : k_trace_few_batch<false>;
             hipLaunchKernelGGL(q, dim3(few_blocks(total)), dim3(64), few_lds(a), stream, a, t);
             const hipError_t e = hipGetLastError();

@@ -1,9 +1,10 @@
-"""GPU parity of the two loops a launch may take: a quad of lanes per ray for
-launches of few rays, a lane per ray for the rest.  The same rays traced alone
-and as the head of a launch past the line (1024 rays per CU) give the same
-(id, t), bit for bit, which are the oracle's -- over the wide and the binary
-records, closest and any hit, masked, at the edges of a block (16 rays), with
-leaves of more triangles than a quad has lanes, ties, NaN and zero rays."""
+"""GPU parity of the loops a launch may take: a quad of lanes per ray for
+launches of few rays, a lane per ray for the rest and a quad for each of its
+waves' last rays.  The same rays traced alone and as the head or the end of a
+launch past the line (512 rays per CU) give the same (id, t), bit for bit, which
+are the oracle's -- over the wide and the binary records, closest and any hit,
+masked, at the edges of a block (16 rays), with leaves of more triangles than a
+quad has lanes, ties, NaN and zero rays, and stacks that leave their LDS rows."""
 import numpy as np
 import pytest
 
@@ -11,7 +12,7 @@ from conftest import random_rays, random_triangles
 
 pytestmark = pytest.mark.gpu
 
-PAST = 1024 * 256 + 1
+PAST = 512 * 256 + 1
 
 
 @pytest.fixture(scope="module")
@@ -51,25 +52,31 @@ def _trace(gpu, tr, rays, n, any_hit, mask):
 @pytest.mark.parametrize("any_hit", [False, True])
 @pytest.mark.parametrize("masked", [False, True])
 @pytest.mark.parametrize("n", [1, 15, 17, 4099])
-def test_both_loops_give_the_same_hits(gpu, orc, scene, wide, any_hit, masked, n):
+@pytest.mark.parametrize("lds_stack,block", [(16, 256), (8, 64)])
+def test_the_loops_give_the_same_hits(gpu, orc, scene, wide, any_hit, masked, n, lds_stack, block):
     tr, c2, centre = scene
     rays = _rays(n, centre)
     mask = (np.arange(PAST) % 3 != 0).astype(np.uint8) if masked else None
     cfg = gpu.get_trace_config()
-    gpu.set_trace_config(**{**cfg, "wide": wide})
+    gpu.set_trace_config(**{**cfg, "wide": wide, "lds_stack": lds_stack, "block": block})
     try:
         few = _trace(gpu, tr, rays, n, any_hit, mask)
-        tail = np.zeros((PAST - n, 8), np.float32)
-        tail[:, 0:3] = 1e6  # rays that miss the root
-        tail[:, 4] = tail[:, 7] = 1.0
-        many = _trace(gpu, tr, np.concatenate([rays, tail]), PAST, any_hit, mask)[:n]
+        rest = np.zeros((PAST - n, 8), np.float32)
+        rest[:, 0:3] = 1e6  # rays that miss the root
+        rest[:, 4] = rest[:, 7] = 1.0
+        head = _trace(gpu, tr, np.concatenate([rays, rest]), PAST, any_hit, mask)[:n]
+        if masked:
+            mask = np.concatenate([mask[n:], mask[:n]])
+        end = _trace(gpu, tr, np.concatenate([rest, rays]), PAST, any_hit, mask)[PAST - n:]
     finally:
         gpu.set_trace_config(**cfg)
-    assert np.array_equal(few["id"], many["id"])
-    assert np.array_equal(few["t"].view(np.uint32), many["t"].view(np.uint32))
+    mask = np.arange(PAST) % 3 != 0
+    for many in (head, end):
+        assert np.array_equal(few["id"], many["id"])
+        assert np.array_equal(few["t"].view(np.uint32), many["t"].view(np.uint32))
     ok = np.isfinite(rays[:, :7]).all(axis=1)
     if masked:
-        ok &= mask[:n] != 0
+        ok &= mask[:n]
     oid, ot = orc.trace_compact2(*c2, np.ascontiguousarray(rays[ok]), any_hit=any_hit)
     assert np.array_equal(few["id"][ok], oid) and np.array_equal(few["t"][ok].view(np.uint32), ot.view(np.uint32))
     if n > 1000 and not masked:
