@@ -23,8 +23,8 @@
 // Connection estimator: pick a light path j uniformly, then one of its n_j
 // stored vertices uniformly, and scale by n_j / connections (unbiased).
 #pragma once
+#include "rb_quad.h"
 #include "rb_shade.h"
-#include "../../include/rb_trace_device.h"
 
 namespace rb {
 
@@ -224,34 +224,69 @@ __device__ __forceinline__ bool light_vertex(const SceneDev& S, const Rng& rng, 
     return true;
 }
 
-// The light paths after their first trace, one thread per path: depth 0's
-// hit comes from the launch that traced the light rays with the camera rays
-// (queue 0, hit q of entry q); every later depth's ray is traced by the
-// thread itself with rb_trace_one, whose (id, t) equal the persistent
-// kernel's bit for bit.  One launch for all depths replaces a trace launch
-// per depth, whose ramp-up and tail dominated the thinning later depths.
+// The light paths after their first trace, a quad of lanes per path and sixteen
+// paths at a time in a one-wave block: depth 0's hit comes from the launch that
+// traced the light rays with the camera rays (queue 0, hit q of entry q); every
+// later depth's rays are traced here (quad_walk, whose (id, t) equal the trace
+// kernels' bit for bit) by the wave that shades them, all four lanes of a quad
+// alike.  One launch for all depths replaces a trace launch per depth, whose
+// ramp-up and tail dominated the thinning later depths.
+// Bound by the chain of a path's traversal steps (a lane per path with
+// rb_trace_one before: 175k paths of depth 6 in 2M triangles 717 -> 538 us, 22k
+// paths in 500k triangles 577 -> 197).  A wave shades once twelve of its
+// quads wait for it (576 us; eight 602, four 608, and 618 with all sixteen in
+// step), five waves to a SIMD (four, without the bound on registers: 576; six,
+// with spills: 564).
 // Optional counters: rays traced (ray_counter) and rays per depth
 // (depth_counter[d], d >= 1).
-__global__ __launch_bounds__(256) void k_light_walk(SceneDev S, RngArg rng_a, LightPath P, LvcBufs C, rb_bvh_dev bv,
-                                                    unsigned long long* ray_counter,
-                                                    unsigned long long* depth_counter) {
+template <bool WIDE>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_light_walk(
+    SceneDev S, RngArg rng_a, LightPath P, LvcBufs C, const float4* nodes, const float4* tris, uint32_t rows,
+    uint32_t* errors, unsigned long long* ray_counter, unsigned long long* depth_counter) {
+    constexpr uint32_t kWait = 12;  // quads that wait for their vertex before the wave shades
+    extern __shared__ int lstack[];
     const Rng rng = rng_a.get();
     const uint32_t count = P.cnt[0];
-    for (uint32_t q = blockIdx.x * blockDim.x + threadIdx.x; q < count; q += gridDim.x * blockDim.x) {
-        const uint32_t j = P.q[q];
-        int2 h = P.hit[q];
-        float4 o = P.ray[2 * (size_t)j], dd = P.ray[2 * (size_t)j + 1];
-        float4 a = P.alpha[j];
-        uint32_t mask = P.mask[j];
-        for (uint32_t d = 0; h.x >= 0 && light_vertex(S, rng, C, j, d, h, &o, &dd, &a, &mask);) {
-            d++;
-            const rb_ray r = {o.x, o.y, o.z, o.w, dd.x, dd.y, dd.z, dd.w};
-            const rb_hit hh = rb_trace_one(bv, r, RB_CLOSEST);
-            h = make_int2(hh.id, __float_as_int(hh.t));
-            if (ray_counter) atomicAdd(ray_counter, 1ull);
-            if (depth_counter) atomicAdd(depth_counter + d, 1ull);
+    const uint32_t lane = threadIdx.x;
+    uint32_t next = blockIdx.x * 16 + (lane >> 2);  // the quad's next path
+    uint32_t j = 0, d = 0, mask = 0;
+    float4 o = {}, dd = {}, a = {};
+    RayRegs r = {};
+    float t = 0.f;
+    int cur = kSentinel, sp = 0, id = -1;
+    bool full = false;
+    uint32_t rays = 0;  // rays of the quad
+    while (true) {
+        if (cur == kSentinel) {
+            int2 h = make_int2(id, __float_as_int(t));
+            if (id < 0 && next < count) {
+                j = P.q[next];
+                h = P.hit[next];
+                o = P.ray[2 * (size_t)j], dd = P.ray[2 * (size_t)j + 1];
+                a = P.alpha[j];
+                mask = P.mask[j];
+                d = 0;
+                next += gridDim.x * 16;
+            }
+            id = -1;
+            if (h.x >= 0 && light_vertex(S, rng, C, j, d, h, &o, &dd, &a, &mask)) {
+                d++;
+                r = ray_regs(V4f{o.x, o.y, o.z, o.w}, V4f{dd.x, dd.y, dd.z, dd.w});
+                t = dd.w;
+                cur = 0;
+                sp = 0;
+                if (depth_counter && (lane & 3) == 0) atomicAdd(depth_counter + d, 1ull);
+                rays++;
+            }
         }
+        const uint32_t busy = (uint32_t)__popcll(__ballot(cur != kSentinel)) / 4;
+        const uint64_t more = __ballot(next < count);
+        if (busy == 0 && more == 0) break;
+        quad_walk<WIDE>((GF4)nodes, (GF4)tris, r, false, lstack, rows, busy > 16 - kWait ? 16 - kWait : 0, cur, sp,
+                        t, id, full);
     }
+    if (full && errors) atomicOr(errors, (uint32_t)RB_TRACE_ERR_STACK);
+    if (ray_counter && (lane & 3) == 0) atomicAdd(ray_counter, (unsigned long long)rays);
 }
 
 // Gather the rays of the emitted light paths into a dense buffer for tracing.

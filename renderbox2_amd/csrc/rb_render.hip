@@ -128,6 +128,11 @@ constexpr uint32_t kMaxConn = 8;
 
 namespace rb {
 
+// Blocks of k_light_walk: as many as the card holds at once at most.
+static uint32_t walk_blocks(uint32_t paths) {
+    return std::min((uint32_t)(((uint64_t)paths + 15) / 16), dev().num_cus * 32);
+}
+
 struct BdArgs {
     LvcBufs C;
     uint32_t nconn;
@@ -978,9 +983,12 @@ struct CameraJob : RenderJob {
             if (p.ray_counter) hipLaunchKernelGGL(k_add_count, dim3(1), dim3(64), 0, s, LP.cnt + 0, p.ray_counter);
             if (p.light_path_counter)
                 hipLaunchKernelGGL(k_add_count, dim3(1), dim3(64), 0, s, LP.cnt + 0, p.light_path_counter);
-            const rb_bvh_dev bv = device_view(bvh);
-            hipLaunchKernelGGL(k_light_walk, dim3(grid_of(NL)), dim3(256), 0, s, S, rng_arg(p.seed, RNG_LIGHT), LP, B.C,
-                               bv, p.ray_counter, p.light_path_counter);
+            const bool wide = dev().cfg.wide && !dev().cfg.speculative && bvh->wnodes;
+            const uint32_t rows = stack_rows(bvh, wide);
+            hipLaunchKernelGGL(wide ? k_light_walk<true> : k_light_walk<false>, dim3(walk_blocks(NL)),
+                               dim3(64), quad_lds(rows), s, S, rng_arg(p.seed, RNG_LIGHT), LP, B.C,
+                               wide ? bvh->wnodes : bvh->nodes, bvh->tris4, rows, dev().errors, p.ray_counter,
+                               p.light_path_counter);
             phase = 2;
         }
         if (phase == 2) {
