@@ -51,6 +51,7 @@ __device__ __forceinline__ rb_hit rb_trace_one(const rb_bvh_dev& b, const rb_ray
     int sp = 0;
     stack[0] = RB_DEV_SENTINEL;
     int nodeAddr = 0, leafAddr = 0, hitIndex = -1;
+    bool strict = false;
     /* the upload refuses trees deep enough to fill the stack; a push past
        it is dropped and flagged (rb_trace_errors) */
 #define RB_DEV_PUSH(v)                                               \
@@ -70,6 +71,18 @@ __device__ __forceinline__ rb_hit rb_trace_one(const rb_bvh_dev& b, const rb_ray
     /* closest hit over the wide records: the same (id, t), about half the
        record fetches (every leaf the binary walk tests is tested) */
     const float4* wnodes = any ? nullptr : reinterpret_cast<const float4*>(b.wnodes);
+    /* after the wide records, two rows per reference: the box of its leaf.  The
+       records' boxes are a little larger; a hit counts if this one passes */
+    const float4* boxes = wnodes ? wnodes + 4 * (size_t)b.n_wnodes : nullptr;
+    auto box_passes = [&](int ref) -> bool {
+        const float4 p = boxes[2 * (size_t)ref], q = boxes[2 * (size_t)ref + 1];
+        const float lox = fmaf(p.x, idx, -oodx), hix = fmaf(p.y, idx, -oodx);
+        const float loy = fmaf(p.z, idy, -oody), hiy = fmaf(p.w, idy, -oody);
+        const float loz = fmaf(q.x, idz, -oodz), hiz = fmaf(q.y, idz, -oodz);
+        return fminf(fminf(fmaxf(lox, hix), fmaxf(loy, hiy)), fmaxf(loz, hiz)) >=
+               fmaxf(fmaxf(fminf(lox, hix), fminf(loy, hiy)), fmaxf(fminf(loz, hiz), tmin));
+    };
+walk:
     while (nodeAddr != RB_DEV_SENTINEL) {
         /* wide records until a leaf is reached */
         while (wnodes && (uint32_t)nodeAddr < (uint32_t)RB_DEV_SENTINEL && leafAddr >= 0) {
@@ -189,7 +202,8 @@ __device__ __forceinline__ rb_hit rb_trace_one(const rb_bvh_dev& b, const rb_ray
                         const float Dy = fmaf(dz, v2.z, fmaf(dy, v2.y, dx * v2.x));
                         const float v = fmaf(t, Dy, Oy);
                         if (v >= 0.0f && u + v <= 1.0f) {
-                            const bool take = t < hitT || b.index[first + k] < b.index[hitIndex];
+                            const bool take = (t < hitT || b.index[first + k] < b.index[hitIndex]) &&
+                                              !(strict && !box_passes((int)(first + k)));
                             if (take) {
                                 hitT = t;
                                 hitIndex = (int)(first + k);
@@ -208,6 +222,14 @@ __device__ __forceinline__ rb_hit rb_trace_one(const rb_bvh_dev& b, const rb_ray
     }
 #undef RB_DEV_PUSH
 #undef RB_DEV_POP
+    if (boxes && hitIndex >= 0 && !strict && !box_passes(hitIndex)) { /* again, counting only such hits */
+        strict = true;
+        hitT = ray.tmax;
+        sp = 0;
+        nodeAddr = leafAddr = 0;
+        hitIndex = -1;
+        goto walk;
+    }
     rb_hit h;
     h.id = hitIndex < 0 ? -1 : (int32_t)b.index[hitIndex];
     h.t = hitT;

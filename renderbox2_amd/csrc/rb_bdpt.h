@@ -241,8 +241,9 @@ __device__ __forceinline__ bool light_vertex(const SceneDev& S, const Rng& rng, 
 // (depth_counter[d], d >= 1).
 template <bool WIDE>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_light_walk(
-    SceneDev S, RngArg rng_a, LightPath P, LvcBufs C, const float4* nodes, const float4* tris, uint32_t rows,
-    uint32_t* errors, unsigned long long* ray_counter, unsigned long long* depth_counter) {
+    SceneDev S, RngArg rng_a, LightPath P, LvcBufs C, const float4* nodes, const float4* tris,
+    const float4* boxes, float reach, uint32_t rows, uint32_t* errors, unsigned long long* ray_counter,
+    unsigned long long* depth_counter) {
     constexpr uint32_t kWait = 12;  // quads that wait for their vertex before the wave shades
     extern __shared__ int lstack[];
     const Rng rng = rng_a.get();
@@ -252,14 +253,20 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_
     uint32_t j = 0, d = 0, mask = 0;
     float4 o = {}, dd = {}, a = {};
     RayRegs r = {};
-    float t = 0.f;
-    int cur = kSentinel, sp = 0, id = -1;
+    QuadHit hit = {0.f, -1, 0, false};
+    int cur = kSentinel, sp = 0;
     bool full = false;
     uint32_t rays = 0;  // rays of the quad
     while (true) {
         if (cur == kSentinel) {
-            int2 h = make_int2(id, __float_as_int(t));
-            if (id < 0 && next < count) {
+            int2 h = make_int2(hit.id, __float_as_int(hit.t));
+            const bool again = WIDE && walk_again((GF4)boxes, reach, r, hit);
+            if (again) {
+                hit = {dd.w, -1, 0, true};
+                cur = 0;
+                sp = 0;
+                h.x = -1;
+            } else if (hit.id < 0 && next < count) {
                 j = P.q[next];
                 h = P.hit[next];
                 o = P.ray[2 * (size_t)j], dd = P.ray[2 * (size_t)j + 1];
@@ -268,11 +275,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_
                 d = 0;
                 next += gridDim.x * 16;
             }
-            id = -1;
+            if (!again) hit.id = -1;
             if (h.x >= 0 && light_vertex(S, rng, C, j, d, h, &o, &dd, &a, &mask)) {
                 d++;
                 r = ray_regs(V4f{o.x, o.y, o.z, o.w}, V4f{dd.x, dd.y, dd.z, dd.w});
-                t = dd.w;
+                hit = {dd.w, -1, 0, false};
                 cur = 0;
                 sp = 0;
                 if (depth_counter && (lane & 3) == 0) atomicAdd(depth_counter + d, 1ull);
@@ -282,8 +289,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_
         const uint32_t busy = (uint32_t)__popcll(__ballot(cur != kSentinel)) / 4;
         const uint64_t more = __ballot(next < count);
         if (busy == 0 && more == 0) break;
-        quad_walk<WIDE>((GF4)nodes, (GF4)tris, r, false, lstack, rows, busy > 16 - kWait ? 16 - kWait : 0, cur, sp,
-                        t, id, full);
+        quad_walk<WIDE>((GF4)nodes, (GF4)tris, (GF4)boxes, r, false, lstack, rows,
+                        busy > 16 - kWait ? 16 - kWait : 0, cur, sp, hit, full);
     }
     if (full && errors) atomicOr(errors, (uint32_t)RB_TRACE_ERR_STACK);
     if (ray_counter && (lane & 3) == 0) atomicAdd(ray_counter, (unsigned long long)rays);

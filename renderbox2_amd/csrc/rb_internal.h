@@ -202,6 +202,20 @@ rb_status export_wide(const std::vector<uint32_t>& bin, std::vector<uint32_t>& w
 // *entries: the most stack entries a ray can need.
 rb_status export_walk(const std::vector<uint32_t>& bin, uint32_t n_refs, std::vector<uint32_t>& walk,
                       uint32_t* entries);
+// The boxes that closest hits and occlusion over the walk's records answer for,
+// eight floats per reference (lo.x, hi.x, lo.y, hi.y, lo.z, hi.z of its leaf,
+// 0, 0): the leaf's box as a record of export_wide holds it where the tree has
+// those, else as the binary record does.  The records' own boxes are a little
+// larger, so that a ray through the crack between two triangles, which passes
+// no leaf's box here, can meet a triangle there (10 of 128 M rays in
+// tessellated rooms, one in six of rays aimed at the edges of a wall's
+// triangles); a hit near the edge of its triangle counts once its leaf's box
+// passes, and a ray whose hit does not count is walked again with that test on
+// every hit.  (Cost: 605 -> 620 us for 2 Mi diffuse rays, the reference of the
+// hit and its distance from the edge kept with it and 1 ray in 80 tested;
+// testing every hit as it is found reads two more rows for each.)  *reach: rays from within this distance of the world's origin
+// need the test only near an edge (edge_band), others always.
+void leaf_boxes(const std::vector<uint32_t>& bin, uint32_t n_refs, std::vector<float>& box, float* reach);
 // Depth of the deepest inner record of an MI355X node array (root = 0);
 // UINT32_MAX when a link leaves the array or the links form a cycle.  A
 // traversal holds at most depth + 1 stack entries (the sentinel, then one

@@ -625,6 +625,48 @@ rb_status export_walk(const std::vector<uint32_t>& bin, uint32_t n_refs, std::ve
     return fail(RB_ERR_UNSUPPORTED, "the tree is too deep for the wide walk's stack");
 }
 
+void leaf_boxes(const std::vector<uint32_t>& bin, uint32_t n_refs, std::vector<float>& box, float* reach) {
+    box.assign(8 * ((size_t)n_refs + 1), 0.0f);
+    auto set = [&](int32_t link, const float lo[3], const float hi[3]) {
+        const uint32_t l = ~(uint32_t)link, first = l >> 5, cnt = l & 31u;
+        for (uint32_t r = first; r < first + cnt && r < n_refs; r++)
+            for (int a = 0; a < 3; a++) {
+                box[8 * (size_t)r + 2 * a] = lo[a];
+                box[8 * (size_t)r + 2 * a + 1] = hi[a];
+            }
+    };
+    float far = 0.0f;
+    for (size_t r = 0; r < bin.size() / 16; r++)
+        for (int c = 0; c < 2; c++) {
+            const WalkChild k = walk_child(&bin[r * 16], c);
+            if (empty_leaf(k.link)) continue;
+            if (r == 0)
+                for (int a = 0; a < 3; a++) far = std::max(far, std::max(std::fabs(k.lo[a]), std::fabs(k.hi[a])));
+            if (k.link < 0) set(k.link, k.lo, k.hi);
+        }
+    *reach = 2.0f * far;
+    std::vector<uint32_t> wide;
+    if (!wide_fits_stack(layout_depth(bin)) || export_wide(bin, wide) != RB_OK) {
+        set_error("");
+        return;
+    }
+    for (size_t r = 0; r < wide.size() / kWideWords; r++) {
+        const uint32_t* w = &wide[r * kWideWords];
+        for (int c = 0; c < 4; c++) {
+            const int32_t link = (int32_t)w[10 + c];
+            if (link >= 0 || empty_leaf(link)) continue;
+            float b[2][3];
+            for (int a = 0; a < 3; a++) {
+                float p;
+                std::memcpy(&p, &w[a], 4);
+                const float s = std::ldexp(1.0f, (int)(w[3] >> (8 * a) & 0xFFu) - 127);
+                for (int e = 0; e < 2; e++) b[e][a] = std::fmaf((float)(w[4 + 2 * a + e] >> (8 * c) & 0xFFu), s, p);
+            }
+            set(link, b[0], b[1]);
+        }
+    }
+}
+
 uint32_t layout_depth(const std::vector<uint32_t>& nodes) {
     const uint32_t n = (uint32_t)(nodes.size() / 16);
     if (n == 0) return 0;

@@ -103,6 +103,30 @@ __device__ __forceinline__ RayRegs ray_regs(V4f o, V4f d) {
     return r;
 }
 
+// Whether a hit on reference `ref`, found over wide records, counts (leaf_boxes):
+// its leaf's box passes the slab test.
+__device__ __forceinline__ bool leaf_box_passes(GF4 boxes, uint32_t ref, float tmin, float idx, float idy, float idz,
+                                                float oodx, float oody, float oodz) {
+    const V4f a = boxes[2 * (size_t)ref], b = boxes[2 * (size_t)ref + 1];
+    const float lox = fmaf(a.x, idx, -oodx), hix = fmaf(a.y, idx, -oodx);
+    const float loy = fmaf(a.z, idy, -oody), hiy = fmaf(a.w, idy, -oody);
+    const float loz = fmaf(b.x, idz, -oodz), hiz = fmaf(b.y, idz, -oodz);
+    const float near = vmax3_(vmin_(lox, hix), vmin_(loy, hiy), vmax_(vmin_(loz, hiz), tmin));
+    const float far = vmin3_(vmax_(lox, hix), vmax_(loy, hiy), vmax_(loz, hiz));
+    return far >= near;
+}
+__device__ __forceinline__ bool leaf_box_passes(GF4 boxes, uint32_t ref, const RayRegs& r) {
+    return leaf_box_passes(boxes, ref, r.tmin, r.idx, r.idy, r.idz, r.oodx, r.oody, r.oodz);
+}
+
+// What a walk over wide records has found: the hit, and the reference it lies
+// on, complemented when it lies near an edge of its triangle.
+struct QuadHit {
+    float t;
+    int id, ref;
+    bool strict;  // a hit counts only if its leaf's box passes: the ray is walked a second time
+};
+
 // One step of every quad of the wave: four lanes per ray, each testing one
 // child of a record (two of them over the binary records) or one triangle of
 // a leaf.  No lane branches: the wave skips the node or the triangle half when
@@ -112,11 +136,12 @@ __device__ __forceinline__ RayRegs ray_regs(V4f o, V4f d) {
 // at_entry(e): where the quad keeps stack entry e (room entries).
 template <bool WIDE, typename Entry>
 __device__ __forceinline__ void quad_step(GF4 nodes, GF4 tris, const RayRegs& ray, bool an, int j, Entry at_entry,
-                                          int room, int* spare, int& cur, int& sp, float& hitT, int& hitId,
-                                          bool& full) {
+                                          int room, int* spare, GF4 boxes, int& cur, int& sp, QuadHit& h, bool& full) {
     const float ox = ray.ox, oy = ray.oy, oz = ray.oz, dx = ray.dx, dy = ray.dy, dz = ray.dz, tmin = ray.tmin;
     const float idx_ = ray.idx, idy_ = ray.idy, idz_ = ray.idz;
     const float oodx = ray.oodx, oody = ray.oody, oodz = ray.oodz;
+    const float hitT = h.t;
+    const int hitId = h.id;
     const bool at_tri = cur < 0;
     const bool at_node = (uint32_t)cur < (uint32_t)kSentinel;
     const uint32_t l = ~(uint32_t)cur, cnt = l & 31u;
@@ -141,10 +166,13 @@ __device__ __forceinline__ void quad_step(GF4 nodes, GF4 tris, const RayRegs& ra
         const float Dy = fmaf(dz, r2.z, fmaf(dy, r2.y, dx * r2.x));
         const float v = fmaf(t, Dy, Oy);
         const int id = __float_as_int(r3.x);
-        const bool hit = there & (t > tmin) & ((t < hitT) | ((t == hitT) & (id < hitId))) & (u >= 0.0f) &
-                         (v >= 0.0f) & (u + v <= 1.0f);
+        const float uv = u + v;
+        bool hit = there & (t > tmin) & ((t < hitT) | ((t == hitT) & (id < hitId))) & (u >= 0.0f) & (v >= 0.0f) &
+                   (uv <= 1.0f);
         bool found = false;
         if (__ballot(hit) != 0) {
+            if (WIDE && __ballot(hit & h.strict) != 0)
+                hit = hit & (!h.strict | leaf_box_passes(boxes, hit ? rec : 0u, ray));
             // one after the other the triangles would leave the nearest
             // hit (the lowest id on ties), or the first for any hit
             float tn = hit ? t : __builtin_inff();
@@ -156,12 +184,20 @@ __device__ __forceinline__ void quad_step(GF4 nodes, GF4 tris, const RayRegs& ra
             found = best != 0x7FFFFFFF;
             const bool take = found & (own == best);
             int tb = take ? __float_as_int(t) : 0, ib = take ? id : 0;
+            int rb = 0;
+            if (WIDE) {
+                const float edge = vmin3_(u, v, 1.0f - uv);
+                rb = take ? (edge < r3.y ? ~(int)rec : (int)rec) : 0;
+                rb |= quad<kQuadXor1>(rb);
+                rb |= quad<kQuadXor2>(rb);
+            }
             tb |= quad<kQuadXor1>(tb);
             ib |= quad<kQuadXor1>(ib);
             tb |= quad<kQuadXor2>(tb);
             ib |= quad<kQuadXor2>(ib);
-            hitT = found ? __int_as_float(tb) : hitT;
-            hitId = found ? ib : hitId;
+            h.t = found ? __int_as_float(tb) : h.t;
+            h.id = found ? ib : h.id;
+            h.ref = found ? rb : h.ref;
         }
         const bool over = found & an;
         pop = at_tri & (cnt <= 4) & !over;
@@ -246,20 +282,29 @@ inline size_t quad_lds(uint32_t rows) { return (rows + 1) * 64 * sizeof(int); }
 
 // The walk of one ray per quad of a one-wave block: cur is 0 for a quad whose ray
 // starts and kSentinel for one whose ray has ended (or that has none); the
-// results are hitT and hitId (-1: a miss).  Steps are made while more than
-// `until` quads have a ray under way.
+// result is h (h.id -1: a miss).  Steps are made while more than `until` quads
+// have a ray under way.
 // stack: quad_lds(rows) bytes; a quad's entry e lies in row e / 4, column e % 4
 // of its four words, and the row behind the last takes the stores of lanes that
 // have nothing to push.
 template <bool WIDE>
-__device__ __forceinline__ void quad_walk(GF4 nodes, GF4 tris, const RayRegs& r, bool an, int* stack, uint32_t rows,
-                                          uint32_t until, int& cur, int& sp, float& hitT, int& hitId, bool& full) {
+__device__ __forceinline__ void quad_walk(GF4 nodes, GF4 tris, GF4 boxes, const RayRegs& r, bool an, int* stack,
+                                          uint32_t rows, uint32_t until, int& cur, int& sp, QuadHit& h, bool& full) {
     const int lane = threadIdx.x, j = lane & 3;
     int* const own = stack + (lane & ~3);
     auto at_entry = [&](int e) -> int* { return own + (e >> 2) * 64 + (e & 3); };
     while ((uint32_t)__popcll(__ballot(cur != kSentinel)) > 4 * until)
-        quad_step<WIDE>(nodes, tris, r, an, j, at_entry, 4 * (int)rows, stack + rows * 64 + lane, cur, sp, hitT, hitId,
+        quad_step<WIDE>(nodes, tris, r, an, j, at_entry, 4 * (int)rows, stack + rows * 64 + lane, boxes, cur, sp, h,
                         full);
+}
+
+// Whether an ended walk over wide records has to be made again, strictly: its
+// hit lies near an edge, or its ray started out of reach, and the leaf's box
+// does not pass.
+__device__ __forceinline__ bool walk_again(GF4 boxes, float reach, const RayRegs& r, const QuadHit& h) {
+    if (h.id < 0 || h.strict) return false;
+    const bool far = !(vmax3_(fabsf(r.ox), fabsf(r.oy), fabsf(r.oz)) <= reach);
+    return (h.ref < 0 || far) && !leaf_box_passes(boxes, (uint32_t)(h.ref < 0 ? ~h.ref : h.ref), r);
 }
 
 }  // namespace rb

@@ -69,6 +69,8 @@ struct TraceArgs {
     uint32_t leaf_gate;  // non-speculative: leave the inner-node phase once <= this many lanes still search
     uint32_t top_nodes;  // node records 0..top_nodes-1 are read from a copy in LDS
     uint32_t stack_rows;  // a ray's stack needs at most four times as many entries
+    const float4* boxes;  // wide records: leaf_boxes
+    float reach;
 };
 
 constexpr uint32_t kMaxBatch = 64;
@@ -84,6 +86,8 @@ struct BatchDesc {
     uint32_t n;             // ray count, or the bound of *n_dev
     uint32_t start;         // first global ray index of the batch (set by the kernel)
     uint32_t any;           // 1: terminate on the first hit
+    float reach;
+    const float4* boxes;    // wide records: leaf_boxes
 };
 
 struct BatchTable {
@@ -333,6 +337,8 @@ __device__ __forceinline__ void trace_steps(const TraceArgs& a, const BatchDesc*
     // cur: the ray's next step -- an inner record (>= 0), a leaf's remaining
     // triangles ~(first << 5 | count), or kSentinel when the ray is done
     int cur = kSentinel, sp = 0, hitId = -1;
+    int hitRef = 0;       // WIDE: as QuadHit's
+    bool strict = false;  // WIDE: likewise
     bool live = false;  // the lane holds a ray whose result is not stored yet
     uint32_t mine = 0;  // the ray's index in the launch
     uint32_t batch = 0;  // MULTI: its batch
@@ -355,6 +361,8 @@ __device__ __forceinline__ void trace_steps(const TraceArgs& a, const BatchDesc*
     auto any = [&]() -> bool { return MULTI ? tab[batch].any != 0 : PAIR ? !second() && a.any0 != 0 : ANY_T; };
     auto rayidx = [&]() -> uint32_t { return MULTI ? mine - tab[batch].start : second() ? mine - n0 : mine; };
     auto rays = [&]() -> GF4 { return MULTI ? (GF4)tab[batch].rays : second() ? (GF4)a.rays2 : (GF4)a.rays; };
+    auto boxes = [&]() -> GF4 { return MULTI ? (GF4)tab[batch].boxes : (GF4)a.boxes; };
+    auto reach = [&]() -> float { return MULTI ? tab[batch].reach : a.reach; };
     auto hits = [&]() -> GI2 { return MULTI ? (GI2)tab[batch].hits : second() ? (GI2)a.hits2 : (GI2)a.hits; };
 
     // The upload refuses trees deep enough to fill the stack, so the last
@@ -408,6 +416,27 @@ __device__ __forceinline__ void trace_steps(const TraceArgs& a, const BatchDesc*
         const uint64_t tm = __ballot(cur == kSentinel);
         const uint32_t busy = 64 - __popcll(tm);
         if (busy == 0 || (pool.drained ? busy <= tail : busy < a.threshold)) {
+            if (WIDE) {
+                // hits that may not count (leaf_boxes): those rays again
+                bool again = false;
+                if (cur == kSentinel && live && hitId >= 0 && !strict) {
+                    const bool far = !(vmax3_(fabsf(ox), fabsf(oy), fabsf(oz)) <= reach());
+                    if (hitRef < 0 || far)
+                        again = !leaf_box_passes(boxes(), (uint32_t)(hitRef < 0 ? ~hitRef : hitRef), tmin, idx_, idy_, idz_,
+                                                 oodx, oody, oodz);
+                }
+                if (__ballot(again) != 0) {
+                    if (again) {
+                        hitT = __builtin_canonicalizef(
+                            ((const __attribute__((address_space(1))) float*)(rays() + 2 * (size_t)rayidx() + 1))[3]);
+                        hitId = -1;
+                        strict = true;
+                        sp = 0;
+                        cur = 0;
+                    }
+                    continue;
+                }
+            }
             if (cur == kSentinel && live) store();
             uint32_t done = pool.drained;
             if (!COUNT && done && busy) {
@@ -423,7 +452,7 @@ __device__ __forceinline__ void trace_steps(const TraceArgs& a, const BatchDesc*
                     to[0] = V4f{ox, oy, oz, tmin};
                     to[1] = V4f{dx, dy, dz, hitT};
                     to[2] = __builtin_bit_cast(V4f, V4i{hitId, cur, sp, (int)mine});
-                    to[3] = __builtin_bit_cast(V4f, V4i{(int)batch, (int)lane, 0, 0});
+                    to[3] = __builtin_bit_cast(V4f, V4i{(int)batch, (int)lane, hitRef, strict ? 1 : 0});
                     for (int e = R; e < sp; e++) ((int*)to)[16 + e - R] = spill[e - R];
                 }
                 asm volatile("" ::: "memory");
@@ -480,6 +509,7 @@ __device__ __forceinline__ void trace_steps(const TraceArgs& a, const BatchDesc*
                 }
                 sp = 0;
                 hitId = -1;
+                strict = false;
                 live = true;
                 cur = (mk && mk[i] == 0) ? kSentinel : 0;
                 if (COUNT) { c_inner = 0; c_tri = 0; c_leaf = 0; }
@@ -612,9 +642,12 @@ __device__ __forceinline__ void trace_steps(const TraceArgs& a, const BatchDesc*
                 const float v = fmaf(t, Dy, Oy);
                 // ties at equal t go to the lowest id
                 const bool nearer = t < hitT || (t == hitT && id < hitId);
-                if (t > tmin && nearer && u >= 0.0f && v >= 0.0f && u + v <= 1.0f) {
+                const float uv = u + v;
+                if (t > tmin && nearer && u >= 0.0f && v >= 0.0f && uv <= 1.0f &&
+                    (!WIDE || !strict || leaf_box_passes(boxes(), l >> 5, tmin, idx_, idy_, idz_, oodx, oody, oodz))) {
                     hitT = t;
                     hitId = id;
+                    if (WIDE) hitRef = vmin3_(u, v, 1.0f - uv) < r3.y ? (int)~(l >> 5) : (int)(l >> 5);
                     if (any()) {
                         cur = kSentinel;
                         done = false;
@@ -635,12 +668,11 @@ __device__ __forceinline__ void trace_steps(const TraceArgs& a, const BatchDesc*
         const V4f* const was = stage + 16 * (has ? q : 0);
         const V4f o = was[0], d = was[1];
         const V4i w = __builtin_bit_cast(V4i, was[2]), x = __builtin_bit_cast(V4i, was[3]);
-        hitT = d.w;
-        hitId = w.x;
         cur = has ? w.y : kSentinel;
         sp = w.z;
         mine = (uint32_t)w.w;
         batch = (uint32_t)x.x;
+        QuadHit h = {d.w, w.x, x.z, x.w != 0};
         if (MULTI) {
             nodes = (GF4)tab[batch].nodes;
             tris = (GF4)tab[batch].tris;
@@ -652,9 +684,22 @@ __device__ __forceinline__ void trace_steps(const TraceArgs& a, const BatchDesc*
         int* const spare = (int*)(stage + 16 * q) + j;
         auto at_entry = [&](int e) -> int* { return e < R ? column + e * BLOCK : deep + (e - R); };
         bool full = false;
-        while (__ballot(cur != kSentinel) != 0)
-            quad_step<WIDE>(nodes, tris, r, an, j, at_entry, R + kDeep, spare, cur, sp, hitT, hitId, full);
+        while (true) {
+            while (__ballot(cur != kSentinel) != 0)
+                quad_step<WIDE>(nodes, tris, r, an, j, at_entry, R + kDeep, spare, boxes(), cur, sp, h, full);
+            const bool again = WIDE && has && walk_again(boxes(), reach(), r, h);
+            if (__ballot(again) == 0) break;
+            if (again) {
+                h = {__builtin_canonicalizef(
+                         ((const __attribute__((address_space(1))) float*)(rays() + 2 * (size_t)rayidx() + 1))[3]),
+                     -1, 0, true};
+                sp = 0;
+                cur = 0;
+            }
+        }
         if (full) atomicOr(a.errors, (uint32_t)RB_TRACE_ERR_STACK);
+        hitT = h.t;
+        hitId = h.id;
         if (has && j == 0) store();
     }
     end_launch<MULTI>(a);
@@ -955,17 +1000,29 @@ __device__ __forceinline__ void trace_quads(const TraceArgs& a, const BatchDesc*
     const size_t ray = MULTI ? mine - tab[batch].start : second ? mine - n0 : mine;
     const V4f o = rays[2 * ray], d = rays[2 * ray + 1];
     const RayRegs r = ray_regs(o, d);
-    float hitT = __builtin_canonicalizef(d.w);
-    int cur = live && !(mk && mk[ray] == 0) ? 0 : kSentinel, sp = 0, hitId = -1;
+    const float hitT = __builtin_canonicalizef(d.w);
+    const GF4 boxes = MULTI ? (GF4)tab[batch].boxes : (GF4)a.boxes;
+    const float reach = MULTI ? tab[batch].reach : a.reach;
+    int cur = live && !(mk && mk[ray] == 0) ? 0 : kSentinel, sp = 0;
+    QuadHit hit = {hitT, -1, 0, false};
     bool full = false;
-    quad_walk<WIDE>(nodes, tris, r, an, lstack, a.stack_rows, 0, cur, sp, hitT, hitId, full);
+    while (true) {
+        quad_walk<WIDE>(nodes, tris, boxes, r, an, lstack, a.stack_rows, 0, cur, sp, hit, full);
+        const bool again = WIDE && walk_again(boxes, reach, r, hit);
+        if (__ballot(again) == 0) break;
+        if (again) {
+            hit = {hitT, -1, 0, true};
+            sp = 0;
+            cur = 0;
+        }
+    }
     if (full) atomicOr(a.errors, (uint32_t)RB_TRACE_ERR_STACK);
     if (live && j == 0) {
         V2i h;
-        h.x = hitId;
+        h.x = hit.id;
         // a miss reports the caller's tmax, bit for bit
-        h.y = hitId < 0 ? __float_as_int(((const __attribute__((address_space(1))) float*)(rays + 2 * ray + 1))[3])
-                        : __float_as_int(hitT);
+        h.y = hit.id < 0 ? __float_as_int(((const __attribute__((address_space(1))) float*)(rays + 2 * ray + 1))[3])
+                         : __float_as_int(hit.t);
         const GI2 hits = MULTI ? (GI2)tab[batch].hits : second ? (GI2)a.hits2 : (GI2)a.hits;
         hits[ray] = h;
     }
@@ -1165,6 +1222,8 @@ rb_status launch_trace(rb_bvh_t bvh, const rb_ray* rays, uint32_t n, uint32_t fl
     a.leaf_gate = cfg.leaf_gate;
     if (wide) a.nodes = bvh->wnodes;
     a.stack_rows = stack_rows(bvh, wide);
+    a.boxes = bvh->wnodes + 4 * (size_t)bvh->n_wnodes;
+    a.reach = bvh->reach;
     // top-of-tree records in LDS: the speculative walk only
     a.top_nodes = !cfg.speculative ? 0 : cfg.lds_nodes < bvh->n_nodes ? cfg.lds_nodes : bvh->n_nodes;
     const size_t top_bytes = (size_t)a.top_nodes * 64;
@@ -1216,6 +1275,8 @@ rb_status launch_trace_pair(rb_bvh_t bvh, const rb_ray* rays0, uint32_t cap0, co
     std::memset(&a, 0, sizeof(a));
     a.nodes = wide ? bvh->wnodes : bvh->nodes;
     a.stack_rows = stack_rows(bvh, wide);
+    a.boxes = bvh->wnodes + 4 * (size_t)bvh->n_wnodes;
+    a.reach = bvh->reach;
     a.tris = bvh->tris4;
     a.index = bvh->index;
     a.rays = reinterpret_cast<const float4*>(rays0);
@@ -1295,6 +1356,8 @@ static rb_status launch_trace_sets_pass(const BatchSet* b, uint32_t nb, hipStrea
             d.n_dev = b[i].n_dev;
             d.n = b[i].n;
             d.any = b[i].any ? 1u : 0u;
+            d.reach = b[i].bvh->reach;
+            d.boxes = b[i].bvh->wnodes + 4 * (size_t)b[i].bvh->n_wnodes;
             rows = std::max(rows, stack_rows(b[i].bvh, wide));
             total += b[i].n;
         }
