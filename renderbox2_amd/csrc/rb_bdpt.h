@@ -92,6 +92,43 @@ __device__ __forceinline__ uint32_t block_reserve(uint32_t* counter, uint32_t c)
     return base;
 }
 
+// Reserves one slot each of the queues of lengths rays[0] (a) and *paths (q) and
+// one each for b and c of the queue of length rays[1]; the first of b's and c's
+// in *sb.  One pass over the workgroup for all three, and two atomics to two
+// cache lines: the shadow and closest queues' as the halves of a 64-bit word.
+__device__ __forceinline__ void block_reserve3(uint32_t* rays, bool a, bool b, bool c, uint32_t* paths, bool q,
+                                               uint32_t* sa, uint32_t* sb, uint32_t* sq) {
+    // per wave and then per workgroup, packed: a in bits 0..9, b and c in 10..20, q in 21..31
+    __shared__ uint32_t s_sum[kQueueBlock / 64];
+    __shared__ uint32_t s_base[3];
+    const uint32_t lane = __lane_id(), wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    const uint64_t ma = __ballot(a), mb = __ballot(b), mc = __ballot(c), mq = __ballot(q);
+    auto count = [](uint64_t x, uint64_t y, uint64_t z, uint64_t w) -> uint32_t {
+        return (uint32_t)__popcll(x) | (uint32_t)(__popcll(y) + __popcll(z)) << 10 | (uint32_t)__popcll(w) << 21;
+    };
+    if (lane == 0) s_sum[wave] = count(ma, mb, mc, mq);
+    __syncthreads();
+    uint32_t at = count(ma & lt, mb & lt, mc & lt, mq & lt);
+    for (uint32_t w = 0; w < wave; w++) at += s_sum[w];
+    if (threadIdx.x == 0) {
+        uint32_t sum = 0;
+        for (uint32_t w = 0; w < nw; w++) sum += s_sum[w];
+        if (sum) {
+            const unsigned long long r =
+                atomicAdd((unsigned long long*)rays, (unsigned long long)(sum & 1023u) | (unsigned long long)(sum >> 10 & 2047u) << 32);
+            s_base[2] = atomicAdd(paths, sum >> 21);
+            s_base[0] = (uint32_t)r;
+            s_base[1] = (uint32_t)(r >> 32);
+        }
+    }
+    __syncthreads();
+    *sa = s_base[0] + (at & 1023u);
+    *sb = s_base[1] + (at >> 10 & 2047u);
+    *sq = s_base[2] + (at >> 21);
+    __syncthreads();  // s_sum and s_base are reused by the next call
+}
+
 // End of a workgroup-uniform loop over n items.
 __device__ __forceinline__ uint32_t uniform_end(uint32_t n) { return (n + blockDim.x - 1) / blockDim.x * blockDim.x; }
 

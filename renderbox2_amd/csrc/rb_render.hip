@@ -39,17 +39,12 @@ __device__ __forceinline__ uint32_t sample_gid(const TileArgs& T, uint32_t i) {
 
 __global__ void k_ao_spawn(const float4* __restrict__ prim, const int2* __restrict__ hits, uint32_t n, TileArgs T,
                            SceneDev S, uint32_t nao, float radius, RngArg rng_a, float4* __restrict__ rays,
-                           uint8_t* __restrict__ mask, unsigned long long* ray_counter) {
+                           uint8_t* __restrict__ mask) {
     const Rng rng = rng_a.get();
     const uint64_t total = (uint64_t)n * nao;
     for (uint64_t j = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; j < total; j += (uint64_t)gridDim.x * blockDim.x) {
         const uint32_t i = (uint32_t)(j / nao), k = (uint32_t)(j % nao);
         const int2 h = hits[i];
-        if (ray_counter) {  // AO rays traced: nao per primary hit, one atomic per wave
-            const uint64_t m = __ballot(k == 0 && h.x >= 0);
-            if (m && __lane_id() == (uint32_t)__builtin_ctzll(m))
-                atomicAdd(ray_counter, (unsigned long long)__popcll(m) * nao);
-        }
         if (h.x < 0) {
             mask[j] = 0;
             rays[2 * j] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -77,16 +72,32 @@ __global__ void k_ao_spawn(const float4* __restrict__ prim, const int2* __restri
 }
 
 // Per sample: unoccluded AO rays / nao (misses give 0), for the film.
-__global__ void k_ao_resolve(const int2* __restrict__ prim_hits, const int2* __restrict__ ao_hits, uint32_t n,
-                             uint32_t nao, float4* __restrict__ L) {
+// Also counts the rays traced, n and nao per primary hit, when asked to: here,
+// where one thread in nao comes by a primary hit, and once per workgroup.  (One
+// atomic per wave of k_ao_spawn, all to the same word, took 80 us of its 100 for
+// 1 Mi rays.)
+__global__ __launch_bounds__(256) void k_ao_resolve(const int2* __restrict__ prim_hits, const int2* __restrict__ ao_hits,
+                                                    uint32_t n, uint32_t nao, float4* __restrict__ L,
+                                                    unsigned long long* ray_counter) {
+    uint32_t found = 0;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         float c = 0.0f;
         if (prim_hits[i].x >= 0) {
+            found++;
             uint32_t open = 0;
             for (uint32_t k = 0; k < nao; k++) open += ao_hits[(size_t)i * nao + k].x < 0 ? 1u : 0u;
             c = (float)open / (float)nao;
         }
         L[i] = make_float4(c, c, c, 0.f);
+    }
+    if (ray_counter) {
+        __shared__ uint32_t s_found;
+        if (threadIdx.x == 0) s_found = 0;
+        __syncthreads();
+        if (found) atomicAdd(&s_found, found);
+        __syncthreads();
+        if (threadIdx.x == 0)
+            atomicAdd(ray_counter, (unsigned long long)s_found * nao + (blockIdx.x == 0 ? n : 0u));
     }
 }
 
@@ -113,7 +124,9 @@ struct PathBufs {
     float4* cc;      // BDPT: connection contributions, kMaxConn per path
     int* cslot;      // BDPT: connection shadow-ray slots, kMaxConn per path
     uint32_t* q[2];  // path queues
-    uint32_t* cnt;   // [0],[1] queue lengths, [2] shadow rays, [3] closest rays
+    const uint32_t* nin;  // length of the queue that this bounce reads
+    uint32_t* nout;       // of the one it appends to
+    uint32_t* nrays;      // [0] its shadow rays, [1] its closest rays
     float4* ra;      // shadow rays
     int2* ha;
     float4* rbc;     // MIS + bounce rays
@@ -121,6 +134,14 @@ struct PathBufs {
 };
 
 constexpr uint32_t kMaxConn = 8;
+
+// The counts of bounce b are words of their own, cnt + kBounceWords * b: paths
+// queued at word 0, rays at words kRayWords and kRayWords + 1, in another cache
+// line.  A pass clears them all at its start and adds them to the caller's
+// counters at its end; with four words cleared before every bounce, and counted
+// after it, a 128x128 path-traced frame of eight bounces had 18 launches more
+// (4-5 us each).
+constexpr uint32_t kBounceWords = 64, kRayWords = 32;
 
 }  // namespace rb
 
@@ -140,30 +161,36 @@ struct BdArgs {
     RngArg crng;
 };
 
-__global__ void k_reset(uint32_t* c, uint32_t a, uint32_t b, uint32_t d) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        c[a] = 0;
-        c[b] = 0;
-        c[d] = 0;
+// A camera pass's start: its counts cleared; BDPT: the light queue's too, and
+// the camera rays counted for the paired launch.
+__global__ void k_pass_start(uint32_t* cnt, uint32_t words, uint32_t* lights, uint32_t* ncam, uint32_t n) {
+    for (uint32_t i = threadIdx.x; i < words; i += blockDim.x) cnt[i] = 0;
+    if (threadIdx.x == 0 && lights) {
+        *lights = 0;
+        *ncam = n;
     }
 }
 
-__global__ void k_set_u32(uint32_t* p, uint32_t v) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) *p = v;
+// Its end: the rays of all bounces, the n camera rays and the light rays of
+// depth 0 to the caller's counters, and the paths per bounce.
+__global__ void k_pass_count(const uint32_t* cnt, uint32_t bounces, uint32_t n, const uint32_t* lights,
+                             unsigned long long* rays, unsigned long long* paths, unsigned long long* light_paths) {
+    unsigned long long sum = 0;
+    for (uint32_t b = threadIdx.x; b < bounces; b += blockDim.x) {
+        const uint32_t* c = cnt + kBounceWords * b;
+        sum += (unsigned long long)c[kRayWords] + c[kRayWords + 1];
+        if (paths) atomicAdd(paths + b, (unsigned long long)c[0]);
+    }
+    if (threadIdx.x == 0) {
+        sum += n;
+        if (lights) sum += *lights;
+        if (lights && light_paths) atomicAdd(light_paths, (unsigned long long)*lights);
+    }
+    if (rays && sum) atomicAdd(rays, sum);
 }
 
 __global__ void k_add64(unsigned long long* total, unsigned long long v) {
     if (threadIdx.x == 0 && blockIdx.x == 0) atomicAdd(total, v);
-}
-
-__global__ void k_add_count(const uint32_t* c, unsigned long long* total) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) atomicAdd(total, (unsigned long long)*c);
-}
-
-// Adds the rays of this bounce (shadow + closest queues) to the caller's counter.
-__global__ void k_count_rays(const uint32_t* c, unsigned long long* total, unsigned long long extra) {
-    if (threadIdx.x == 0 && blockIdx.x == 0 && total)
-        atomicAdd(total, (unsigned long long)c[2] + (unsigned long long)c[3] + extra);
 }
 
 // Rays asked for by one shaded camera vertex: light sample (A, shadow
@@ -372,13 +399,13 @@ __device__ __forceinline__ bool connect_vertex(const PathBufs& P, uint32_t pid, 
 //          roulette thins, where the queue is short);
 //  MODE 2: contributions only (after the last bounce).
 // Shaded non-emitter vertices are appended to queue qi ^ 1 and their rays to
-// the shadow (cnt[2]) and closest (cnt[3]) queues.
+// the shadow (nrays[0]) and closest (nrays[1]) queues.
 template <bool BD, int MODE>
 __global__ __launch_bounds__(kQueueBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_pt_step(
     PathBufs P, uint32_t qi, uint32_t n0, TileArgs T, SceneDev S, RngArg rng_a, uint32_t max_depth,
     uint32_t rr_start, float rr_prob, float nlights, BdArgs B) {
     const Rng rng = rng_a.get();
-    const uint32_t count = MODE == 0 ? n0 : P.cnt[qi];
+    const uint32_t count = MODE == 0 ? n0 : *P.nin;
     const uint32_t stride = gridDim.x * blockDim.x;
     const uint32_t end = uniform_end(count);  // whole workgroups iterate together
     for (uint32_t q = blockIdx.x * blockDim.x + threadIdx.x; q < end; q += stride) {
@@ -411,9 +438,8 @@ __global__ __launch_bounds__(kQueueBlock) __attribute__((amdgpu_waves_per_eu(4))
         // these): shadow queue = light sample; closest queue = MIS ray, then
         // the bounce ray; the shaded vertices to the next path queue.  BDPT
         // connection rays are appended by k_lvc_connect.
-        const uint32_t sa = block_reserve(&P.cnt[2], R.wantA ? 1u : 0u);
-        const uint32_t sb = block_reserve(&P.cnt[3], (R.wantB ? 1u : 0u) + (R.wantC ? 1u : 0u));
-        const uint32_t sq = block_reserve(&P.cnt[qi ^ 1], shaded ? 1u : 0u);
+        uint32_t sa, sb, sq;
+        block_reserve3(P.nrays, R.wantA, R.wantB, R.wantC, P.nout, shaded, &sa, &sb, &sq);
         const uint32_t sc = sb + (R.wantB ? 1u : 0u);
         if (R.wantA) {
             P.ra[2 * (size_t)sa] = R.ra0;
@@ -450,7 +476,7 @@ __global__ __launch_bounds__(kQueueBlock) void k_lvc_connect(PathBufs P, uint32_
                                                              uint32_t max_depth, BdArgs B) {
     const Rng crng = B.crng.get();
     const uint32_t nconn = B.nconn;
-    const uint32_t total = P.cnt[qi] * nconn;
+    const uint32_t total = *P.nout * nconn;
     const uint32_t stride = gridDim.x * blockDim.x;
     const uint32_t end = uniform_end(total);  // whole workgroups iterate together (block_reserve)
     for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < end; t += stride) {
@@ -536,7 +562,7 @@ __global__ __launch_bounds__(kQueueBlock) void k_lvc_connect(PathBufs P, uint32_
                 P.cc[(size_t)pid * kMaxConn + i] = contrib;
             }
         }
-        const uint32_t si = block_reserve(&P.cnt[2], want ? 1u : 0u);
+        const uint32_t si = block_reserve(P.nrays, want ? 1u : 0u);
         if (valid) P.cslot[(size_t)pid * kMaxConn + i] = want ? (int)si : -1;
         if (want) {
             P.ra[2 * (size_t)si] = r0;
@@ -845,8 +871,7 @@ struct AoJob : RenderJob {
         } else if (state == 1) {
             TileArgs T{cam.width, x0, y0, w, p.spp};
             hipLaunchKernelGGL(k_ao_spawn, dim3(grid_of(na)), dim3(256), 0, s, rays, hits, n, T, scene_of(bvh),
-                               p.ao_samples, p.ao_radius, rng_arg(p.seed, RNG_AO), arays, amask, p.ray_counter);
-            if (p.ray_counter) hipLaunchKernelGGL(k_add64, dim3(1), dim3(64), 0, s, p.ray_counter, (unsigned long long)n);
+                               p.ao_samples, p.ao_radius, rng_arg(p.seed, RNG_AO), arays, amask);
             // AO rays are short (tmax = the AO radius): a wave finishes a
             // claim of rays quickly and the launch's work-counter atomics set
             // the pace; claims of 128 rays halve them (AO frame -19% at 2 Mi
@@ -858,7 +883,8 @@ struct AoJob : RenderJob {
             sets[0] = TraceSet{arays, ahits, (uint32_t)na, nullptr, RB_ANY | kOcclusion | RB_MASKED, amask, ao_cfg};
             *nsets = 1;
         } else {
-            hipLaunchKernelGGL(k_ao_resolve, dim3(grid_of(n)), dim3(256), 0, s, hits, ahits, n, p.ao_samples, Ls);
+            hipLaunchKernelGGL(k_ao_resolve, dim3(grid_of(n)), dim3(256), 0, s, hits, ahits, n, p.ao_samples, Ls,
+                               p.ray_counter);
             hipError_t e = hipGetLastError();
             if (e != hipSuccess) return hip_fail(e, "AO launch");
             if ((st = film(Ls, &cam, x0, y0, w, h, &p, out, s)) != RB_OK) return st;
@@ -925,9 +951,10 @@ struct CameraJob : RenderJob {
     float4* rbcq[2];
     int2* hbcq[2];
     // BDPT light pass
-    LightPath LP;
+    LightPath LP = {};
     float4* lrays = nullptr;
     uint32_t* ncam = nullptr;
+    uint32_t* cnt = nullptr;  // kBounceWords words per bounce
     uint32_t NL = 0, D = 0;
     // progress: 0 start, 1 light pass, 2 camera bounces, 3 last contributions
     int phase = 0;
@@ -961,6 +988,8 @@ struct CameraJob : RenderJob {
         const TileArgs T = tile();
         const SceneDev S = scene_of(bvh);
         if (phase == 0) {
+            hipLaunchKernelGGL(k_pass_start, dim3(1), dim3(256), 0, s, cnt, kBounceWords * (p.max_depth + 1), LP.cnt, ncam,
+                               n);
             if ((st = rb_raygen_camera(&cam, x0, y0, w, h, p.spp, p.seed, 1, (rb_ray*)prim, s)) != RB_OK) return st;
             if (!bd) {
                 sets[0] = TraceSet{prim, phits, n, nullptr, RB_CLOSEST | kCoherent, nullptr, dev().cfg};
@@ -968,8 +997,6 @@ struct CameraJob : RenderJob {
                 phase = 2;
                 return RB_OK;
             }
-            hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(64), 0, s, ncam, n);
-            hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, s, LP.cnt, 0u, 1u, 2u);
             hipLaunchKernelGGL(k_light_emit, dim3(grid_q(NL)), dim3(kQueueBlock), 0, s, NL, S,
                                rng_arg(p.seed, RNG_LIGHT), LP, B.C);
             hipLaunchKernelGGL(k_light_gather, dim3(grid_of(NL)), dim3(256), 0, s, LP, lrays);
@@ -980,9 +1007,6 @@ struct CameraJob : RenderJob {
             return RB_OK;
         }
         if (phase == 1) {  // light depth 0 has been traced: the rest of the light pass, then the camera pass
-            if (p.ray_counter) hipLaunchKernelGGL(k_add_count, dim3(1), dim3(64), 0, s, LP.cnt + 0, p.ray_counter);
-            if (p.light_path_counter)
-                hipLaunchKernelGGL(k_add_count, dim3(1), dim3(64), 0, s, LP.cnt + 0, p.light_path_counter);
             const bool wide = dev().cfg.wide && !dev().cfg.speculative && bvh->wnodes;
             const uint32_t rows = stack_rows(bvh, wide);
             hipLaunchKernelGGL(wide ? k_light_walk<true> : k_light_walk<false>, dim3(walk_blocks(NL)),
@@ -993,9 +1017,6 @@ struct CameraJob : RenderJob {
             phase = 2;
         }
         if (phase == 2) {
-            if (b > 0 && p.ray_counter)  // the previous bounce's rays
-                hipLaunchKernelGGL(k_count_rays, dim3(1), dim3(64), 0, s, (const uint32_t*)P.cnt, p.ray_counter,
-                                   b == 1 ? (unsigned long long)n : 0ull);
             if (b > p.max_depth) {
                 phase = 3;
             } else {
@@ -1007,16 +1028,15 @@ struct CameraJob : RenderJob {
                 P.T = Tq[b & 1];
                 P.Tn = Tq[(b + 1) & 1];
                 P.Tprev = Tq[(b + 1) & 1];  // bounce b - 1's T; this bounce's Tn overwrites it path by path
-                hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, s, P.cnt, qout, 2u, 3u);
+                P.nout = cnt + kBounceWords * b;
+                P.nin = P.nout - (b ? kBounceWords : 0);
+                P.nrays = P.nout + kRayWords;
                 launch_step(s, b == 0 ? 0 : 1, qin);
                 if (bd && B.nconn)
                     hipLaunchKernelGGL(k_lvc_connect, dim3(grid_q((uint64_t)n * B.nconn)), dim3(kQueueBlock), 0, s, P,
                                        qout, T, S, p.max_depth, B);
-                if (p.path_counter)
-                    hipLaunchKernelGGL(k_add_count, dim3(1), dim3(64), 0, s, (const uint32_t*)P.cnt + qout,
-                                       p.path_counter + b);
-                sets[0] = TraceSet{P.ra, P.ha, na, P.cnt + 2, RB_ANY | kOcclusion, nullptr, dev().cfg};
-                sets[1] = TraceSet{P.rbc, P.hbc, 2 * n, P.cnt + 3, RB_CLOSEST, nullptr, dev().cfg};
+                sets[0] = TraceSet{P.ra, P.ha, na, P.nrays, RB_ANY | kOcclusion, nullptr, dev().cfg};
+                sets[1] = TraceSet{P.rbc, P.hbc, 2 * n, P.nrays + 1, RB_CLOSEST, nullptr, dev().cfg};
                 *nsets = 2;
                 b++;
                 return RB_OK;
@@ -1025,7 +1045,11 @@ struct CameraJob : RenderJob {
         // the last bounce's contributions, then the film
         P.phit = hbcq[p.max_depth & 1];
         P.Tprev = Tq[p.max_depth & 1];
+        P.nin = cnt + kBounceWords * p.max_depth;
         launch_step(s, 2, p.max_depth & 1);
+        if (p.ray_counter || p.path_counter || (bd && p.light_path_counter))
+            hipLaunchKernelGGL(k_pass_count, dim3(1), dim3(64), 0, s, (const uint32_t*)cnt, p.max_depth + 1, n,
+                               (const uint32_t*)LP.cnt, p.ray_counter, p.path_counter, p.light_path_counter);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return hip_fail(e, "camera pass launch");
         if ((st = film(P.L, &cam, x0, y0, w, h, &p, out, s)) != RB_OK) return st;
@@ -1144,7 +1168,7 @@ rb_status make_render_job(uint32_t kind, rb_bvh_t bvh, const rb_camera* cam, uin
         P.info = M.get<uint32_t>(n);
         P.q[0] = M.get<uint32_t>(n);
         P.q[1] = M.get<uint32_t>(n);
-        P.cnt = M.get<uint32_t>(4);
+        J->cnt = M.get<uint32_t>(kBounceWords * ((size_t)p->max_depth + 1));
         P.ra = M.get<float4>(2 * (size_t)J->na);
         P.ha = M.get<int2>(J->na);
         for (int k = 0; k < 2; k++) {
@@ -1211,10 +1235,11 @@ rb_status render_bdpt(rb_bvh_t bvh, const rb_camera* cam, uint32_t x0, uint32_t 
 uint64_t render_scratch_bytes(uint32_t kind, uint32_t w, uint32_t h, const rb_render_params* p) {
     const uint64_t n = (uint64_t)w * h * (p->spp ? p->spp : 1);
     const uint64_t slack = 64 * 40;  // per-allocation padding and alignment
+    const uint64_t counts = 4ull * kBounceWords * ((uint64_t)p->max_depth + 1);
     switch (kind) {
         case RB_REQ_AO: return n * 56 + n * (p->ao_samples ? p->ao_samples : 1) * 41 + slack;
-        case RB_REQ_PT: return n * 352 + slack;
-        case RB_REQ_BDPT: return bdpt_scratch_bytes(w, h, p) + slack;
+        case RB_REQ_PT: return n * 352 + counts + slack;
+        case RB_REQ_BDPT: return bdpt_scratch_bytes(w, h, p) + counts + slack;
         case RB_REQ_RAYCAST: return n * 56 + slack;
         default: return slack;
     }
