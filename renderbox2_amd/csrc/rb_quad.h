@@ -277,10 +277,10 @@ __device__ __forceinline__ void quad_step(GF4 nodes, GF4 tris, const RayRegs& ra
 
 // Rows of four entries that a ray's stack can need.
 inline uint32_t stack_rows(rb_bvh_t bvh, bool wide) { return ((wide ? bvh->wide_stack : bvh->stack) + 3) / 4; }
-// LDS of a one-wave block whose quads walk with such stacks.
+// LDS of a wave whose quads walk with such stacks.
 inline size_t quad_lds(uint32_t rows) { return (rows + 1) * 64 * sizeof(int); }
 
-// The walk of one ray per quad of a one-wave block: cur is 0 for a quad whose ray
+// The walk of one ray per quad of the wave: cur is 0 for a quad whose ray
 // starts and kSentinel for one whose ray has ended (or that has none); the
 // result is h (h.id -1: a miss).  Steps are made while more than `until` quads
 // have a ray under way.
@@ -290,7 +290,7 @@ inline size_t quad_lds(uint32_t rows) { return (rows + 1) * 64 * sizeof(int); }
 template <bool WIDE>
 __device__ __forceinline__ void quad_walk(GF4 nodes, GF4 tris, GF4 boxes, const RayRegs& r, bool an, int* stack,
                                           uint32_t rows, uint32_t until, int& cur, int& sp, QuadHit& h, bool& full) {
-    const int lane = threadIdx.x, j = lane & 3;
+    const int lane = (int)__lane_id(), j = lane & 3;
     int* const own = stack + (lane & ~3);
     auto at_entry = [&](int e) -> int* { return own + (e >> 2) * 64 + (e & 3); };
     while ((uint32_t)__popcll(__ballot(cur != kSentinel)) > 4 * until)

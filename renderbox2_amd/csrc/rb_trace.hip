@@ -68,6 +68,7 @@ struct TraceArgs {
     uint32_t threshold;
     uint32_t leaf_gate;  // non-speculative: leave the inner-node phase once <= this many lanes still search
     uint32_t top_nodes;  // node records 0..top_nodes-1 are read from a copy in LDS
+    uint32_t few;         // a launch of at most so many rays, known to the kernel only, gives each a quad
     uint32_t stack_rows;  // a ray's stack needs at most four times as many entries
     const float4* boxes;  // wide records: leaf_boxes
     float reach;
@@ -285,6 +286,81 @@ __device__ __forceinline__ void stage_records(const V4f* rec, uint32_t lane, V4f
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
+// The step loop for launches of few rays: four lanes per ray from the start,
+// sixteen rays per one-wave block, no refill and so no work counters.
+//
+// With a lane per ray such a launch takes as long as its longest ray, whose
+// steps wait for each other: 0.78 us a step, the chain of its instructions
+// (8-10 cycles for each that needs the one before, 80 for each branch that
+// part of the lanes take) and a record from L2 (240).  With a quad per ray a
+// leaf of four triangles is one step and no lane branches: 0.37 us a step.
+// Two children per record leave half of the quad idle, but keep the latency.
+//
+// Measured, a lane per ray throughout -> a quad for each wave's last rays
+// (trace_steps) -> quads throughout (us), rays from surfaces among 1M
+// triangles: 64 rays 109 -> 83 -> 54, 16 Ki 173 -> 132 -> 95, 64 Ki 196 -> 153
+// -> 129, 128 Ki 226 -> 178 -> 186, 256 Ki 281 -> 226 -> 282; first camera rays
+// of 200k triangles: 32 Ki 30 -> 22 -> 9, 128 Ki 50 -> 51 -> 24, 256 Ki 106 ->
+// 97 -> 66; 4099 rays of 20k triangles 107 -> 83 -> 48.  Any hit over the
+// binary records: 128 Ki 322 -> 262 -> 252, 192 Ki 346 -> 286 -> 336.  (Quads
+// are bound by VALU issue from about 100k rays on: a node step is 105
+// instructions for 16 rays, in the other loop 115 for up to 64.)  Rows of the
+// stack for what the tree can need, not for the most any tree may: 4 KB a wave
+// for 1M triangles, so that eight waves fit a SIMD (256 Ki rays 292 -> 282).
+template <bool ANY_T, bool MULTI, bool PAIR, bool WIDE>
+__device__ __forceinline__ void trace_quads(const TraceArgs& a, const BatchDesc* tab, uint32_t nb, uint32_t nrays,
+                                            uint32_t n0, int* lstack, uint32_t group) {
+    const int lane = (int)__lane_id(), j = lane & 3;
+    uint32_t mine = group * 16 + ((uint32_t)lane >> 2);
+    const bool live = mine < nrays;
+    mine = live ? mine : 0u;
+    uint32_t batch = 0;
+    if (MULTI) {  // the last batch starting at or before `mine` (empty batches share their successor's start)
+        uint32_t lo = 0, hi = nb;
+        while (hi - lo > 1) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (tab[mid].start <= mine) lo = mid;
+            else hi = mid;
+        }
+        batch = lo;
+    }
+    const bool second = PAIR && mine >= n0;
+    const bool an = MULTI ? tab[batch].any != 0 : PAIR ? !second && a.any0 != 0 : ANY_T;
+    const GF4 nodes = MULTI ? (GF4)tab[batch].nodes : (GF4)a.nodes;
+    const GF4 tris = MULTI ? (GF4)tab[batch].tris : (GF4)a.tris;
+    const GF4 rays = MULTI ? (GF4)tab[batch].rays : second ? (GF4)a.rays2 : (GF4)a.rays;
+    const uint8_t* const mk = MULTI ? tab[batch].mask : a.mask;
+    const size_t ray = MULTI ? mine - tab[batch].start : second ? mine - n0 : mine;
+    const V4f o = rays[2 * ray], d = rays[2 * ray + 1];
+    const RayRegs r = ray_regs(o, d);
+    const float hitT = __builtin_canonicalizef(d.w);
+    const GF4 boxes = MULTI ? (GF4)tab[batch].boxes : (GF4)a.boxes;
+    const float reach = MULTI ? tab[batch].reach : a.reach;
+    int cur = live && !(mk && mk[ray] == 0) ? 0 : kSentinel, sp = 0;
+    QuadHit hit = {hitT, -1, 0, false};
+    bool full = false;
+    while (true) {
+        quad_walk<WIDE>(nodes, tris, boxes, r, an, lstack, a.stack_rows, 0, cur, sp, hit, full);
+        const bool again = WIDE && walk_again(boxes, reach, r, hit);
+        if (__ballot(again) == 0) break;
+        if (again) {
+            hit = {hitT, -1, 0, true};
+            sp = 0;
+            cur = 0;
+        }
+    }
+    if (full) atomicOr(a.errors, (uint32_t)RB_TRACE_ERR_STACK);
+    if (live && j == 0) {
+        V2i h;
+        h.x = hit.id;
+        // a miss reports the caller's tmax, bit for bit
+        h.y = hit.id < 0 ? __float_as_int(((const __attribute__((address_space(1))) float*)(rays + 2 * ray + 1))[3])
+                         : __float_as_int(hit.t);
+        const GI2 hits = MULTI ? (GI2)tab[batch].hits : second ? (GI2)a.hits2 : (GI2)a.hits;
+        hits[ray] = h;
+    }
+}
+
 // One traversal body for every launch form but the speculative one.
 // PAIR: rays [0, n0) are the first set (a.rays / a.hits; any hit when
 // a.any0), rays [n0, nrays) the closest-hit set (a.rays2 / a.hits2).
@@ -324,8 +400,10 @@ __device__ __forceinline__ void trace_steps(const TraceArgs& a, const BatchDesc*
     // are the most that keep 20 waves on a CU, which 16 did not: 671 us on 2
     // Mi diffuse rays against 684 with 12 and 720 with 16)
     constexpr int R = S - 1;
-    __shared__ int lstack[R * BLOCK];
-    __shared__ V4f staged[4 * BLOCK];
+    constexpr int kLds = (16 + R) * BLOCK;  // words
+    __shared__ V4f staged[kLds / 4];
+    int* const lds = (int*)staged;
+    int* const lstack = lds + 16 * BLOCK;
     int spill[kMaxStack - 1 - R];
     constexpr int kDeep = 48;  // a quad's entries past those, once a wave has given its last rays a quad each
     const int tid = threadIdx.x;
@@ -335,6 +413,12 @@ __device__ __forceinline__ void trace_steps(const TraceArgs& a, const BatchDesc*
     const V4f* const mine_staged = stage + 64 * (lane & 3) + 4 * (lane >> 2);
 
     const uint32_t nrays = __builtin_amdgcn_readfirstlane(n_rays);
+    if (!COUNT && (MULTI || PAIR) && nrays <= a.few) {
+        const uint32_t wave = blockIdx.x * (BLOCK / 64) + (uint32_t)__builtin_amdgcn_readfirstlane(tid >> 6);
+        for (uint32_t g = wave; g * 16 < nrays; g += gridDim.x * (BLOCK / 64))
+            trace_quads<ANY_T, MULTI, PAIR, WIDE>(a, tab, nb, nrays, n0, lds + (tid >> 6) * (kLds / (BLOCK / 64)), g);
+        return;
+    }
     RayPool pool;
     pool.init();
     // cur: the ray's next step -- an inner record (>= 0), a leaf's remaining
@@ -954,83 +1038,6 @@ __device__ __forceinline__ void trace_spec(const TraceArgs& a, const BatchDesc* 
 #undef RB_PUSH
 #undef RB_POP
 
-// The step loop for launches of few rays: four lanes per ray from the start,
-// sixteen rays per one-wave block, no refill and so no work counters.
-//
-// With a lane per ray such a launch takes as long as its longest ray, whose
-// steps wait for each other: 0.78 us a step, the chain of its instructions
-// (8-10 cycles for each that needs the one before, 80 for each branch that
-// part of the lanes take) and a record from L2 (240).  With a quad per ray a
-// leaf of four triangles is one step and no lane branches: 0.37 us a step.
-// Two children per record leave half of the quad idle, but keep the latency.
-//
-// Measured, a lane per ray throughout -> a quad for each wave's last rays
-// (trace_steps) -> quads throughout (us), rays from surfaces among 1M
-// triangles: 64 rays 109 -> 83 -> 54, 16 Ki 173 -> 132 -> 95, 64 Ki 196 -> 153
-// -> 129, 128 Ki 226 -> 178 -> 186, 256 Ki 281 -> 226 -> 282; first camera rays
-// of 200k triangles: 32 Ki 30 -> 22 -> 9, 128 Ki 50 -> 51 -> 24, 256 Ki 106 ->
-// 97 -> 66; 4099 rays of 20k triangles 107 -> 83 -> 48.  Any hit over the
-// binary records: 128 Ki 322 -> 262 -> 252, 192 Ki 346 -> 286 -> 336.  (Quads
-// are bound by VALU issue from about 100k rays on: a node step is 105
-// instructions for 16 rays, in the other loop 115 for up to 64.)  Rows of the
-// stack for what the tree can need, not for the most any tree may: 4 KB a wave
-// for 1M triangles, so that eight waves fit a SIMD (256 Ki rays 292 -> 282).
-template <bool ANY_T, bool MULTI, bool PAIR, bool WIDE>
-__device__ __forceinline__ void trace_quads(const TraceArgs& a, const BatchDesc* tab, uint32_t nb, uint32_t nrays,
-                                            uint32_t n0 = 0) {
-    extern __shared__ int lstack[];
-    const int lane = threadIdx.x, j = lane & 3;
-    if (blockIdx.x * 16 >= nrays) return;
-    uint32_t mine = blockIdx.x * 16 + ((uint32_t)lane >> 2);
-    const bool live = mine < nrays;
-    mine = live ? mine : 0u;
-    uint32_t batch = 0;
-    if (MULTI) {  // the last batch starting at or before `mine` (empty batches share their successor's start)
-        uint32_t lo = 0, hi = nb;
-        while (hi - lo > 1) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (tab[mid].start <= mine) lo = mid;
-            else hi = mid;
-        }
-        batch = lo;
-    }
-    const bool second = PAIR && mine >= n0;
-    const bool an = MULTI ? tab[batch].any != 0 : PAIR ? !second && a.any0 != 0 : ANY_T;
-    const GF4 nodes = MULTI ? (GF4)tab[batch].nodes : (GF4)a.nodes;
-    const GF4 tris = MULTI ? (GF4)tab[batch].tris : (GF4)a.tris;
-    const GF4 rays = MULTI ? (GF4)tab[batch].rays : second ? (GF4)a.rays2 : (GF4)a.rays;
-    const uint8_t* const mk = MULTI ? tab[batch].mask : a.mask;
-    const size_t ray = MULTI ? mine - tab[batch].start : second ? mine - n0 : mine;
-    const V4f o = rays[2 * ray], d = rays[2 * ray + 1];
-    const RayRegs r = ray_regs(o, d);
-    const float hitT = __builtin_canonicalizef(d.w);
-    const GF4 boxes = MULTI ? (GF4)tab[batch].boxes : (GF4)a.boxes;
-    const float reach = MULTI ? tab[batch].reach : a.reach;
-    int cur = live && !(mk && mk[ray] == 0) ? 0 : kSentinel, sp = 0;
-    QuadHit hit = {hitT, -1, 0, false};
-    bool full = false;
-    while (true) {
-        quad_walk<WIDE>(nodes, tris, boxes, r, an, lstack, a.stack_rows, 0, cur, sp, hit, full);
-        const bool again = WIDE && walk_again(boxes, reach, r, hit);
-        if (__ballot(again) == 0) break;
-        if (again) {
-            hit = {hitT, -1, 0, true};
-            sp = 0;
-            cur = 0;
-        }
-    }
-    if (full) atomicOr(a.errors, (uint32_t)RB_TRACE_ERR_STACK);
-    if (live && j == 0) {
-        V2i h;
-        h.x = hit.id;
-        // a miss reports the caller's tmax, bit for bit
-        h.y = hit.id < 0 ? __float_as_int(((const __attribute__((address_space(1))) float*)(rays + 2 * ray + 1))[3])
-                         : __float_as_int(hit.t);
-        const GI2 hits = MULTI ? (GI2)tab[batch].hits : second ? (GI2)a.hits2 : (GI2)a.hits;
-        hits[ray] = h;
-    }
-}
-
 template <bool ANY, bool COUNT, int S, int BLOCK, bool SPEC>
 __global__ __launch_bounds__(BLOCK) void k_trace(TraceArgs a) {
     const uint32_t nrays = a.n_dev ? __builtin_nontemporal_load(a.n_dev) : a.n;
@@ -1089,14 +1096,17 @@ __global__ __launch_bounds__(BLOCK) void k_trace_batch(TraceArgs a, BatchTable t
 template <bool ANY, bool WIDE>
 __global__ __launch_bounds__(64) void k_trace_few(TraceArgs a) {
     const uint32_t nrays = a.n_dev ? __builtin_nontemporal_load(a.n_dev) : a.n;
-    trace_quads<ANY, false, false, WIDE>(a, nullptr, 0, nrays);
+    extern __shared__ int lstack[];
+    if (blockIdx.x * 16 < nrays) trace_quads<ANY, false, false, WIDE>(a, nullptr, 0, nrays, 0, lstack, blockIdx.x);
 }
 
 template <bool WIDE>
 __global__ __launch_bounds__(64) void k_trace_few_pair(TraceArgs a) {
     const uint32_t n0 = __builtin_nontemporal_load(a.n_dev);
     const uint32_t n1 = __builtin_nontemporal_load(a.n_dev2);
-    trace_quads<true, false, true, WIDE>(a, nullptr, 0, n0 + n1, n0);
+    extern __shared__ int lstack[];
+    if (blockIdx.x * 16 < n0 + n1)
+        trace_quads<true, false, true, WIDE>(a, nullptr, 0, n0 + n1, n0, lstack, blockIdx.x);
 }
 
 template <bool WIDE>
@@ -1104,7 +1114,9 @@ __global__ __launch_bounds__(64) void k_trace_few_batch(TraceArgs a, BatchTable 
     __shared__ BatchDesc tab[kMaxBatch];
     __shared__ uint32_t s_total;
     batch_table(t, tab, &s_total);
-    trace_quads<false, true, false, WIDE>(a, tab, t.nb, s_total);
+    extern __shared__ int lstack[];
+    if (blockIdx.x * 16 < s_total)
+        trace_quads<false, true, false, WIDE>(a, tab, t.nb, s_total, 0, lstack, blockIdx.x);
 }
 
 // ---------------------------------------------------------------- launch --
@@ -1162,13 +1174,22 @@ static bool wide_walk(const rb_trace_config& cfg, rb_bvh_t bvh, uint32_t flags) 
     return cfg.wide && !cfg.speculative && bvh->wnodes && (!(flags & RB_ANY) || (flags & kOcclusion));
 }
 
-// Whether a launch of at most n rays takes trace_quads: up to where both loops
-// are level on rays that scatter (the figures are at trace_quads), over the
-// wide and the binary records alike; three times as many camera rays, whose
-// quads share their lines and branches (384 Ki: 148 us in trace_steps, 115 in
-// trace_quads; 512 Ki: 171 and 161).
+// Launches of up to this many rays per CU take trace_quads: where both loops are
+// level on rays that scatter (the figures are at trace_quads), over the wide and
+// the binary records alike.  Three times as many camera rays, whose quads share
+// their lines and branches (384 Ki: 148 us in trace_steps, 115 in trace_quads;
+// 512 Ki: 171 and 161).
+constexpr uint32_t kFewPerCu = 512, kFewCoherentPerCu = 1536;
 static bool few_rays(const rb_trace_config& cfg, uint64_t n, bool coherent = false) {
-    return !cfg.speculative && n <= (uint64_t)dev().num_cus * (coherent ? 1536 : 512);
+    return !cfg.speculative && n <= (uint64_t)dev().num_cus * (coherent ? kFewCoherentPerCu : kFewPerCu);
+}
+// The same for a launch with a larger bound whose ray counts only the kernel
+// knows, where a wave's LDS holds the quads' stacks.  (The later bounces of a
+// path-traced frame, whose bound is two rays per path: 24 served tiles 11.1 ->
+// 9.8 ms, a 512x512x4 BDPT frame 6.79 -> 6.74, a 1024x1024x8 path-traced one 17.99
+// -> 17.88.)
+static uint32_t few_known_late(const rb_trace_config& cfg, uint32_t rows) {
+    return rows + 1 <= cfg.lds_stack + 15 ? dev().num_cus * kFewPerCu : 0;
 }
 static uint32_t few_blocks(uint64_t n) { return (uint32_t)((n + 15) / 16); }
 
@@ -1294,6 +1315,7 @@ rb_status launch_trace_pair(rb_bvh_t bvh, const rb_ray* rays0, uint32_t cap0, co
     a.chunk = cfg.chunk;
     a.threshold = cfg.fetch_threshold;
     a.leaf_gate = cfg.leaf_gate;
+    a.few = few_known_late(cfg, a.stack_rows);
     const size_t lds = trace_lds(cfg);
     if (lds > dev().lds_per_block)
         return fail(RB_ERR_INVALID, "trace config needs %zu bytes of LDS per block; the device allows %zu", lds,
@@ -1374,6 +1396,7 @@ static rb_status launch_trace_sets_pass(const BatchSet* b, uint32_t nb, hipStrea
         a.chunk = cfg.chunk;
         a.threshold = cfg.fetch_threshold;
         a.leaf_gate = cfg.leaf_gate;
+        a.few = few_known_late(cfg, a.stack_rows);
         if (few_rays(cfg, total)) {
             BatchKernel q = wide ? k_trace_few_batch<true> : k_trace_few_batch<false>;
             hipLaunchKernelGGL(q, dim3(few_blocks(total)), dim3(64), quad_lds(a.stack_rows), stream, a, t);

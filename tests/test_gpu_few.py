@@ -81,3 +81,26 @@ def test_the_loops_give_the_same_hits(gpu, orc, scene, wide, any_hit, masked, n,
     assert np.array_equal(few["id"][ok], oid) and np.array_equal(few["t"][ok].view(np.uint32), ot.view(np.uint32))
     if n > 1000 and not masked:
         assert (oid >= 0).sum() > n // 4
+
+
+@pytest.mark.parametrize("kind", ["pt", "bdpt"])
+@pytest.mark.parametrize("lds_stack,block,wide", [(16, 256, 1), (8, 64, 1), (16, 512, 0)])
+def test_frames_equal_their_tiles(gpu, kind, lds_stack, block, wide):
+    """A frame's bounces, whose launches learn in the kernel that they have few
+    rays, against those of its tiles, whose launches are known to have few."""
+    s = gpu.scenes.pt_room(spheres_hi=4, spheres_lo=10)
+    tr = gpu.CudaTracer(gpu.scenes.build(s), s)
+    cam = gpu.scenes.pt_camera(256, 192)
+    cfg = gpu.get_trace_config()
+    gpu.set_trace_config(**{**cfg, "lds_stack": lds_stack, "block": block, "wide": wide})
+    try:
+        kw = dict(light_paths=500, light_max_depth=3, connections=1) if kind == "bdpt" else {}
+        r = gpu.SamplerRenderer(tr, cam, kind, spp=1, seed=4, max_depth=6, rr_start=1, rr_prob=0.5, **kw)
+        frame = r.render()
+        assert np.isfinite(frame).all() and frame.max() > 0
+        for y in range(0, 192, 48):
+            for x in range(0, 256, 128):
+                tile = r.render((x, y, 128, 48))
+                assert np.array_equal(tile.view(np.uint32), frame[y:y + 48, x:x + 128].view(np.uint32))
+    finally:
+        gpu.set_trace_config(**cfg)
