@@ -541,16 +541,18 @@ def main():
     ids, _, gcnt = tracer.trace_counts(d_diff.download(np.float32, n * 8).reshape(n, 8))
     gpu_bpr = float((40 + 64 * gcnt[:, 0] + 48 * gcnt[:, 1] + 16 * gcnt[:, 2] + 4 * (ids >= 0)).mean())
     # bytes the timed kernel itself reads and writes per ray: the ray (32),
-    # the hit (8), each visited record (64, binary or wide), each tested
-    # triangle (48) and the hit's index entry (4)
+    # the hit (8), each visited record (64, binary or wide) and each tested
+    # triangle (64 with its id; the speculative walk: 48, and 4 for the hit's
+    # index entry)
     wide = bool(cfg["wide"]) and not cfg["speculative"]
     if wide:
         wids, _, wcnt = tracer.trace_counts(d_diff.download(np.float32, n * 8).reshape(n, 8), wide=True)
-        kernel_bpr = float((40 + 64 * wcnt[:, 0] + 48 * wcnt[:, 1] + 4 * (wids >= 0)).mean())
+        kernel_bpr = float((40 + 64 * wcnt[:, 0] + 64 * wcnt[:, 1]).mean())
         wide_records = float(wcnt[:, 0].mean())
         del wids, wcnt
     else:
-        kernel_bpr = float((40 + 64 * gcnt[:, 0] + 48 * gcnt[:, 1] + 4 * (ids >= 0)).mean())
+        spec = bool(cfg["speculative"])
+        kernel_bpr = float((40 + 64 * gcnt[:, 0] + (48 if spec else 64) * gcnt[:, 1] + (4 * (ids >= 0) if spec else 0)).mean())
         wide_records = None
 
     # CPU baseline (the oracle's restatement of the reference traversal) and

@@ -652,9 +652,9 @@ __global__ void k_film(const float4* __restrict__ L, uint32_t npix, uint32_t spp
 // nothing is stored; sums run in a fixed order (neighbour row, column,
 // sample), so images are reproducible.  A workgroup draws the positions of a
 // row of its pixels' neighbours once, into LDS, and adds them before the next
-// row; with a draw per pixel and neighbour 401x299 pixels of 5 samples under a
+// row; with a draw per pixel and neighbour 401x299 pixels of 4 samples under a
 // Gaussian of radius 2 took 88 us, now 75: the window tests and weights of the
-// 245 samples a pixel looks at.  (32x8 pixels with several rows at a time: 85.)
+// 196 samples a pixel looks at.  (32x8 pixels with several rows at a time: 85.)
 struct FilmFilter {
     float xw, yw, inv_xw, inv_yw;
     float table[256];  // [y * 16 + x]
