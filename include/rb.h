@@ -301,7 +301,8 @@ typedef struct rb_bvh_dev {
     const uint32_t* index;  /* uint32[n_refs]: original triangle id per reference */
     uint32_t n_nodes, n_refs;
     uint32_t* errors;       /* device word for RB_TRACE_ERR_* flags (rb_trace_errors); may be NULL */
-    const void* wnodes;     /* float4[4 * n_wnodes]: wide (4-child) records, which rb_trace_one
+    const void* wnodes;     /* float4[4 * n_wnodes]: wide (4-child) records, then float4[2 * n_refs]:
+                               the box of each reference's leaf, which rb_trace_one
                                walks for closest hits (the same (id, t)); NULL: the binary
                                records only.  Set when rb_trace_config.wide is on */
     uint32_t n_wnodes;
@@ -383,7 +384,9 @@ rb_status rb_trace_batch(const rb_batch_desc* batches, uint32_t nb, void* stream
 
 /* Traversal tuning: the knobs the autotuner searches (the reference
  * hard-codes STACK_SIZE 64 / DYNAMIC_FETCH_THRESHOLD 20 / 720 warps of
- * (32,4), kepler_dynamic_fetch.h:62-63 and cudatracer.cu:170-171). */
+ * (32,4), kepler_dynamic_fetch.h:62-63 and cudatracer.cu:170-171).  A
+ * non-speculative launch of up to 512 rays per CU gives each ray four lanes
+ * and its block, grid and claims follow from the ray count alone. */
 typedef struct rb_trace_config {
     uint32_t block;          /* threads per block: 64, 128, 256, 512, 1024 */
     uint32_t lds_stack;      /* stack entries per lane kept in LDS: 8..24 (8..16 at
