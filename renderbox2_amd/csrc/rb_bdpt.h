@@ -279,7 +279,7 @@ __device__ __forceinline__ bool light_vertex(const SceneDev& S, const Rng& rng, 
 template <bool WIDE>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_light_walk(
     SceneDev S, RngArg rng_a, LightPath P, LvcBufs C, const float4* nodes, const float4* tris,
-    const float4* boxes, float reach, uint32_t rows, uint32_t* errors, unsigned long long* ray_counter,
+    const float4* boxes, uint32_t rows, uint32_t* errors, unsigned long long* ray_counter,
     unsigned long long* depth_counter) {
     constexpr uint32_t kWait = 12;  // quads that wait for their vertex before the wave shades
     extern __shared__ int lstack[];
@@ -297,7 +297,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_
     while (true) {
         if (cur == kSentinel) {
             int2 h = make_int2(hit.id, __float_as_int(hit.t));
-            const bool again = WIDE && walk_again((GF4)boxes, reach, r, hit);
+            const bool again = WIDE && walk_again((GF4)boxes, r, hit);
             if (again) {
                 hit = {dd.w, -1, 0, true};
                 cur = 0;

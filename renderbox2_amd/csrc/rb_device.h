@@ -211,10 +211,9 @@ struct rb_bvh_s {
     float4* nodes = nullptr;    // 4 float4 per inner node (MI355X layout)
     float4* wnodes = nullptr;   // 4 float4 per wide (4-child) record (export_walk), then 2 per reference (leaf_boxes)
     uint32_t n_wnodes = 0;
-    float reach = 0;            // leaf_boxes
     uint32_t stack = 0, wide_stack = 0;  // most stack entries a ray of the binary / wide walk can need
     float4* tris = nullptr;     // 3 float4 Woop rows per triangle reference
-    float4* tris4 = nullptr;    // the same in 64 bytes each: 3 Woop rows, then id|edge band|0|0; one more, all zero
+    float4* tris4 = nullptr;    // the same in 64 bytes each: 3 Woop rows, then id|0|0|0; one more, all zero
     uint32_t* index = nullptr;  // original triangle id per reference
     uint32_t n_nodes = 0, n_refs = 0;
     // shading data (Scene::gpu_prepare, src/core/scene.cpp:166-301)

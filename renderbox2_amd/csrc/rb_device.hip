@@ -329,32 +329,12 @@ rb_status rb_event_synchronize(void* ev) {
 
 // ------------------------------------------------------------- upload --
 
-// Hits whose smallest barycentric coordinate is below this are near an edge of
-// the triangle with these Woop rows: within 2^-20 of the reach, which is more
-// than the roundings of a slab test (16 units of 2^-24 of half the reach, from
-// two planes' products and the origin's) and of a hit's coordinates (12) move
-// a box and the hit by.
-static float edge_band(const float* woop, float reach) {
-    float g = 0.0f;  // of the coordinates, the steepest one's slope
-    float sum = 0.0f, u = 0.0f, v = 0.0f;
-    for (int a = 0; a < 3; a++) {
-        u += woop[4 + a] * woop[4 + a];
-        v += woop[8 + a] * woop[8 + a];
-        const float w = woop[4 + a] + woop[8 + a];
-        sum += w * w;
-    }
-    g = std::sqrt(std::max(u, std::max(v, sum)));
-    const float band = g * reach * 0x1p-20f;
-    return band < 2.0f ? band : 2.0f;  // (a coordinate is at most 1: every hit)
-}
-
 rb_status rb_bvh_upload(rb_host_bvh_t hb, rb_scene_t scene, rb_bvh_t* out) {
     if (!hb || !out) return fail(RB_ERR_INVALID, "NULL argument");
     RB_ENSURE();
     Mi355Layout L;
     std::vector<uint32_t> wide;
     uint32_t stack = 0, wide_stack = 0, n_wide = 0;
-    float reach = 0.0f;
     try {
         rb_status st = export_mi355x(*hb->b, L);
         if (st != RB_OK) return st;
@@ -376,7 +356,7 @@ rb_status rb_bvh_upload(rb_host_bvh_t hb, rb_scene_t scene, rb_bvh_t* out) {
         n_wide = (uint32_t)(wide.size() / kWideWords);
         if (n_wide) {
             std::vector<float> box;
-            leaf_boxes(L.nodes, (uint32_t)L.index.size(), box, &reach);
+            leaf_boxes(L.nodes, (uint32_t)L.index.size(), box);
             const size_t at = wide.size();
             wide.resize(at + box.size());
             std::memcpy(&wide[at], box.data(), 4 * box.size());
@@ -406,7 +386,6 @@ rb_status rb_bvh_upload(rb_host_bvh_t hb, rb_scene_t scene, rb_bvh_t* out) {
     B->wide_stack = wide_stack;
     if ((st = up((void**)&B->nodes, L.nodes.data(), L.nodes.size() * 4)) != RB_OK) { cleanup(); return st; }
     B->n_wnodes = n_wide;
-    B->reach = reach;
     if (!wide.empty() && (st = up((void**)&B->wnodes, wide.data(), wide.size() * 4)) != RB_OK) { cleanup(); return st; }
     // after the references the zero triangle of the wide records' empty
     // slots (no ray hits it)
@@ -418,8 +397,6 @@ rb_status rb_bvh_upload(rb_host_bvh_t hb, rb_scene_t scene, rb_bvh_t* out) {
         for (uint32_t r = 0; r <= B->n_refs; r++) {
             std::memcpy(&t4[16 * (size_t)r], &L.tris[12 * (size_t)r], 48);
             t4[16 * (size_t)r + 12] = L.index[r];
-            const float band = r < B->n_refs ? edge_band(&L.tris[12 * (size_t)r], reach) : 0.0f;
-            std::memcpy(&t4[16 * (size_t)r + 13], &band, 4);
         }
         if ((st = up((void**)&B->tris4, t4.data(), t4.size() * 4)) != RB_OK) { cleanup(); return st; }
     }

@@ -209,13 +209,19 @@ rb_status export_walk(const std::vector<uint32_t>& bin, uint32_t n_refs, std::ve
 // larger, so that a ray through the crack between two triangles, which passes
 // no leaf's box here, can meet a triangle there (10 of 128 M rays in
 // tessellated rooms, one in six of rays aimed at the edges of a wall's
-// triangles); a hit near the edge of its triangle counts once its leaf's box
-// passes, and a ray whose hit does not count is walked again with that test on
-// every hit.  (Cost: 605 -> 620 us for 2 Mi diffuse rays, the reference of the
-// hit and its distance from the edge kept with it and 1 ray in 80 tested;
-// testing every hit as it is found reads two more rows for each.)  *reach: rays from within this distance of the world's origin
-// need the test only near an edge (edge_band), others always.
-void leaf_boxes(const std::vector<uint32_t>& bin, uint32_t n_refs, std::vector<float>& box, float* reach);
+// triangles).  So the box of a ray's hit is tested when the ray ends, and a ray
+// whose hit does not count is walked again with that test on every hit.
+// Every ray that hits is tested, wherever on its triangle: a slab test's
+// rounding moves its point along the ray, across a triangle that the ray grazes
+// by as much more as the ray lies in its plane, and a box cut by a spatial split
+// ends far from its triangle's edges.  (Tested only near an edge, 13,000 to
+// 20,000 of 400,000 rays that graze a wall hit what they pass.  The test of all,
+// against that: 632 -> 643 us for 2 Mi diffuse rays at 1M triangles, 799 -> 809
+// for a 128x128 path-traced tile; testing every hit as it is found reads two
+// more rows for each, and with the box loaded as a quad finds its hit, instead
+// of at the end, 2 Mi diffuse rays took 644 us and ambient occlusion 512x512
+// 354 against 346.)
+void leaf_boxes(const std::vector<uint32_t>& bin, uint32_t n_refs, std::vector<float>& box);
 // Depth of the deepest inner record of an MI355X node array (root = 0);
 // UINT32_MAX when a link leaves the array or the links form a cycle.  A
 // traversal holds at most depth + 1 stack entries (the sentinel, then one

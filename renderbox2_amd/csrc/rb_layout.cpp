@@ -625,7 +625,7 @@ rb_status export_walk(const std::vector<uint32_t>& bin, uint32_t n_refs, std::ve
     return fail(RB_ERR_UNSUPPORTED, "the tree is too deep for the wide walk's stack");
 }
 
-void leaf_boxes(const std::vector<uint32_t>& bin, uint32_t n_refs, std::vector<float>& box, float* reach) {
+void leaf_boxes(const std::vector<uint32_t>& bin, uint32_t n_refs, std::vector<float>& box) {
     box.assign(8 * ((size_t)n_refs + 1), 0.0f);
     auto set = [&](int32_t link, const float lo[3], const float hi[3]) {
         const uint32_t l = ~(uint32_t)link, first = l >> 5, cnt = l & 31u;
@@ -635,16 +635,11 @@ void leaf_boxes(const std::vector<uint32_t>& bin, uint32_t n_refs, std::vector<f
                 box[8 * (size_t)r + 2 * a + 1] = hi[a];
             }
     };
-    float far = 0.0f;
     for (size_t r = 0; r < bin.size() / 16; r++)
         for (int c = 0; c < 2; c++) {
             const WalkChild k = walk_child(&bin[r * 16], c);
-            if (empty_leaf(k.link)) continue;
-            if (r == 0)
-                for (int a = 0; a < 3; a++) far = std::max(far, std::max(std::fabs(k.lo[a]), std::fabs(k.hi[a])));
-            if (k.link < 0) set(k.link, k.lo, k.hi);
+            if (k.link < 0 && !empty_leaf(k.link)) set(k.link, k.lo, k.hi);
         }
-    *reach = 2.0f * far;
     std::vector<uint32_t> wide;
     if (!wide_fits_stack(layout_depth(bin)) || export_wide(bin, wide) != RB_OK) {
         set_error("");

@@ -120,7 +120,7 @@ __device__ __forceinline__ bool leaf_box_passes(GF4 boxes, uint32_t ref, const R
 }
 
 // What a walk over wide records has found: the hit, and the reference it lies
-// on, complemented when it lies near an edge of its triangle.
+// on.
 struct QuadHit {
     float t;
     int id, ref;
@@ -186,8 +186,7 @@ __device__ __forceinline__ void quad_step(GF4 nodes, GF4 tris, const RayRegs& ra
             int tb = take ? __float_as_int(t) : 0, ib = take ? id : 0;
             int rb = 0;
             if (WIDE) {
-                const float edge = vmin3_(u, v, 1.0f - uv);
-                rb = take ? (edge < r3.y ? ~(int)rec : (int)rec) : 0;
+                rb = take ? (int)rec : 0;
                 rb |= quad<kQuadXor1>(rb);
                 rb |= quad<kQuadXor2>(rb);
             }
@@ -298,13 +297,10 @@ __device__ __forceinline__ void quad_walk(GF4 nodes, GF4 tris, GF4 boxes, const 
                         full);
 }
 
-// Whether an ended walk over wide records has to be made again, strictly: its
-// hit lies near an edge, or its ray started out of reach, and the leaf's box
-// does not pass.
-__device__ __forceinline__ bool walk_again(GF4 boxes, float reach, const RayRegs& r, const QuadHit& h) {
-    if (h.id < 0 || h.strict) return false;
-    const bool far = !(vmax3_(fabsf(r.ox), fabsf(r.oy), fabsf(r.oz)) <= reach);
-    return (h.ref < 0 || far) && !leaf_box_passes(boxes, (uint32_t)(h.ref < 0 ? ~h.ref : h.ref), r);
+// Whether an ended walk over wide records has to be made again, strictly: the
+// box of its hit's leaf does not pass.
+__device__ __forceinline__ bool walk_again(GF4 boxes, const RayRegs& r, const QuadHit& h) {
+    return h.id >= 0 && !h.strict && !leaf_box_passes(boxes, (uint32_t)h.ref, r);
 }
 
 }  // namespace rb

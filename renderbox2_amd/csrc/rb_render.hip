@@ -1059,7 +1059,7 @@ struct CameraJob : RenderJob {
             hipLaunchKernelGGL(wide ? k_light_walk<true> : k_light_walk<false>, dim3(walk_blocks(NL)),
                                dim3(64), quad_lds(rows), s, S, rng_arg(p.seed, RNG_LIGHT), LP, B.C,
                                wide ? bvh->wnodes : bvh->nodes, bvh->tris4,
-                               bvh->wnodes + 4 * (size_t)bvh->n_wnodes, bvh->reach, rows, dev().errors, p.ray_counter,
+                               bvh->wnodes + 4 * (size_t)bvh->n_wnodes, rows, dev().errors, p.ray_counter,
                                p.light_path_counter);
             phase = 2;
         }

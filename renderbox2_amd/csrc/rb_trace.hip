@@ -71,7 +71,6 @@ struct TraceArgs {
     uint32_t few;         // a launch of at most so many rays, known to the kernel only, gives each a quad
     uint32_t stack_rows;  // a ray's stack needs at most four times as many entries
     const float4* boxes;  // wide records: leaf_boxes
-    float reach;
 };
 
 constexpr uint32_t kMaxBatch = 64;
@@ -87,7 +86,6 @@ struct BatchDesc {
     uint32_t n;             // ray count, or the bound of *n_dev
     uint32_t start;         // first global ray index of the batch (set by the kernel)
     uint32_t any;           // 1: terminate on the first hit
-    float reach;
     const float4* boxes;    // wide records: leaf_boxes
 };
 
@@ -335,13 +333,12 @@ __device__ __forceinline__ void trace_quads(const TraceArgs& a, const BatchDesc*
     const RayRegs r = ray_regs(o, d);
     const float hitT = __builtin_canonicalizef(d.w);
     const GF4 boxes = MULTI ? (GF4)tab[batch].boxes : (GF4)a.boxes;
-    const float reach = MULTI ? tab[batch].reach : a.reach;
     int cur = live && !(mk && mk[ray] == 0) ? 0 : kSentinel, sp = 0;
     QuadHit hit = {hitT, -1, 0, false};
     bool full = false;
     while (true) {
         quad_walk<WIDE>(nodes, tris, boxes, r, an, lstack, a.stack_rows, 0, cur, sp, hit, full);
-        const bool again = WIDE && walk_again(boxes, reach, r, hit);
+        const bool again = WIDE && walk_again(boxes, r, hit);
         if (__ballot(again) == 0) break;
         if (again) {
             hit = {hitT, -1, 0, true};
@@ -449,7 +446,6 @@ __device__ __forceinline__ void trace_steps(const TraceArgs& a, const BatchDesc*
     auto rayidx = [&]() -> uint32_t { return MULTI ? mine - tab[batch].start : second() ? mine - n0 : mine; };
     auto rays = [&]() -> GF4 { return MULTI ? (GF4)tab[batch].rays : second() ? (GF4)a.rays2 : (GF4)a.rays; };
     auto boxes = [&]() -> GF4 { return MULTI ? (GF4)tab[batch].boxes : (GF4)a.boxes; };
-    auto reach = [&]() -> float { return MULTI ? tab[batch].reach : a.reach; };
     auto hits = [&]() -> GI2 { return MULTI ? (GI2)tab[batch].hits : second() ? (GI2)a.hits2 : (GI2)a.hits; };
 
     // The upload refuses trees deep enough to fill the stack, so the last
@@ -506,12 +502,8 @@ __device__ __forceinline__ void trace_steps(const TraceArgs& a, const BatchDesc*
             if (WIDE) {
                 // hits that may not count (leaf_boxes): those rays again
                 bool again = false;
-                if (cur == kSentinel && live && hitId >= 0 && !strict) {
-                    const bool far = !(vmax3_(fabsf(ox), fabsf(oy), fabsf(oz)) <= reach());
-                    if (hitRef < 0 || far)
-                        again = !leaf_box_passes(boxes(), (uint32_t)(hitRef < 0 ? ~hitRef : hitRef), tmin, idx_, idy_, idz_,
-                                                 oodx, oody, oodz);
-                }
+                if (cur == kSentinel && live && hitId >= 0 && !strict)
+                    again = !leaf_box_passes(boxes(), (uint32_t)hitRef, tmin, idx_, idy_, idz_, oodx, oody, oodz);
                 if (__ballot(again) != 0) {
                     if (again) {
                         hitT = __builtin_canonicalizef(
@@ -734,7 +726,7 @@ __device__ __forceinline__ void trace_steps(const TraceArgs& a, const BatchDesc*
                     (!WIDE || !strict || leaf_box_passes(boxes(), l >> 5, tmin, idx_, idy_, idz_, oodx, oody, oodz))) {
                     hitT = t;
                     hitId = id;
-                    if (WIDE) hitRef = vmin3_(u, v, 1.0f - uv) < r3.y ? (int)~(l >> 5) : (int)(l >> 5);
+                    if (WIDE) hitRef = (int)(l >> 5);
                     if (any()) {
                         cur = kSentinel;
                         done = false;
@@ -774,7 +766,7 @@ __device__ __forceinline__ void trace_steps(const TraceArgs& a, const BatchDesc*
         while (true) {
             while (__ballot(cur != kSentinel) != 0)
                 quad_step<WIDE>(nodes, tris, r, an, j, at_entry, R + kDeep, spare, boxes(), cur, sp, h, full);
-            const bool again = WIDE && has && walk_again(boxes(), reach(), r, h);
+            const bool again = WIDE && has && walk_again(boxes(), r, h);
             if (__ballot(again) == 0) break;
             if (again) {
                 h = {__builtin_canonicalizef(
@@ -1247,7 +1239,6 @@ rb_status launch_trace(rb_bvh_t bvh, const rb_ray* rays, uint32_t n, uint32_t fl
     if (wide) a.nodes = bvh->wnodes;
     a.stack_rows = stack_rows(bvh, wide);
     a.boxes = bvh->wnodes + 4 * (size_t)bvh->n_wnodes;
-    a.reach = bvh->reach;
     // top-of-tree records in LDS: the speculative walk only
     a.top_nodes = !cfg.speculative ? 0 : cfg.lds_nodes < bvh->n_nodes ? cfg.lds_nodes : bvh->n_nodes;
     const size_t top_bytes = (size_t)a.top_nodes * 64;
@@ -1300,7 +1291,6 @@ rb_status launch_trace_pair(rb_bvh_t bvh, const rb_ray* rays0, uint32_t cap0, co
     a.nodes = wide ? bvh->wnodes : bvh->nodes;
     a.stack_rows = stack_rows(bvh, wide);
     a.boxes = bvh->wnodes + 4 * (size_t)bvh->n_wnodes;
-    a.reach = bvh->reach;
     a.tris = bvh->tris4;
     a.index = bvh->index;
     a.rays = reinterpret_cast<const float4*>(rays0);
@@ -1381,7 +1371,6 @@ static rb_status launch_trace_sets_pass(const BatchSet* b, uint32_t nb, hipStrea
             d.n_dev = b[i].n_dev;
             d.n = b[i].n;
             d.any = b[i].any ? 1u : 0u;
-            d.reach = b[i].bvh->reach;
             d.boxes = b[i].bvh->wnodes + 4 * (size_t)b[i].bvh->n_wnodes;
             rows = std::max(rows, stack_rows(b[i].bvh, wide));
             total += b[i].n;
