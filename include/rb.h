@@ -427,7 +427,8 @@ rb_status rb_trace_set_config(const rb_trace_config* c);
  * coordinate descent over block, lds_stack, chunk, fetch_threshold,
  * waves_per_cu and leaf_gate (lds_nodes in the speculative order, which is
  * kept as set), installs the fastest and returns it with its time per
- * launch. */
+ * launch.  Rays too few for their launch to use the configuration
+ * (rb_trace_config) leave it as it is; their time is that of their launch. */
 rb_status rb_trace_autotune(rb_bvh_t bvh, const rb_ray* rays, uint32_t n, uint32_t flags, rb_hit* hits,
                             uint32_t reps, rb_trace_config* best, float* best_ms, void* stream);
 /* Traversal error flags raised on the device since the last call (the

@@ -490,7 +490,8 @@ def set_trace_config(**kw):
 
 
 def autotune(tracer, d_rays, n, d_hits, any_hit=False, reps=3, stream=None):
-    """Pick and install the fastest traversal configuration for this batch."""
+    """Pick and install the fastest traversal configuration for this batch
+    (kept as it is for up to 512 rays per CU, whose launches do not use it)."""
     c = L.rb_trace_config()
     ms = C.c_float()
     check(lib().rb_trace_autotune(tracer.handle, _dp(d_rays), n, L.RB_ANY if any_hit else L.RB_CLOSEST,

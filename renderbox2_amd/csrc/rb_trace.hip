@@ -1520,7 +1520,11 @@ rb_status rb_trace_autotune(rb_bvh_t bvh, const rb_ray* rays, uint32_t n, uint32
         const uint32_t waves[] = {8, 12, 16, 20, 24, 32};
         const uint32_t gates[] = {16, 24, 32, 40, 48, 56, 63};
         const uint32_t tops[] = {0, 64, 128, 192, 256, 384};
-        for (int pass = 0; pass < 2; pass++) {
+        // launches of few rays do not use the configuration: every candidate
+        // would be the same launch, and the one that noise favours would be
+        // installed for the large ones
+        const int passes = few_rays(cur, n) ? 0 : 2;
+        for (int pass = 0; pass < passes; pass++) {
             for (int dim = 0; dim < 7; dim++) {
                 const uint32_t* vals;
                 int nv;
