@@ -254,12 +254,19 @@ rb_status rb_bvh_host_release(rb_host_bvh_t b);
  * terminators / uint32 index); MI355X is this library's traversal layout.
  * Call with NULL buffers to get the sizes in bytes. */
 enum { RB_LAYOUT_REF_COMPACT2 = 1, RB_LAYOUT_MI355X = 2,
-       RB_LAYOUT_MI355X_WIDE = 3 /* no counterpart: the MI355X triangles and index with wide
-                                    (4-child, 64-byte) records as nodes, every inner child of a
-                                    binary record replaced by its own two and boxes in
-                                    power-of-two steps; RB_ERR_UNSUPPORTED where they cannot
-                                    hold a box.  (The records the upload walks choose their
-                                    children by surface area and have steps of any size) */ };
+       RB_LAYOUT_MI355X_WIDE = 3, /* no counterpart: the MI355X triangles and index with wide
+                                     (4-child, 64-byte) records as nodes, every inner child of a
+                                     binary record replaced by its own two and boxes in
+                                     power-of-two steps; RB_ERR_UNSUPPORTED where they cannot
+                                     hold a box */
+       RB_LAYOUT_MI355X_WALK = 4  /* no counterpart: what the upload has the kernels walk.  Nodes:
+                                     wide records, children chosen by surface area and boxes in
+                                     steps of any size, then 32 bytes per reference (and for one
+                                     more), the box that a hit on it has to pass.  Triangles: 64
+                                     bytes per reference (three Woop rows, id), then one all
+                                     zero.  Index: as MI355X's, then the most stack entries a
+                                     ray can need.  RB_ERR_UNSUPPORTED where the upload keeps the
+                                     binary walk only */ };
 rb_status rb_bvh_export(rb_host_bvh_t b, uint32_t layout, void* nodes, size_t* nodes_bytes,
                         void* tris, size_t* tris_bytes, void* index, size_t* index_bytes);
 

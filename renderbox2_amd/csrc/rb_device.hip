@@ -333,8 +333,8 @@ rb_status rb_bvh_upload(rb_host_bvh_t hb, rb_scene_t scene, rb_bvh_t* out) {
     if (!hb || !out) return fail(RB_ERR_INVALID, "NULL argument");
     RB_ENSURE();
     Mi355Layout L;
-    std::vector<uint32_t> wide;
-    uint32_t stack = 0, wide_stack = 0, n_wide = 0;
+    WalkLayout W;
+    uint32_t stack = 0;
     try {
         rb_status st = export_mi355x(*hb->b, L);
         if (st != RB_OK) return st;
@@ -346,21 +346,11 @@ rb_status rb_bvh_upload(rb_host_bvh_t hb, rb_scene_t scene, rb_bvh_t* out) {
         // wide records only where their walk fits the same stack and their
         // 8-bit steps can hold the boxes (else the binary walk alone)
         stack = depth + 1;  // one postponed child per record on the way
-        st = export_walk(L.nodes, (uint32_t)L.index.size(), wide, &wide_stack);
-        if (st == RB_ERR_UNSUPPORTED) {
-            wide.clear();
+        st = walk_layout(L, W);
+        if (st == RB_ERR_UNSUPPORTED)
             set_error("");
-        } else if (st != RB_OK) {
+        else if (st != RB_OK)
             return st;
-        }
-        n_wide = (uint32_t)(wide.size() / kWideWords);
-        if (n_wide) {
-            std::vector<float> box;
-            leaf_boxes(L.nodes, (uint32_t)L.index.size(), box);
-            const size_t at = wide.size();
-            wide.resize(at + box.size());
-            std::memcpy(&wide[at], box.data(), 4 * box.size());
-        }
     } catch (...) {
         return fail(RB_ERR_OOM, "layout export failed (host allocation)");
     }
@@ -383,23 +373,16 @@ rb_status rb_bvh_upload(rb_host_bvh_t hb, rb_scene_t scene, rb_bvh_t* out) {
     B->n_nodes = (uint32_t)(L.nodes.size() / 16);
     B->n_refs = (uint32_t)L.index.size();
     B->stack = stack;
-    B->wide_stack = wide_stack;
+    B->wide_stack = W.entries;
     if ((st = up((void**)&B->nodes, L.nodes.data(), L.nodes.size() * 4)) != RB_OK) { cleanup(); return st; }
-    B->n_wnodes = n_wide;
-    if (!wide.empty() && (st = up((void**)&B->wnodes, wide.data(), wide.size() * 4)) != RB_OK) { cleanup(); return st; }
+    B->n_wnodes = W.n_records;
+    if (!W.nodes.empty() && (st = up((void**)&B->wnodes, W.nodes.data(), W.nodes.size() * 4)) != RB_OK) { cleanup(); return st; }
     // after the references the zero triangle of the wide records' empty
     // slots (no ray hits it)
     L.tris.resize(L.tris.size() + 12, 0.0f);
     if ((st = up((void**)&B->tris, L.tris.data(), L.tris.size() * 4)) != RB_OK) { cleanup(); return st; }
     L.index.push_back(0);
-    {
-        std::vector<uint32_t> t4(((size_t)B->n_refs + 1) * 16, 0u);
-        for (uint32_t r = 0; r <= B->n_refs; r++) {
-            std::memcpy(&t4[16 * (size_t)r], &L.tris[12 * (size_t)r], 48);
-            t4[16 * (size_t)r + 12] = L.index[r];
-        }
-        if ((st = up((void**)&B->tris4, t4.data(), t4.size() * 4)) != RB_OK) { cleanup(); return st; }
-    }
+    if ((st = up((void**)&B->tris4, W.tris.data(), W.tris.size() * 4)) != RB_OK) { cleanup(); return st; }
     if ((st = up((void**)&B->index, L.index.data(), L.index.size() * 4)) != RB_OK) { cleanup(); return st; }
     if (scene) {
         const Scene& Sc = scene->s;

@@ -609,6 +609,17 @@ rb_status rb_bvh_export(rb_host_bvh_t b, uint32_t layout, void* nodes, size_t* n
             if ((st = copy_out(L.tris.data(), L.tris.size() * 4, tris, tb)) != RB_OK) return st;
             return copy_out(L.index.data(), L.index.size() * 4, index, ib);
         }
+        if (layout == RB_LAYOUT_MI355X_WALK) {
+            Mi355Layout L;
+            rb_status st = export_mi355x(*b->b, L);
+            if (st != RB_OK) return st;
+            WalkLayout W;
+            if ((st = walk_layout(L, W)) != RB_OK) return st;
+            L.index.push_back(W.entries);
+            if ((st = copy_out(W.nodes.data(), W.nodes.size() * 4, nodes, nb)) != RB_OK) return st;
+            if ((st = copy_out(W.tris.data(), W.tris.size() * 4, tris, tb)) != RB_OK) return st;
+            return copy_out(L.index.data(), L.index.size() * 4, index, ib);
+        }
     } catch (...) {
         return fail(RB_ERR_OOM, "layout export failed (host allocation)");
     }

@@ -222,6 +222,16 @@ rb_status export_walk(const std::vector<uint32_t>& bin, uint32_t n_refs, std::ve
 // of at the end, 2 Mi diffuse rays took 644 us and ambient occlusion 512x512
 // 354 against 346.)
 void leaf_boxes(const std::vector<uint32_t>& bin, uint32_t n_refs, std::vector<float>& box);
+// What the kernels walk closest hits with, as it goes to the device.
+struct WalkLayout {
+    std::vector<uint32_t> nodes;  // the wide records (export_walk), then leaf_boxes; empty where the binary walk is kept
+    std::vector<uint32_t> tris;   // 16 words per reference: Woop rows, id, 0, 0, 0; one more, all zero
+    uint32_t n_records = 0;
+    uint32_t entries = 0;         // export_walk's
+};
+// RB_ERR_UNSUPPORTED, with the triangles alone, where the records cannot hold
+// the tree or their walk needs more stack than there is.
+rb_status walk_layout(const Mi355Layout& L, WalkLayout& out);
 // Depth of the deepest inner record of an MI355X node array (root = 0);
 // UINT32_MAX when a link leaves the array or the links form a cycle.  A
 // traversal holds at most depth + 1 stack entries (the sentinel, then one

@@ -662,6 +662,28 @@ void leaf_boxes(const std::vector<uint32_t>& bin, uint32_t n_refs, std::vector<f
     }
 }
 
+rb_status walk_layout(const Mi355Layout& L, WalkLayout& out) {
+    const uint32_t n_refs = (uint32_t)L.index.size();
+    out = WalkLayout();
+    out.tris.assign(((size_t)n_refs + 1) * 16, 0u);
+    for (uint32_t r = 0; r < n_refs; r++) {
+        std::memcpy(&out.tris[16 * (size_t)r], &L.tris[12 * (size_t)r], 48);
+        out.tris[16 * (size_t)r + 12] = L.index[r];
+    }
+    const rb_status st = export_walk(L.nodes, n_refs, out.nodes, &out.entries);
+    if (st != RB_OK) {
+        out.nodes.clear();
+        return st;
+    }
+    out.n_records = (uint32_t)(out.nodes.size() / kWideWords);
+    std::vector<float> box;
+    leaf_boxes(L.nodes, n_refs, box);
+    const size_t at = out.nodes.size();
+    out.nodes.resize(at + box.size());
+    std::memcpy(&out.nodes[at], box.data(), 4 * box.size());
+    return RB_OK;
+}
+
 uint32_t layout_depth(const std::vector<uint32_t>& nodes) {
     const uint32_t n = (uint32_t)(nodes.size() / 16);
     if (n == 0) return 0;
