@@ -334,7 +334,10 @@ rb_status rb_bvh_upload(rb_host_bvh_t hb, rb_scene_t scene, rb_bvh_t* out) {
     RB_ENSURE();
     Mi355Layout L;
     WalkLayout W;
-    uint32_t stack = 0;
+    uint32_t stack = 0, n_refs = 0;
+    std::vector<float> tv, tn;  // the scene's triangles, and their shading normals where some have them
+    std::unique_ptr<rb_bvh_s> B;
+    // every host allocation, before the first on the device
     try {
         rb_status st = export_mi355x(*hb->b, L);
         if (st != RB_OK) return st;
@@ -351,13 +354,41 @@ rb_status rb_bvh_upload(rb_host_bvh_t hb, rb_scene_t scene, rb_bvh_t* out) {
             set_error("");
         else if (st != RB_OK)
             return st;
+        if (scene && scene->s.num_tris() != (uint32_t)(hb->b->idx.size() / 3))
+            return fail(RB_ERR_INVALID, "scene has %u triangles, the BVH was built over %zu", scene->s.num_tris(),
+                        hb->b->idx.size() / 3);
+        // after the references the zero triangle of the wide records' empty
+        // slots (no ray hits it)
+        n_refs = (uint32_t)L.index.size();
+        L.tris.resize(L.tris.size() + 12, 0.0f);
+        L.index.push_back(0);
+        if (scene) {
+            const Scene& Sc = scene->s;
+            const uint32_t n_tris = Sc.num_tris();
+            tv.resize((size_t)n_tris * 12);
+            // shading normals: 3 float4 per triangle, only when some triangle has them
+            tn.resize(Sc.nidx.empty() ? 0 : (size_t)n_tris * 12, 0.0f);
+            for (uint32_t t = 0; t < n_tris; t++) {
+                const bool has_n = Sc.tri_has_normals(t);
+                for (int k = 0; k < 3; k++) {
+                    uint32_t vi = Sc.idx[3 * (size_t)t + k];
+                    tv[12 * (size_t)t + 4 * k + 0] = Sc.verts[3 * (size_t)vi];
+                    tv[12 * (size_t)t + 4 * k + 1] = Sc.verts[3 * (size_t)vi + 1];
+                    tv[12 * (size_t)t + 4 * k + 2] = Sc.verts[3 * (size_t)vi + 2];
+                    // v0.w: material; v1.w: flags (kTriHasNormals = 1)
+                    uint32_t w = k == 0 ? Sc.tri_mat[t] : (k == 1 && has_n ? 1u : 0u);
+                    std::memcpy(&tv[12 * (size_t)t + 4 * k + 3], &w, 4);
+                    if (has_n) {
+                        const uint32_t ni = Sc.nidx[3 * (size_t)t + k];
+                        for (int c = 0; c < 3; c++) tn[12 * (size_t)t + 4 * k + c] = Sc.normals[3 * (size_t)ni + c];
+                    }
+                }
+            }
+        }
+        B.reset(new rb_bvh_s());
     } catch (...) {
-        return fail(RB_ERR_OOM, "layout export failed (host allocation)");
+        return fail(RB_ERR_OOM, "BVH upload failed (host allocation)");
     }
-    if (scene && scene->s.num_tris() != (uint32_t)(hb->b->idx.size() / 3))
-        return fail(RB_ERR_INVALID, "scene has %u triangles, the BVH was built over %zu", scene->s.num_tris(),
-                    hb->b->idx.size() / 3);
-    std::unique_ptr<rb_bvh_s> B(new rb_bvh_s());
     auto up = [&](void** dst, const void* src, size_t bytes) -> rb_status {
         rb_status st = dalloc(dst, bytes);
         if (st != RB_OK) return st;
@@ -371,41 +402,18 @@ rb_status rb_bvh_upload(rb_host_bvh_t hb, rb_scene_t scene, rb_bvh_t* out) {
     auto cleanup = [&]() { rb_bvh_release(B.release()); };
     rb_status st;
     B->n_nodes = (uint32_t)(L.nodes.size() / 16);
-    B->n_refs = (uint32_t)L.index.size();
+    B->n_refs = n_refs;
     B->stack = stack;
     B->wide_stack = W.entries;
     if ((st = up((void**)&B->nodes, L.nodes.data(), L.nodes.size() * 4)) != RB_OK) { cleanup(); return st; }
     B->n_wnodes = W.n_records;
     if (!W.nodes.empty() && (st = up((void**)&B->wnodes, W.nodes.data(), W.nodes.size() * 4)) != RB_OK) { cleanup(); return st; }
-    // after the references the zero triangle of the wide records' empty
-    // slots (no ray hits it)
-    L.tris.resize(L.tris.size() + 12, 0.0f);
     if ((st = up((void**)&B->tris, L.tris.data(), L.tris.size() * 4)) != RB_OK) { cleanup(); return st; }
-    L.index.push_back(0);
     if ((st = up((void**)&B->tris4, W.tris.data(), W.tris.size() * 4)) != RB_OK) { cleanup(); return st; }
     if ((st = up((void**)&B->index, L.index.data(), L.index.size() * 4)) != RB_OK) { cleanup(); return st; }
     if (scene) {
         const Scene& Sc = scene->s;
         B->n_tris = Sc.num_tris();
-        std::vector<float> tv((size_t)B->n_tris * 12);
-        // shading normals: 3 float4 per triangle, only when some triangle has them
-        std::vector<float> tn(Sc.nidx.empty() ? 0 : (size_t)B->n_tris * 12, 0.0f);
-        for (uint32_t t = 0; t < B->n_tris; t++) {
-            const bool has_n = Sc.tri_has_normals(t);
-            for (int k = 0; k < 3; k++) {
-                uint32_t vi = Sc.idx[3 * (size_t)t + k];
-                tv[12 * (size_t)t + 4 * k + 0] = Sc.verts[3 * (size_t)vi];
-                tv[12 * (size_t)t + 4 * k + 1] = Sc.verts[3 * (size_t)vi + 1];
-                tv[12 * (size_t)t + 4 * k + 2] = Sc.verts[3 * (size_t)vi + 2];
-                // v0.w: material; v1.w: flags (kTriHasNormals = 1)
-                uint32_t w = k == 0 ? Sc.tri_mat[t] : (k == 1 && has_n ? 1u : 0u);
-                std::memcpy(&tv[12 * (size_t)t + 4 * k + 3], &w, 4);
-                if (has_n) {
-                    const uint32_t ni = Sc.nidx[3 * (size_t)t + k];
-                    for (int c = 0; c < 3; c++) tn[12 * (size_t)t + 4 * k + c] = Sc.normals[3 * (size_t)ni + c];
-                }
-            }
-        }
         if ((st = up((void**)&B->tri_v, tv.data(), tv.size() * 4)) != RB_OK) { cleanup(); return st; }
         if (!tn.empty() && (st = up((void**)&B->tri_n, tn.data(), tn.size() * 4)) != RB_OK) { cleanup(); return st; }
         B->n_mats = (uint32_t)Sc.mats.size();
