@@ -99,6 +99,7 @@ __device__ __forceinline__ uint32_t block_reserve(uint32_t* counter, uint32_t c)
 __device__ __forceinline__ void block_reserve3(uint32_t* rays, bool a, bool b, bool c, uint32_t* paths, bool q,
                                                uint32_t* sa, uint32_t* sb, uint32_t* sq) {
     // per wave and then per workgroup, packed: a in bits 0..9, b and c in 10..20, q in 21..31
+    static_assert(kQueueBlock < 1024, "a workgroup's counts overflow their bits");
     __shared__ uint32_t s_sum[kQueueBlock / 64];
     __shared__ uint32_t s_base[3];
     const uint32_t lane = __lane_id(), wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
