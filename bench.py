@@ -543,11 +543,11 @@ def main():
     # bytes the timed kernel itself reads and writes per ray: the ray (32),
     # the hit (8), each visited record (64, binary or wide) and each tested
     # triangle (64 with its id; the speculative walk: 48, and 4 for the hit's
-    # index entry)
+    # index entry), and over wide records the box of the hit's leaf (32)
     wide = bool(cfg["wide"]) and not cfg["speculative"]
     if wide:
         wids, _, wcnt = tracer.trace_counts(d_diff.download(np.float32, n * 8).reshape(n, 8), wide=True)
-        kernel_bpr = float((40 + 64 * wcnt[:, 0] + 64 * wcnt[:, 1]).mean())
+        kernel_bpr = float((40 + 64 * wcnt[:, 0] + 64 * wcnt[:, 1] + 32 * (wids >= 0)).mean())
         wide_records = float(wcnt[:, 0].mean())
         del wids, wcnt
     else:

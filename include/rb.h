@@ -310,7 +310,7 @@ typedef struct rb_bvh_dev {
     uint32_t* errors;       /* device word for RB_TRACE_ERR_* flags (rb_trace_errors); may be NULL */
     const void* wnodes;     /* float4[4 * n_wnodes]: wide (4-child) records, then float4[2 * n_refs]:
                                the box of each reference's leaf, which rb_trace_one
-                               walks for closest hits (the same (id, t)); NULL: the binary
+                               walks for closest hits (rb_trace's (id, t)); NULL: the binary
                                records only.  Set when rb_trace_config.wide is on */
     uint32_t n_wnodes;
     uint32_t n_tris;        /* triangles of the scene the BVH was uploaded with (0: none) */
@@ -423,9 +423,12 @@ typedef struct rb_trace_config {
                                 buffer walk 4-child records (subtrees of the binary
                                 tree chosen by surface area; 64 bytes, boxes in 8-bit
                                 steps that hold the exact ones), about half the
-                                dependent fetches per ray.  The same (id, t) as the
-                                binary walk, whose order any-hit traces and visit
-                                counts keep; 0: the binary records for every trace */
+                                dependent fetches per ray.  The (id, t) of the binary
+                                walk, whose order any-hit traces and visit counts
+                                keep, but for rays that pass a leaf's box in its
+                                8-bit form only, at the cracks between triangles (3
+                                of 128 M diffuse rays); 0: the binary records for
+                                every trace */
 } rb_trace_config;
 rb_status rb_trace_get_config(rb_trace_config* c);
 rb_status rb_trace_set_config(const rb_trace_config* c);

@@ -68,8 +68,8 @@ __device__ __forceinline__ rb_hit rb_trace_one(const rb_bvh_dev& b, const rb_ray
         (dst) = stack[sp];   \
         --sp;                \
     } while (0)
-    /* closest hit over the wide records: the same (id, t), about half the
-       record fetches (every leaf the binary walk tests is tested) */
+    /* closest hit over the wide records, as rb_trace: about half the record
+       fetches (every leaf the binary walk tests is tested) */
     const float4* wnodes = any ? nullptr : reinterpret_cast<const float4*>(b.wnodes);
     /* after the wide records, two rows per reference: the box of its leaf.  The
        records' boxes are a little larger; a hit counts if this one passes */

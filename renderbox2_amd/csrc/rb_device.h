@@ -14,7 +14,7 @@ namespace rb {
 // the work counter of ray band b (b < kRayBands), each on a 128-byte line of
 // its own (with all eight on one line, claims from different XCDs contend
 // for it: 1.43 against 0.97 ms on a 2 Mi-ray launch); [0] the one work
-// counter of a batched launch; the rest unused.  The
+// counter of a speculative batched launch; the rest unused.  The
 // last block out resets them to zero, so no memset node is needed between
 // launches or inside captured graphs.  A
 // slot is reused kCounterSlots launches later; when that launch is on
@@ -22,10 +22,12 @@ namespace rb {
 // event recorded after the slot's previous launch, so two launches never
 // share a counter whatever the streams and the number in flight.
 constexpr uint32_t kCounterSlots = 4096;
-// A launch's rays are split into this many contiguous bands, one per XCD:
-// the waves of an XCD claim rays from the band of its number first, so the
-// rays that share an XCD's L2 start near each other (contiguous rays are
-// neighbouring pixels' rays), then from the other bands in turn.
+// A launch's rays are split into this many bands, one per XCD: the waves of
+// an XCD claim rays from the band of its number first, then from the others
+// in turn.  In the step loop runs of claims go to the bands in turn (RayPool),
+// in a single-set speculative launch each band is an eighth of the rays; in
+// both, rays that share an XCD's L2 start near each other (rays next to each
+// other are neighbouring pixels').
 constexpr uint32_t kRayBands = 8;
 constexpr uint32_t kBandStride = 32;  // words: one 128-byte line per counter
 constexpr uint32_t kCounterWords = kBandStride * (kRayBands + 1);
@@ -116,8 +118,9 @@ rb_bvh_dev device_view(rb_bvh_t bvh);
 
 // Internal trace flag, beside RB_ANY: an any-hit set whose consumer reads
 // only hit / miss (hit.x < 0).  Such a set may walk the wide records, which
-// find a hit exactly when the binary walk does but not necessarily the same
-// first one.  The public entry points refuse the bit.
+// find a hit when the binary walk does (leaf_boxes: and for which rays more)
+// but not necessarily the same first one.  The public entry points refuse the
+// bit.
 constexpr uint32_t kOcclusion = 1u << 16;
 // And: neighbouring rays of the set start together and run alike (camera
 // rays), which moves the line up to which launches give each ray a quad.

@@ -170,10 +170,8 @@ rb_status export_mi355x(const HostBvh& b, Mi355Layout& out);
 // hi.z (plane = fmaf(q, s, p), a box holding the exact one), words 10..13
 // their links (>= 0: wide record; < 0: leaf, as in the binary records;
 // kWideEmpty: no child), words 14..15 unused.  Record 0 is the root, the
-// records are numbered breadth-first.  Closest-hit results do not depend on
-// the visit order (ties at equal t go to the lowest triangle id) and every
-// leaf the binary walk tests is tested, so the wide traversal returns the
-// binary one's (id, t).
+// records are numbered breadth-first.  They are handed out, and give
+// leaf_boxes its boxes; the kernels walk export_walk's.
 constexpr uint32_t kWideWords = 16;
 constexpr int32_t kWideEmpty = 0x7FFFFFFF;
 rb_status export_wide(const std::vector<uint32_t>& bin, std::vector<uint32_t>& wide);
@@ -196,9 +194,8 @@ rb_status export_wide(const std::vector<uint32_t>& bin, std::vector<uint32_t>& w
 // cross the record's children and by 2^-24 of the distance itself; their
 // planes lie outside the boxes by 2^-20 of the children's extent, and the
 // walk widens a span by 2^-22 of its far end.  So a ray passes a child's box
-// whenever it passes the binary walk's, every leaf the binary walk tests is
-// tested, and closest hits, which do not depend on the visit order (ties at
-// equal t go to the lowest triangle id), have the same (id, t).
+// whenever it passes the binary walk's and every leaf the binary walk tests is
+// tested.  Which of the hits count, leaf_boxes says.
 // *entries: the most stack entries a ray can need.
 rb_status export_walk(const std::vector<uint32_t>& bin, uint32_t n_refs, std::vector<uint32_t>& walk,
                       uint32_t* entries);
@@ -214,7 +211,16 @@ rb_status export_walk(const std::vector<uint32_t>& bin, uint32_t n_refs, std::ve
 // Every ray that hits is tested, wherever on its triangle: a slab test's
 // rounding moves its point along the ray, across a triangle that the ray grazes
 // by as much more as the ray lies in its plane, and a box cut by a spatial split
-// ends far from its triangle's edges.  (Tested only near an edge, 13,000 to
+// ends far from its triangle's edges.
+// These boxes are the binary ones or up to a step of 8 bits larger, so closest
+// hits over the records are the binary walk's but for rays that meet a triangle
+// between the two: 3 of 128 M in rooms and among spheres.  Of rays aimed within
+// 3e-4 of the grid lines of a tessellated wall of 10 x 10 units one in 17 differs
+// for 27 x 27 squares, whose corners are no multiples of a power of two, and none
+// for 32 x 32.  (The binary leaf boxes would give the binary walk's hit and miss
+// for all of them, but not the images of the two-level records, which all of
+// those 128 M rays do.)
+// (Tested only near an edge, 13,000 to
 // 20,000 of 400,000 rays that graze a wall hit what they pass.  The test of all,
 // against that: 632 -> 643 us for 2 Mi diffuse rays at 1M triangles, 799 -> 809
 // for a 128x128 path-traced tile; testing every hit as it is found reads two

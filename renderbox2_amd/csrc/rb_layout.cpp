@@ -403,7 +403,9 @@ rb_status export_wide(const std::vector<uint32_t>& bin, std::vector<uint32_t>& w
 // Walk records (rb_internal.h), the wide records the upload makes.
 //
 // Which binary records become wide ones is chosen by the surface-area
-// heuristic: cost(n, k) is the cheapest way to represent the subtree of
+// heuristic, with the dynamic program of Ylitie, Karras and Laine, "Efficient
+// Incoherent Ray Traversal on GPUs Through Compressed Wide BVHs" (2017):
+// cost(n, k) is the cheapest way to represent the subtree of
 // binary record n by at most k child slots, each slot a leaf or a wide record
 // of its own (which costs its area and spreads its two children over four
 // slots).  Against replacing every inner child by its own two this reads 3-4%

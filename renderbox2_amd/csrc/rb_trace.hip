@@ -369,7 +369,7 @@ __device__ __forceinline__ void trace_quads(const TraceArgs& a, const BatchDesc*
 // own ray, a node record or one triangle of a leaf, and the records of both
 // kinds are loaded together before either kind of step runs.  The launch is
 // bound by VALU issue (2 Mi diffuse rays, 1M triangles: 85% of the issue
-// slots; 348 M instructions per launch), with the drain of the last rays
+// slots; 337 M instructions per launch), with the drain of the last rays
 // behind it, so what counts is instructions per step and the lanes each
 // instruction serves.  Measured on that launch against a node loop and a leaf
 // loop in turn over power-of-two records (lanes that reached a leaf waited
@@ -1207,8 +1207,8 @@ rb_status launch_trace(rb_bvh_t bvh, const rb_ray* rays, uint32_t n, uint32_t fl
     if (n > 0x7FFFFFFFu) return fail(RB_ERR_INVALID, "too many rays in one call (%u)", n);
     if ((flags & RB_MASKED) && !mask) return fail(RB_ERR_INVALID, "RB_MASKED without a mask");
     const bool any = (flags & RB_ANY) != 0;
-    // Closest hit (the same (id, t)) and occlusion walk the wide records;
-    // visit counts follow the binary walk unless RB_WIDE_COUNTS asks for the
+    // Closest hit and occlusion walk the wide records (leaf_boxes: whose hits
+    // they are); visit counts follow the binary walk unless RB_WIDE_COUNTS asks for the
     // wide one.
     const bool wide_counts = (flags & RB_WIDE_COUNTS) != 0;
     if (wide_counts && (!counts || any || cfg.speculative))
